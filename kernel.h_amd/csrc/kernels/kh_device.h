@@ -138,6 +138,24 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(readlane(v, 0), readlane(v, 16)), fmaxf(readlane(v, 32), readlane(v, 48)));
 }
 
+// The same inside each 16-lane row only: lanes 0-15, 16-31, 32-47 and 48-63
+// each end with their own row's result.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += ror<8>(v);
+  v += ror<4>(v);
+  v += ror<2>(v);
+  v += ror<1>(v);
+  return v;
+}
+
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, ror<8>(v));
+  v = fmaxf(v, ror<4>(v));
+  v = fmaxf(v, ror<2>(v));
+  v = fmaxf(v, ror<1>(v));
+  return v;
+}
+
 // dwordx4 loads/stores with the nontemporal hint: streamed data that is
 // touched once should not displace reusable lines in L2 / the MALL. On
 // MI355X this lifts streaming kernels from ~5.4 to ~5.9-6.1 TB/s.
@@ -171,6 +189,16 @@ __device__ __forceinline__ void buf_store4_nt(__amdgpu_buffer_rsrc_t r, uint32_t
   const u32x4_t u = {__float_as_uint(f.x), __float_as_uint(f.y), __float_as_uint(f.z), __float_as_uint(f.w)};
   __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, kBufNt);
 }
+
+__device__ __forceinline__ float4 buf_load4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  const u32x4_t u = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
+  return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
+}
+__device__ __forceinline__ void buf_store1(__amdgpu_buffer_rsrc_t r, uint32_t off, float f) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(f), r, off, 0, 0);
+}
+// An offset outside every span_rsrc: loads read 0, stores are dropped.
+constexpr uint32_t kOutside = 0x80000000u;
 
 // Waits until at most N vector-memory operations of this wave are in flight
 // (gfx9 s_waitcnt: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] at
@@ -211,6 +239,27 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// All-reduce over a workgroup of nw whole waves: each wave's result through
+// LDS (red: one float per wave), combined in the same order by every wave.
+// One barrier; the caller must not write red again before another barrier
+// that follows every wave's return.
+constexpr int kMaxWaves = 16;
+__device__ __forceinline__ float block_max(float v, float (&red)[kMaxWaves], int nw, int lane, int wave) {
+  v = wave_max(v);
+  if (lane == 0) red[wave] = v;
+  lds_barrier();
+  const int i = lane & 15;
+  return row16_max(i < nw ? red[i] : -__builtin_inff());
+}
+
+__device__ __forceinline__ float block_sum(float v, float (&red)[kMaxWaves], int nw, int lane, int wave) {
+  v = wave_sum(v);
+  if (lane == 0) red[wave] = v;
+  lds_barrier();
+  const int i = lane & 15;
+  return row16_sum(i < nw ? red[i] : 0.0f);
 }
 
 }  // namespace kh

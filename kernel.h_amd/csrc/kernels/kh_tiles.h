@@ -7,6 +7,12 @@
 // grid-stride step.
 #define KH_EW_UNROLL 4
 
+// Row templates. Rows of at most KH_ROW16_COLS floats take 16 lanes each,
+// four to a wave; a workgroup holds rows of up to KH_ROW_BLOCK_MAX floats in
+// registers (1024 threads x 16 float4).
+#define KH_ROW16_COLS 256
+#define KH_ROW_BLOCK_MAX 65536
+
 // Scan: workgroup size chosen by the launcher (the kernel accepts 256..1024).
 // One wave of each workgroup runs the look-back; every other thread owns
 // KH_SCAN_PER_THREAD consecutive elements, so a tile is

@@ -370,6 +370,27 @@ bool need(const Shape &s, const char *key, int64_t &v) {
   return true;
 }
 
+// How softmax holds a row of `cols` floats (kh_tiles.h): the symbol
+// that runs it, the threads of a workgroup and the rows it takes at a time.
+struct RowPlan {
+  const char *symbol;
+  unsigned threads;
+  int64_t rows_per_block;
+};
+
+RowPlan softmax_plan(int64_t cols) {
+  if (cols <= KH_ROW16_COLS) return {"softmax", 256, 16};
+  if (cols <= 1024) return {"softmax", 256, 4};
+  if (cols <= 2048) return {"softmax_wide", 256, 4};
+  // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
+  // per thread.
+  auto threads = [&](int v) { return static_cast<unsigned>(64 * ceil_div(ceil_div(cols, 4), 64 * v)); };
+  if (cols <= 4096) return {"softmax_wide", threads(4), 1};
+  if (cols <= 4096 * 4) return {"softmax", threads(4), 1};
+  if (cols <= 4096 * 8) return {"softmax", threads(8), 1};
+  return {"softmax_block", cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
+}
+
 // Launcher-owned geometry per template (see each kernel's header comment).
 int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block) {
   block = {256, 1, 1};
@@ -389,7 +410,13 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
     if (!need(s, "rows", rows) || !need(s, "cols", cols)) {
       return khrt::fail(KHRT_E_INVALID, t + ": shape attributes 'rows' and 'cols' are required and must be positive");
     }
-    grid.x = clamp_grid(ceil_div(rows, 4));
+    if (t == "softmax") {
+      const RowPlan p = softmax_plan(cols);
+      block.x = p.threads;
+      grid.x = clamp_grid(ceil_div(rows, p.rows_per_block));
+    } else {
+      grid.x = clamp_grid(ceil_div(rows, 4));
+    }
   } else if (t == "scan" || t == "scan_totals") {
     if (!need(s, "n", n)) return khrt::fail(KHRT_E_INVALID, t + ": shape attribute 'n' is required and must be positive");
     if (t == "scan") {
@@ -429,11 +456,13 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
 // layernorm rows of 1025..4096 floats use the *_wide variant).
 const char *launch_symbol(const Template *t, const Shape &s) {
   const std::string n = t->name;
-  if (n == "softmax" || n == "layernorm") {
+  if (n == "softmax") {
     auto it = s.find("cols");
-    if (it != s.end() && it->second > 1024 && it->second <= 4096 && (it->second & 3) == 0) {
-      return n == "softmax" ? "softmax_wide" : "layernorm_wide";
-    }
+    if (it != s.end()) return softmax_plan(it->second).symbol;
+  }
+  if (n == "layernorm") {
+    auto it = s.find("cols");
+    if (it != s.end() && it->second > 1024 && it->second <= 4096 && (it->second & 3) == 0) return "layernorm_wide";
   }
   if (n == "gemm") {
     auto m = s.find("m"), nn = s.find("n"), k = s.find("k");

@@ -189,3 +189,66 @@ def test_rows_blocks_of_partial_waves(dev, template, cols):
     kh.synchronize()
     got = down(dy, rows * cols).reshape(rows, cols)
     assert np.max(np.abs(got - ref)) <= 1e-4
+
+
+# Edges of softmax's row paths: 16 lanes (one, two, four float4 each), a wave,
+# a workgroup of 4, 8 and 16 float4 per thread, two sweeps; one column either
+# side of each and widths that leave 1-3 floats in the last float4.
+SOFTMAX_EDGES = [1, 3, 63, 64, 65, 127, 129, 254, 256, 257, 511, 513, 1023, 1025, 2047, 2049, 4095, 4097, 16383,
+                 16385, 32767, 32769, 65535, 65537]
+
+
+@pytest.mark.parametrize("cols", SOFTMAX_EDGES)
+def test_softmax_path_edges(dev, cols):
+    # Rows at odd addresses, a guard after the output, and 5 rows so that a
+    # wave's last group of four is partial. Each output is e/s with exponents
+    # of magnitude up to ~30 (error 2^-24 * 30 each before it cancels), two
+    # roundings of e and 1/s and a sum of positive terms: 1e-6 of the largest.
+    rows, guard = 5, 64
+    x = O.normal(rows * cols, 0x50F7 + cols, 0.0, 4.0)
+    ref = O.ref_softmax(x, rows, cols)
+    dx, dy = up(np.concatenate([np.full(1, np.nan, np.float32), x])), empty(rows * cols + guard, -7.0)
+    say(f"softmax rows={rows} cols={cols}")
+    kh.softmax(dx.ptr + 4, dy, rows, cols)
+    out = down(dy, rows * cols + guard)
+    assert np.all(out[rows * cols:] == -7.0)
+    assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-6 * np.max(ref)
+
+
+@pytest.mark.parametrize("cols", [40, 200, 300, 700, 1500, 3001, 5000, 20001, 40001, 70001])
+def test_softmax_extreme_rows(dev, cols):
+    # Rows of the type's lowest value, of one large value, half masked with
+    # either, and with an infinity or NaN: uniform, the softmax of the rest,
+    # or NaN, as in 64 bits.
+    low = np.finfo(np.float32).min
+    x = O.normal(8 * cols, 0xE27, 0.0, 1.0).reshape(8, cols)
+    x[0], x[1], x[2] = low, 1e9, -np.inf
+    x[3, :cols // 2], x[4, : cols // 2] = -np.inf, low
+    x[5, 0], x[6, cols - 1], x[7] = np.inf, np.nan, -3e38
+    with np.errstate(invalid="ignore"):
+        e = np.exp(x.astype(np.float64) - np.max(x.astype(np.float64), axis=1, keepdims=True))
+        ref = e / e.sum(axis=1, keepdims=True)
+    got = _softmax(x.ravel(), 8, cols)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.nanmax(np.abs(got - ref)) <= 1e-6
+
+
+@pytest.mark.parametrize("symbol", ["softmax", "softmax_wide", "softmax_block"])
+@pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
+@pytest.mark.parametrize("block", [64, 256])
+def test_softmax_padded_rows_any_symbol(dev, symbol, cols, block):
+    # Rows further apart than their width (x and y each by its own stride):
+    # pads are NaN in x and keep their value in y.
+    rows, xs, ys = 11, cols + 5, cols + 3
+    x = O.normal(rows * cols, 0x77, 0.0, 4.0)
+    xp = np.full((rows, xs), np.nan, np.float32)
+    xp[:, :cols] = x.reshape(rows, cols)
+    dx, dy = up(xp.ravel()), empty(rows * ys, -7.0)
+    args = kh.LaunchArgs().add_memref(dx, [rows, cols]).add_memref(dy, [rows, cols])
+    args.slots[5], args.slots[7 + 5] = xs, ys
+    f = kh.GpuModule(kh.code_object("softmax")).get_function(symbol)
+    say(f"{symbol} rows={rows} cols={cols} strides={xs},{ys} block={block}")
+    kh.kernel_launch(f, (2, 1, 1), (block, 1, 1), args)
+    out = down(dy, rows * ys).reshape(rows, ys)
+    assert np.all(out[:, cols:] == -7.0)
+    assert np.max(np.abs(out[:, :cols] - O.ref_softmax(x, rows, cols))) <= 1e-6
