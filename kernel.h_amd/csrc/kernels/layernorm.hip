@@ -5,60 +5,149 @@
 // (lib/dsl/kernels/layernorm.cpp:58-153): x [rows, cols], gamma [cols],
 // beta [cols], y [rows, cols], 24 parameters. Two-pass statistics as the
 // template pins them (mean first, then the mean of squared deviations; no
-// Welford), but the row is read from HBM once: one wavefront holds the row
-// in registers (dwordx4 loads), so the second pass runs on registers. Rows
-// up to 1024 floats read gamma and beta once per workgroup into LDS; wider
-// rows re-read them per row from L2. Every row shares them, so HBM sees them
-// once either way. Traffic: 8 B per element + 8 B per column.
+// Welford), but the row is read from HBM once, into registers, and the second
+// pass runs there. Traffic: 8 B per element + 8 B per column (every row
+// shares gamma and beta, so HBM sees them once). What holds a row depends on
+// its width:
 //
-// Wider rows than the register path, unaligned or odd-width rows take a
-// streaming form with the same two-pass statistics (the row is re-read from
-// cache for the variance and the output). Rows are grid-strided over
-// wavefronts; any block that is a multiple of 64 threads is correct,
-// including the reference's rows x 256 geometry (kernelh_backend.cpp:290).
+//   cols <= 256            16 lanes, four rows per wavefront (rows16)
+//   cols <= 2048           one wavefront (rows_regs; the wide symbol past 1024)
+//   cols <= 65536          one workgroup (row_block)
+//   beyond                 one workgroup, three sweeps (row_stream)
+//
+// No path asks anything of alignment: a dwordx4 buffer access needs 4-byte
+// alignment only and is range-checked dword by dword. Rows are grid-strided;
+// any block is correct, including the reference's rows x 256 geometry
+// (kernelh_backend.cpp:290).
 #include <type_traits>
 
 #include "kh_device.h"
-
-#ifndef KH_LN_MAXV
-#define KH_LN_MAXV 16  // float4 per lane on the register path: cols <= 4096
-#endif
+#include "kh_tiles.h"
 
 namespace {
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kEps = 1e-5f;
 
 // Columns the narrow symbol stages gamma and beta for in LDS.
 constexpr int kStageCols = 1024;
 
-// gamma and beta (cols x 8 B, shared by every row) are not held in
-// registers: that doubled the register footprint and halved the number of
-// rows in flight. With STAGED (cols <= kStageCols) the workgroup copies them
-// into Gs/Bs once, after its waves have issued their first row's loads, and
-// the output reads them from LDS; otherwise each row re-reads them from L2.
-// The LDS copy takes 4x fewer L2 requests for the same 64 lines, which every
-// wave on the chip asks for at the same time. Measured at 4096x1024 it runs
-// level with the L2 re-read (7.4-7.8 us) in a quiet sequence, but held
-// 7.4-7.7 us in the first launches after a run of long GEMMs, where the L2
-// re-read took 8.0-8.4 us.
-// Rows move through buffer resources spanning exactly cols floats: columns
-// past the end read 0 (kept out of the variance by a select) and their
-// stores are dropped, so the path has no per-lane branches. For a wave's first
-// staged row, in a launch that fits one round, and four or more float4 per
-// lane, the loads go out in two halves, the second once the first has landed
-// (kh::kFirstBurst). Without STAGED, gamma and beta are read
+__device__ __forceinline__ float sum4(float4 v) { return (v.x + v.y) + (v.z + v.w); }
+
+// A lane's first column, 4 i. Opaque, so that the tail comparisons made from
+// it stay inside the row loop: hoisted out of it, V x 4 lane masks take more
+// scalar registers than there are.
+__device__ __forceinline__ int first_col(int i) {
+  int c = 4 * i;
+  asm volatile("" : "+v"(c));
+  return c;
+}
+
+// v - mean, 0 past the row's end: component k of the float4 at column c.
+__device__ __forceinline__ float4 deviation(float4 v, float mean, int c, int cols) {
+  return make_float4(c < cols ? v.x - mean : 0.0f, c + 1 < cols ? v.y - mean : 0.0f, c + 2 < cols ? v.z - mean : 0.0f,
+                     c + 3 < cols ? v.w - mean : 0.0f);
+}
+
+__device__ __forceinline__ float squares4(float4 d) { return (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w); }
+
+__device__ __forceinline__ float4 affine4(float4 d, float inv, float4 g, float4 b) {
+  return make_float4(fmaf(d.x * inv, g.x, b.x), fmaf(d.y * inv, g.y, b.y), fmaf(d.z * inv, g.z, b.z),
+                     fmaf(d.w * inv, g.w, b.w));
+}
+
+// gamma and beta are not held in registers: that doubled the register
+// footprint and halved the number of rows in flight. The narrow symbol copies
+// them into Gs/Bs (kStageCols floats each, 0 past cols) once per workgroup,
+// after its waves have issued their first row's loads, and the output reads
+// them from LDS; wider rows re-read them per row from L2. The LDS copy takes
+// 4x fewer L2 requests for the same 64 lines, which every wave on the chip
+// asks for at the same time. Measured at 4096x1024 it runs level with the L2
+// re-read (7.4-7.8 us) in a quiet sequence, but held 7.4-7.7 us in the first
+// launches after a run of long GEMMs, where the L2 re-read took 8.0-8.4 us.
+// Every thread of the block reaches the barrier.
+__device__ __forceinline__ void stage_affine(const float *__restrict__ G, const float *__restrict__ B, int cols,
+                                             int bd, float *Gs, float *Bs) {
+  const __amdgpu_buffer_rsrc_t rg = kh::span_rsrc(G, (uint32_t)cols * 4u), rb = kh::span_rsrc(B, (uint32_t)cols * 4u);
+  for (int i = threadIdx.x; 4 * i < cols; i += bd) {
+    reinterpret_cast<float4 *>(Gs)[i] = kh::buf_load4(rg, 16u * i);
+    reinterpret_cast<float4 *>(Bs)[i] = kh::buf_load4(rb, 16u * i);
+  }
+  kh::lds_barrier();
+}
+
+// Four rows per wavefront, 16 lanes each (V float4 per lane, cols <= 64 V):
+// the reductions stay inside a 16-lane DPP row, and a wave's load instruction
+// covers four rows' worth of memory instead of a quarter of one. One resource
+// spans the rows that exist; a lane's float4 past cols would store over the
+// next row, so its offset is moved outside the resource, and the one float4
+// that straddles cols goes out as dwords. Against a wave per row: 32768x64
+// 10.3 -> 5.4 us. r0, rstep: in rows.
+template <int V>
+__device__ __forceinline__ void layernorm_rows16(const float *__restrict__ X, const float *__restrict__ G,
+                                                 const float *__restrict__ B, float *__restrict__ Y, int64_t rows,
+                                                 int cols, int64_t xs, int64_t ys, int64_t r0, int64_t rstep, int bd,
+                                                 int lane, float *Gs, float *Bs) {
+  const int g = lane >> 4, c = lane & 15;
+  const uint32_t xo = (uint32_t)(g * xs) * 4u, yo = (uint32_t)(g * ys) * 4u;
+  const float n = (float)cols;
+  float4 v[V];
+  auto load_rows = [&](int64_t r) __attribute__((always_inline)) {
+    const int nr = rows - r < 4 ? (int)(rows - r) : 4;
+    const __amdgpu_buffer_rsrc_t rx = kh::span_rsrc(X + r * xs, (uint32_t)((nr - 1) * xs + cols) * 4u);
+#pragma unroll
+    for (int j = 0; j < V; ++j) v[j] = kh::buf_load4_nt(rx, xo + (uint32_t)(c + 16 * j) * 16u);
+  };
+  if (r0 < rows) load_rows(r0);
+  stage_affine(G, B, cols, bd, Gs, Bs);
+  for (int64_t r = r0; r < rows; r += rstep) {
+    if (r != r0) load_rows(r);
+    const int nr = rows - r < 4 ? (int)(rows - r) : 4;
+    const __amdgpu_buffer_rsrc_t ry = kh::span_rsrc(Y + r * ys, (uint32_t)((nr - 1) * ys + cols) * 4u);
+    const int col0 = first_col(c);
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) s += sum4(deviation(v[j], 0.0f, col0 + 64 * j, cols));
+    const float mean = kh::row16_sum(s) / n;
+    float q = 0.0f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      v[j] = deviation(v[j], mean, col0 + 64 * j, cols);
+      q += squares4(v[j]);
+    }
+    const float inv = __builtin_amdgcn_rsqf(kh::row16_sum(q) / n + kEps);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const int col = col0 + 64 * j;
+      const uint32_t off = yo + (uint32_t)col * 4u;
+      const float4 o = affine4(v[j], inv, *reinterpret_cast<const float4 *>(Gs + col),
+                               *reinterpret_cast<const float4 *>(Bs + col));
+      kh::buf_store4_nt(ry, col + 3 < cols ? off : kh::kOutside, o);
+      if ((cols & 3) != 0 && cols / 64 == j) {  // uniform: the float4s that hold the rows' last columns
+        const bool last = col < cols && col + 3 >= cols;
+        kh::buf_store1(ry, last ? off : kh::kOutside, o.x);
+        kh::buf_store1(ry, last && col + 1 < cols ? off + 4u : kh::kOutside, o.y);
+        kh::buf_store1(ry, last && col + 2 < cols ? off + 8u : kh::kOutside, o.z);
+      }
+    }
+  }
+}
+
+// One row per wavefront. Rows move through buffer resources spanning exactly
+// cols floats: columns past the end read 0 (kept out of the deviations by a
+// select) and their stores are dropped, so the path has no per-lane branches.
+// For a wave's first staged row, in a launch that fits one round, and four or
+// more float4 per lane, the loads go out in two halves, the second once the
+// first has landed (kh::kFirstBurst). Without STAGED, gamma and beta are read
 // the same way; with it, from LDS (a lane past cols reads a staged slot it
 // does not use: every path that stages has 4 V float4 <= kStageCols).
 template <int V, bool STAGED>
 __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X, const float *__restrict__ G,
                                                     const float *__restrict__ B, float *__restrict__ Y,
-                                                    int64_t rows, int64_t cols, int64_t xs, int64_t ys,
-                                                    int64_t r0, int64_t rstep, int64_t bd, int lane, float *Gs,
+                                                    int64_t rows, int cols, int64_t xs, int64_t ys,
+                                                    int64_t r0, int64_t rstep, int bd, int lane, float *Gs,
                                                     float *Bs) {
   static_assert(!STAGED || 4 * V * kh::kWave <= kStageCols, "staged slots cover every lane's columns");
-  const float inv_cols = 1.0f / (float)cols;
+  const float n = (float)cols;
   const uint32_t row_bytes = (uint32_t)cols * 4u;
   constexpr int kHalf = V >= 4 ? V / 2 : V;
   float4 v[V];
@@ -71,21 +160,16 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
     }
   };
   if constexpr (STAGED) {
-    // Every thread of the block reaches the barrier: the staging sits
-    // outside the row loop, and the path choice is uniform over the launch.
-    // The first row's loads go out before the gamma/beta copy, whose LDS
-    // writes wait for them as well (issue order).
+    // The staging sits outside the row loop, and the path choice is uniform
+    // over the launch. The first row's loads go out before the gamma/beta
+    // copy, whose LDS writes wait for them as well (issue order).
     if (r0 < rows) {
       if (kh::split_first_burst(rstep * kh::kWave))  // launch threads
         load_row(r0, std::true_type{});
       else
         load_row(r0, std::false_type{});
     }
-    for (int64_t i = threadIdx.x; 4 * i < cols; i += bd) {
-      reinterpret_cast<float4 *>(Gs)[i] = reinterpret_cast<const float4 *>(G)[i];
-      reinterpret_cast<float4 *>(Bs)[i] = reinterpret_cast<const float4 *>(B)[i];
-    }
-    kh::lds_barrier();
+    stage_affine(G, B, cols, bd, Gs, Bs);
   }
   const __amdgpu_buffer_rsrc_t rg = kh::span_rsrc(G, row_bytes), rb = kh::span_rsrc(B, row_bytes);
   for (int64_t r = r0; r < rows; r += rstep) {
@@ -93,17 +177,16 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
     if (!STAGED || r != r0) load_row(r, std::false_type{});
     float s = 0.0f;
 #pragma unroll
-    for (int j = 0; j < V; ++j) s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
-    const float mean = kh::wave_sum(s) * inv_cols;
+    for (int j = 0; j < V; ++j) s += sum4(v[j]);
+    const float mean = kh::wave_sum(s) / n;
+    const int col0 = first_col(lane);
     float q = 0.0f;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      const float dx = v[j].x - mean, dy = v[j].y - mean, dz = v[j].z - mean, dw = v[j].w - mean;
-      const float qj = (dx * dx + dy * dy) + (dz * dz + dw * dw);
-      q += (int64_t)(lane + j * kh::kWave) * 4 < cols ? qj : 0.0f;
+      v[j] = deviation(v[j], mean, col0 + 4 * kh::kWave * j, cols);
+      q += squares4(v[j]);
     }
-    const float var = kh::wave_sum(q) * inv_cols;
-    const float inv = __builtin_amdgcn_rsqf(var + kEps);
+    const float inv = __builtin_amdgcn_rsqf(kh::wave_sum(q) / n + kEps);
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const uint32_t c = (uint32_t)(lane + j * kh::kWave) * 4u;
@@ -112,35 +195,100 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
         g = *reinterpret_cast<const float4 *>(Gs + c);
         b = *reinterpret_cast<const float4 *>(Bs + c);
       } else {
-        const u32x4 gu = __builtin_amdgcn_raw_buffer_load_b128(rg, 4u * c, 0, 0);
-        const u32x4 bu = __builtin_amdgcn_raw_buffer_load_b128(rb, 4u * c, 0, 0);
-        g = make_float4(__uint_as_float(gu.x), __uint_as_float(gu.y), __uint_as_float(gu.z), __uint_as_float(gu.w));
-        b = make_float4(__uint_as_float(bu.x), __uint_as_float(bu.y), __uint_as_float(bu.z), __uint_as_float(bu.w));
+        g = kh::buf_load4(rg, 4u * c);
+        b = kh::buf_load4(rb, 4u * c);
       }
-      float4 o;
-      o.x = fmaf((v[j].x - mean) * inv, g.x, b.x);
-      o.y = fmaf((v[j].y - mean) * inv, g.y, b.y);
-      o.z = fmaf((v[j].z - mean) * inv, g.z, b.z);
-      o.w = fmaf((v[j].w - mean) * inv, g.w, b.w);
-      kh::buf_store4_nt(ry, 4u * c, o);
+      kh::buf_store4_nt(ry, 4u * c, affine4(v[j], inv, g, b));
     }
   }
 }
 
+// One row per workgroup of nt threads, V float4 per thread (cols <= 4 V nt),
+// as many threads as hold the row at V = 4: every load of the row in flight,
+// one read and one write per element (gamma and beta come from L2). The wave
+// per row that took such rows a float at a time, in three sweeps, was bound
+// by that one wave's load latency: 2048x5000 76.6 -> 17.1 us (4.8 TB/s),
+// 512x32001 508 -> 29, 1024x3001 35.0 -> 5.4, 16x65536 602 -> 14.4. More
+// threads than the row needs were slower (512x12000 8.3 us at 768, 11.2 at
+// 1024; 16384x4096 88.5 at 256, 103 at 512).
+template <int V>
+__device__ __forceinline__ void layernorm_row_block(const float *__restrict__ xr, const float *__restrict__ G,
+                                                    const float *__restrict__ B, float *__restrict__ yr, int cols,
+                                                    int nt, int lane, int wave, float (&red)[2][kh::kMaxWaves]) {
+  const uint32_t row_bytes = (uint32_t)cols * 4u;
+  const __amdgpu_buffer_rsrc_t rx = kh::span_rsrc(xr, row_bytes), ry = kh::span_rsrc(yr, row_bytes);
+  const __amdgpu_buffer_rsrc_t rg = kh::span_rsrc(G, row_bytes), rb = kh::span_rsrc(B, row_bytes);
+  const int tid = threadIdx.x, nw = nt / kh::kWave;
+  const float n = (float)cols;
+  float4 v[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j) v[j] = kh::buf_load4_nt(rx, (uint32_t)(tid + j * nt) * 16u);
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < V; ++j) s += sum4(v[j]);
+  const float mean = kh::block_sum(s, red[0], nw, lane, wave) / n;
+  const int col0 = first_col(tid);
+  float q = 0.0f;
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    v[j] = deviation(v[j], mean, col0 + 4 * nt * j, cols);
+    q += squares4(v[j]);
+  }
+  const float inv = __builtin_amdgcn_rsqf(kh::block_sum(q, red[1], nw, lane, wave) / n + kEps);
+#pragma unroll
+  for (int j = 0; j < V; ++j) {
+    const uint32_t off = (uint32_t)(tid + j * nt) * 16u;
+    kh::buf_store4_nt(ry, off, affine4(v[j], inv, kh::buf_load4(rg, off), kh::buf_load4(rb, off)));
+    if (j & 1) __builtin_amdgcn_sched_barrier(0);  // two float4s of gamma and beta in registers at a time
+  }
+}
+
+// Rows past the registers of a workgroup: the same two-pass statistics and
+// the output in three sweeps over chunks of kStreamV float4 per thread.
+constexpr int kStreamV = 4;
 __device__ __forceinline__ void layernorm_row_stream(const float *__restrict__ xr, const float *__restrict__ G,
                                                      const float *__restrict__ B, float *__restrict__ yr,
-                                                     int64_t cols, int lane) {
-  float s = 0.0f;
-  for (int64_t c = lane; c < cols; c += kh::kWave) s += xr[c];
-  const float mean = kh::wave_sum(s) / (float)cols;
-  float q = 0.0f;
-  for (int64_t c = lane; c < cols; c += kh::kWave) {
-    const float d = xr[c] - mean;
-    q += d * d;
+                                                     int64_t cols, int nt, int lane, int wave,
+                                                     float (&red)[2][kh::kMaxWaves]) {
+  const int tid = threadIdx.x, nw = nt / kh::kWave, chunk = 4 * kStreamV * nt;
+  const float n = (float)cols;
+  float mean = 0.0f, s = 0.0f;
+  for (int sweep = 0; sweep < 2; ++sweep) {
+    s = 0.0f;
+    for (int64_t c0 = 0; c0 < cols; c0 += chunk) {
+      const int nc = cols - c0 < chunk ? (int)(cols - c0) : chunk;
+      const __amdgpu_buffer_rsrc_t rx = kh::span_rsrc(xr + c0, (uint32_t)nc * 4u);
+      float4 v[kStreamV];
+#pragma unroll
+      for (int j = 0; j < kStreamV; ++j) v[j] = kh::buf_load4(rx, (uint32_t)(tid + j * nt) * 16u);
+      const int col0 = first_col(tid);
+      float t = 0.0f;
+#pragma unroll
+      for (int j = 0; j < kStreamV; ++j) {
+        const float4 d = deviation(v[j], mean, col0 + 4 * nt * j, nc);
+        t += sweep == 0 ? sum4(d) : squares4(d);
+      }
+      s += t;
+    }
+    s = kh::block_sum(s, red[sweep], nw, lane, wave) / n;
+    if (sweep == 0) mean = s;
   }
-  const float var = kh::wave_sum(q) / (float)cols;
-  const float inv = __builtin_amdgcn_rsqf(var + kEps);
-  for (int64_t c = lane; c < cols; c += kh::kWave) yr[c] = fmaf((xr[c] - mean) * inv, G[c], B[c]);
+  const float inv = __builtin_amdgcn_rsqf(s + kEps);
+  for (int64_t c0 = 0; c0 < cols; c0 += chunk) {
+    const int nc = cols - c0 < chunk ? (int)(cols - c0) : chunk;
+    const uint32_t bytes = (uint32_t)nc * 4u;
+    const __amdgpu_buffer_rsrc_t rx = kh::span_rsrc(xr + c0, bytes), ry = kh::span_rsrc(yr + c0, bytes);
+    const __amdgpu_buffer_rsrc_t rg = kh::span_rsrc(G + c0, bytes), rb = kh::span_rsrc(B + c0, bytes);
+    float4 v[kStreamV];
+#pragma unroll
+    for (int j = 0; j < kStreamV; ++j) v[j] = kh::buf_load4(rx, (uint32_t)(tid + j * nt) * 16u);
+#pragma unroll
+    for (int j = 0; j < kStreamV; ++j) {
+      const uint32_t off = (uint32_t)(tid + j * nt) * 16u;
+      const float4 d = make_float4(v[j].x - mean, v[j].y - mean, v[j].z - mean, v[j].w - mean);
+      kh::buf_store4_nt(ry, off, affine4(d, inv, kh::buf_load4(rg, off), kh::buf_load4(rb, off)));
+    }
+  }
 }
 
 // Blocks that are not whole wavefronts (the reference's own layernorm
@@ -162,68 +310,94 @@ __device__ __forceinline__ void layernorm_row_serial(const float *__restrict__ x
   for (int64_t c = 0; c < cols; ++c) yr[c] = fmaf((xr[c] - mean) * inv, G[c], B[c]);
 }
 
-// Shared by both symbols; WIDE selects the register-path widths compiled in
-// (the kernel's register allocation is that of its widest path). Gs and Bs
-// hold kStageCols floats each in the narrow symbol and are unused (null) in
-// the wide one.
-template <bool WIDE>
+// Which register paths a symbol compiles in: the kernel's register
+// allocation is that of its widest path. Gs and Bs hold kStageCols floats
+// each in the narrow symbol and are unused (null) in the others.
+enum Symbol { kNarrow, kWide, kBlock };
+
+template <Symbol S>
 __device__ __forceinline__ void layernorm_all(const float *__restrict__ X, const float *__restrict__ G,
                                               const float *__restrict__ B, float *__restrict__ Y, int64_t rows,
-                                              int64_t cols, int64_t xs, int64_t ys, int64_t bd, int64_t nb,
-                                              float *Gs, float *Bs) {
+                                              int64_t cols, int64_t xs, int64_t ys, int bd, int64_t nb,
+                                              float (&red)[2][kh::kMaxWaves], float *Gs, float *Bs) {
   if (bd % kh::kWave != 0) {  // uniform over the block: no thread reaches a barrier below
     for (int64_t r = (int64_t)blockIdx.x * bd + threadIdx.x; r < rows; r += bd * nb)
       layernorm_row_serial(X + r * xs, G, B, Y + r * ys, cols);
     return;
   }
   const int lane = kh::lane_id();
-  const int64_t waves_per_block = bd / kh::kWave;
+  const int waves_per_block = bd / kh::kWave;
   // Uniform per wave (readfirstlane): the row loop and its buffer resources stay scalar.
-  const int64_t r0 = blockIdx.x * waves_per_block + __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int64_t r0 = (int64_t)blockIdx.x * waves_per_block + wave;
   const int64_t rstep = waves_per_block * nb;
-  const bool vec = ((cols & 3) == 0) && ((xs & 3) == 0) && ((ys & 3) == 0) && kh::aligned16(X) &&
-                   kh::aligned16(Y) && kh::aligned16(G) && kh::aligned16(B);
-  const int64_t v4 = (cols + 255) / 256;
-  static_assert(kStageCols == 4 * 4 * kh::kWave, "the narrow symbol stages every column its widest path holds");
-  if (!WIDE && vec && v4 <= 1) {
-    layernorm_rows_regs<1, true>(X, G, B, Y, rows, cols, xs, ys, r0, rstep, bd, lane, Gs, Bs);
-  } else if (!WIDE && vec && v4 <= 2) {
-    layernorm_rows_regs<2, true>(X, G, B, Y, rows, cols, xs, ys, r0, rstep, bd, lane, Gs, Bs);
-  } else if (!WIDE && vec && v4 <= 4) {
-    layernorm_rows_regs<4, true>(X, G, B, Y, rows, cols, xs, ys, r0, rstep, bd, lane, Gs, Bs);
-  } else if (WIDE && vec && v4 <= 8) {
-    layernorm_rows_regs<8, false>(X, G, B, Y, rows, cols, xs, ys, r0, rstep, bd, lane, nullptr, nullptr);
-  } else if (WIDE && vec && v4 <= KH_LN_MAXV) {
-    layernorm_rows_regs<KH_LN_MAXV, false>(X, G, B, Y, rows, cols, xs, ys, r0, rstep, bd, lane, nullptr, nullptr);
+  const int c = (int)(cols < KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
+  static_assert(kStageCols == 4 * 4 * kh::kWave, "the narrow symbol stages every column its widest wave path holds");
+  if (S == kNarrow && c <= KH_ROW16_COLS && xs >= cols && ys >= cols && (xs | ys) < (1 << 26)) {
+    if (c <= 64)
+      layernorm_rows16<1>(X, G, B, Y, rows, c, xs, ys, 4 * r0, 4 * rstep, bd, lane, Gs, Bs);
+    else if (c <= 128)
+      layernorm_rows16<2>(X, G, B, Y, rows, c, xs, ys, 4 * r0, 4 * rstep, bd, lane, Gs, Bs);
+    else
+      layernorm_rows16<4>(X, G, B, Y, rows, c, xs, ys, 4 * r0, 4 * rstep, bd, lane, Gs, Bs);
+  } else if (S == kNarrow && c <= 512) {
+    layernorm_rows_regs<2, true>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, Gs, Bs);
+  } else if (S == kNarrow && c <= 1024) {
+    layernorm_rows_regs<4, true>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, Gs, Bs);
+  } else if (S == kWide && c <= 2048) {
+    layernorm_rows_regs<8, false>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, nullptr, nullptr);
   } else {
-    for (int64_t r = r0; r < rows; r += rstep) layernorm_row_stream(X + r * xs, G, B, Y + r * ys, cols, lane);
+    for (int64_t r = blockIdx.x; r < rows; r += nb) {
+      const float *xr = X + r * xs;
+      float *yr = Y + r * ys;
+      if (S != kBlock && c <= 16 * bd)
+        layernorm_row_block<4>(xr, G, B, yr, c, bd, lane, wave, red);
+      else if (S == kNarrow && c <= 32 * bd)
+        layernorm_row_block<8>(xr, G, B, yr, c, bd, lane, wave, red);
+      else if (S == kBlock && c <= 64 * bd)
+        layernorm_row_block<16>(xr, G, B, yr, c, bd, lane, wave, red);
+      else
+        layernorm_row_stream(xr, G, B, yr, cols, bd, lane, wave, red);
+    }
   }
 }
 
 }  // namespace
 
-// The reference symbol: register path for rows up to 1024 floats, any other
-// shape through the streaming path.
-extern "C" __global__ void __launch_bounds__(256)
+#define KH_LAYERNORM_BODY(S, GS, BS)                                                                           \
+  __shared__ float red[2][kh::kMaxWaves];                                                                      \
+  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();                                         \
+  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, gamma_base, gamma_off, beta_base, beta_off, y_base, y_off,    \
+                y_s0, gw, nb);                                                                                 \
+  layernorm_all<S>(KH_PTR(x), KH_PTR(gamma), KH_PTR(beta), KH_PTR(y), x_n0, x_n1, x_s0, y_s0,                  \
+                   (int)kh::threads_x_of(gw), nb, red, GS, BS)
+
+// The reference symbol: rows up to 1024 floats in 16 lanes or a wave, wider
+// ones in a workgroup.
+extern "C" __global__ void __launch_bounds__(1024)
 layernorm(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
           KH_MEMREF2(float, y)) {
   __shared__ __attribute__((aligned(16))) float Gs[kStageCols];
   __shared__ __attribute__((aligned(16))) float Bs[kStageCols];
-  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();
-  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, gamma_base, gamma_off, beta_base, beta_off, y_base, y_off, y_s0,
-                gw, nb);
-  layernorm_all<false>(KH_PTR(x), KH_PTR(gamma), KH_PTR(beta), KH_PTR(y), x_n0, x_n1, x_s0, y_s0,
-                       kh::threads_x_of(gw), nb, Gs, Bs);
+  KH_LAYERNORM_BODY(kNarrow, Gs, Bs);
 }
 
-// Same arguments and results; register path for rows of 1025..4096 floats
-// (the launcher picks it for those widths).
+// Same arguments and results for rows of 1025..4096 floats (the launcher
+// picks it there): a wave per row up to 2048, a workgroup past that. Events
+// around rotated launches, wave against workgroup: 4096x1100 7.4 vs 8.7 us,
+// 4096x2048 10.9 vs 13.0, 1024x2047 4.8 vs 4.6; past 2048 the wave's 16
+// float4 and its share of gamma and beta took 242 registers (16384x4096 91.4
+// vs 88.5).
 extern "C" __global__ void __launch_bounds__(256)
 layernorm_wide(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
                KH_MEMREF2(float, y)) {
-  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();
-  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, gamma_base, gamma_off, beta_base, beta_off, y_base, y_off, y_s0,
-                gw, nb);
-  layernorm_all<true>(KH_PTR(x), KH_PTR(gamma), KH_PTR(beta), KH_PTR(y), x_n0, x_n1, x_s0, y_s0,
-                      kh::threads_x_of(gw), nb, nullptr, nullptr);
+  KH_LAYERNORM_BODY(kWide, nullptr, nullptr);
+}
+
+// Same arguments and results; one workgroup per row with 16 float4 per
+// thread, for rows past what the reference symbol's eight hold.
+extern "C" __global__ void __launch_bounds__(1024)
+layernorm_block(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
+                KH_MEMREF2(float, y)) {
+  KH_LAYERNORM_BODY(kBlock, nullptr, nullptr);
 }

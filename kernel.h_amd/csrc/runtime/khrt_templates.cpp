@@ -370,25 +370,28 @@ bool need(const Shape &s, const char *key, int64_t &v) {
   return true;
 }
 
-// How softmax holds a row of `cols` floats (kh_tiles.h): the symbol
-// that runs it, the threads of a workgroup and the rows it takes at a time.
+// How softmax and layernorm hold a row of `cols` floats (kh_tiles.h): the
+// symbol that runs it, the threads of a workgroup and the rows it takes at a
+// time.
 struct RowPlan {
   const char *symbol;
   unsigned threads;
   int64_t rows_per_block;
 };
 
-RowPlan softmax_plan(int64_t cols) {
-  if (cols <= KH_ROW16_COLS) return {"softmax", 256, 16};
-  if (cols <= 1024) return {"softmax", 256, 4};
-  if (cols <= 2048) return {"softmax_wide", 256, 4};
+RowPlan row_plan(bool softmax, int64_t cols) {
+  const char *narrow = softmax ? "softmax" : "layernorm", *wide = softmax ? "softmax_wide" : "layernorm_wide",
+             *block = softmax ? "softmax_block" : "layernorm_block";
+  if (cols <= KH_ROW16_COLS) return {narrow, 256, 16};
+  if (cols <= 1024) return {narrow, 256, 4};
+  if (cols <= 2048) return {wide, 256, 4};
   // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
   // per thread.
   auto threads = [&](int v) { return static_cast<unsigned>(64 * ceil_div(ceil_div(cols, 4), 64 * v)); };
-  if (cols <= 4096) return {"softmax_wide", threads(4), 1};
-  if (cols <= 4096 * 4) return {"softmax", threads(4), 1};
-  if (cols <= 4096 * 8) return {"softmax", threads(8), 1};
-  return {"softmax_block", cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
+  if (cols <= 4096) return {wide, threads(4), 1};
+  if (cols <= 4096 * 4) return {narrow, threads(4), 1};
+  if (cols <= 4096 * 8) return {narrow, threads(8), 1};
+  return {block, cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
 }
 
 // Launcher-owned geometry per template (see each kernel's header comment).
@@ -410,13 +413,9 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
     if (!need(s, "rows", rows) || !need(s, "cols", cols)) {
       return khrt::fail(KHRT_E_INVALID, t + ": shape attributes 'rows' and 'cols' are required and must be positive");
     }
-    if (t == "softmax") {
-      const RowPlan p = softmax_plan(cols);
-      block.x = p.threads;
-      grid.x = clamp_grid(ceil_div(rows, p.rows_per_block));
-    } else {
-      grid.x = clamp_grid(ceil_div(rows, 4));
-    }
+    const RowPlan p = row_plan(t == "softmax", cols);
+    block.x = p.threads;
+    grid.x = clamp_grid(ceil_div(rows, p.rows_per_block));
   } else if (t == "scan" || t == "scan_totals") {
     if (!need(s, "n", n)) return khrt::fail(KHRT_E_INVALID, t + ": shape attribute 'n' is required and must be positive");
     if (t == "scan") {
@@ -452,17 +451,12 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
 
 // Symbol the launcher runs for a template at a shape. Every symbol of a
 // template takes the same arguments and computes the same result; the
-// variants differ in which register paths they compile in (softmax and
-// layernorm rows of 1025..4096 floats use the *_wide variant).
+// variants differ in which register paths they compile in (row_plan).
 const char *launch_symbol(const Template *t, const Shape &s) {
   const std::string n = t->name;
-  if (n == "softmax") {
+  if (n == "softmax" || n == "layernorm") {
     auto it = s.find("cols");
-    if (it != s.end()) return softmax_plan(it->second).symbol;
-  }
-  if (n == "layernorm") {
-    auto it = s.find("cols");
-    if (it != s.end() && it->second > 1024 && it->second <= 4096 && (it->second & 3) == 0) return "layernorm_wide";
+    if (it != s.end()) return row_plan(n == "softmax", it->second).symbol;
   }
   if (n == "gemm") {
     auto m = s.find("m"), nn = s.find("n"), k = s.find("k");

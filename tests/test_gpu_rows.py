@@ -252,3 +252,47 @@ def test_softmax_padded_rows_any_symbol(dev, symbol, cols, block):
     out = down(dy, rows * ys).reshape(rows, ys)
     assert np.all(out[:, cols:] == -7.0)
     assert np.max(np.abs(out[:, :cols] - O.ref_softmax(x, rows, cols))) <= 1e-6
+
+
+@pytest.mark.parametrize("cols", SOFTMAX_EDGES)
+def test_layernorm_path_edges(dev, cols):
+    # The same edges, every operand at an odd address. Rows of N(3, 4^2): the
+    # mean carries 2^-24 * 12 (the sum's rounding) and the deviations, scaled
+    # to |d| <= ~5 by up to 1/4 (sqrt(1/eps) for the single column, whose
+    # deviation is an exact 0), 2^-24 of themselves: 1e-5 covers both.
+    rows, guard = 5, 64
+    x = O.normal(rows * cols, 0x1A7E + cols, 3.0, 4.0)
+    if cols > 1:  # no row whose few values happen to lie close together
+        x[::cols], x[1::cols] = 9.0, -3.0
+    g = O.uniform(cols, 0x1A7F, 0.5, 1.5)
+    b = O.uniform(cols, 0x1A80, -0.1, 0.1)
+    ref = O.ref_layernorm(x, g, b, rows, cols)
+    nan = np.full(1, np.nan, np.float32)
+    dx, dg, db = (up(np.concatenate([nan, t, nan])) for t in (x, g, b))
+    dy = empty(rows * cols + guard, -7.0)
+    say(f"layernorm rows={rows} cols={cols}")
+    kh.layernorm(dx.ptr + 4, dg.ptr + 4, db.ptr + 4, dy, rows, cols)
+    out = down(dy, rows * cols + guard)
+    assert np.all(out[rows * cols:] == -7.0)
+    assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-5
+
+
+@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wide", "layernorm_block"])
+@pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
+@pytest.mark.parametrize("block", [64, 256])
+def test_layernorm_padded_rows_any_symbol(dev, symbol, cols, block):
+    rows, xs, ys = 11, cols + 5, cols + 3
+    x = O.normal(rows * cols, 0x77, 0.0, 4.0)
+    g, b = O.uniform(cols, 0x78, 0.5, 1.5), O.uniform(cols, 0x79, -0.1, 0.1)
+    xp = np.full((rows, xs), np.nan, np.float32)
+    xp[:, :cols] = x.reshape(rows, cols)
+    dx, dg, db, dy = up(xp.ravel()), up(g), up(b), empty(rows * ys, -7.0)
+    args = kh.LaunchArgs().add_memref(dx, [rows, cols]).add_memref(dg, [cols]).add_memref(db, [cols])
+    args.add_memref(dy, [rows, cols])
+    args.slots[5], args.slots[17 + 5] = xs, ys
+    f = kh.GpuModule(kh.code_object("layernorm")).get_function(symbol)
+    say(f"{symbol} rows={rows} cols={cols} strides={xs},{ys} block={block}")
+    kh.kernel_launch(f, (2, 1, 1), (block, 1, 1), args)
+    out = down(dy, rows * ys).reshape(rows, ys)
+    assert np.all(out[:, cols:] == -7.0)
+    assert np.max(np.abs(out[:, :cols] - O.ref_layernorm(x, g, b, rows, cols))) <= 1e-5
