@@ -54,9 +54,13 @@
 //     ds_read_b32), both conflict-free: rows padded by 4 floats when slabs are
 //     staged through registers; for direct-to-LDS slabs, whose loads write 64
 //     float4s contiguously, A's rows are unpadded with their float4s
-//     XOR-swizzled and B's rows padded per group a wave loads. Slab loads are
-//     branch-free buffer loads for aligned operands with k, n multiples of 4;
-//     their range checks zero-fill the tails (the guarded per-element form of
+//     XOR-swizzled and B's rows padded per group a wave loads. The
+//     direct-to-LDS symbols' slab loads are unconditional at any alignment and
+//     extent: a dwordx4 buffer load needs 4-byte alignment only and is
+//     range-checked dword by dword, and what it carries past K is zeroed in
+//     the fragments of a tile's last slab. The register-staged ones' are
+//     branch-free buffer loads for aligned operands with k, n multiples of 4,
+//     whose range checks zero-fill the tails (the guarded per-element form of
 //     the generic path made the compiler split every load into branches and
 //     dword pieces, which cost 15% of the MFMA rate).
 //   * K order inside an MFMA: the instruction sums k over its two lane
@@ -113,8 +117,8 @@ static_assert(Tile<2, 4, 32, true, 4, 2, 16>::BM == KH_GEMM_WIDE_BM &&
 // as float4s (MFMA operands swapped so a lane holds four consecutive
 // columns) let the stores overlap the next tile, but its 32-byte row pieces
 // doubled the kernel's L2 misses and measured 0.7% slower at 8192^3; C goes
-// out as whole 128-byte lines. K <= 16 and unaligned operands take the
-// per-tile pipeline (or the generic path).
+// out as whole 128-byte lines. K <= 16 takes the per-tile pipeline (or the
+// generic path).
 extern "C" __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 gemm(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
   KH_GEMM_ENTRY_CHECK(kThreads);

@@ -126,10 +126,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const float *base, i
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), (short)0, (int)(rows * ld * 4), kRsrcWord3);
 }
 
-// The same resource as four dwords, for the direct-to-LDS loads below.
-__device__ __forceinline__ u32x4 rows_desc(const float *base, int64_t rows, int64_t ld) {
+// The same as four dwords, for the direct-to-LDS loads below, ending with the
+// last row's `cols` floats: a float4 that straddles them reads the next row's
+// (or 0: the range check is per dword), never past the matrix.
+__device__ __forceinline__ u32x4 rows_desc(const float *base, int64_t rows, int64_t ld, int64_t cols) {
   const uint64_t b = reinterpret_cast<uint64_t>(base);
-  return u32x4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, (uint32_t)(rows * ld * 4), (uint32_t)kRsrcWord3};
+  return u32x4{(uint32_t)b, (uint32_t)(b >> 32) & 0xffffu, (uint32_t)(((rows - 1) * ld + cols) * 4),
+               (uint32_t)kRsrcWord3};
 }
 
 __device__ __forceinline__ float4 as_float4(u32x4 u) {
@@ -199,27 +202,34 @@ __device__ __forceinline__ void dma16(u32x4 rsrc, uint32_t voff, uint32_t lds) {
 
 __device__ __forceinline__ uint32_t lds_addr(const float *p) { return (uint32_t)reinterpret_cast<uintptr_t>(p); }
 
-// Direct-to-LDS slab load for 16-byte aligned A and B with k and n multiples
-// of 4. Each wave's instruction lands 64 float4s contiguously, so the lane ->
+// Direct-to-LDS slab load, at any (4-byte) alignment, for lda >= K and
+// ldb >= N. Each wave's instruction lands 64 float4s contiguously, so the lane ->
 // global mapping realises the layout: in A, lane l of a wave fills physical
 // quad l % QP of its row and so fetches logical quad (l % QP) ^ aswz(row); B
 // is row-major within a group. Callers fetch slabs with k0 < K (or k0 = 0
 // when K = 0, which reads nothing). `wave` must be wave-uniform.
 //
-// ALN (K a multiple of BK, N of BN): no float4 of a slab reaches past K or
-// N, so the per-load tail selects go and each offset is a loop-invariant
-// 32-bit term plus a wave-uniform one (k0 for A, n0 for B), which keeps the
-// offsets of every load of a slab in registers even where the tile's
-// accumulators leave few (rows past M still read 0 through the resource).
+// SELECT: float4s past K (A) or N (B) are sent to an offset outside the
+// resource and read 0; for K and N multiples of 4. Without it nothing is
+// selected: a float4 at or past K or N carries what follows in memory (the
+// next row, or 0 past the matrix). Columns of B past N only feed columns of C
+// that are not stored, rows of B past K read 0 through the range check, and
+// the caller zeroes A's k past K in the fragments (mask_k). Each offset is
+// then a loop-invariant 32-bit term plus a wave-uniform one (k0 for A, n0 for
+// B), which keeps the offsets of every load of a slab in registers even where
+// the tile's accumulators leave few: 8192^3 142.8 -> 146.8 TFLOP/s.
+//
+// WHOLE: every slab the caller fetches has BK rows of B, so the resource's
+// size is the same for all of them (else it is computed per slab).
 //
 // dma_part issues loads L0..L1-1 of a slab (A's NA, then B's NB), so that a
 // slab's loads can be spread between MFMAs; dma_slab issues all of them.
-template <class T, bool ALN, int L0, int L1>
+template <class T, bool SELECT, int L0, int L1, bool WHOLE = false>
 __device__ __forceinline__ void dma_part(const float *__restrict__ A, const float *__restrict__ B, int64_t M,
                                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t m0, int64_t n0,
                                          int64_t k0, float *As, float *Bs, int wave, int lane) {
-  const u32x4 ra = rows_desc(A + m0 * lda, (M - m0) < T::BM ? (M - m0) : T::BM, lda);
-  const u32x4 rb = rows_desc(B + k0 * ldb, (K - k0) < T::BK ? (K - k0) : T::BK, ldb);
+  const u32x4 ra = rows_desc(A + m0 * lda, (M - m0) < T::BM ? (M - m0) : T::BM, lda, K);
+  const u32x4 rb = rows_desc(B + k0 * ldb, WHOLE ? T::BK : (K - k0) < T::BK ? (K - k0) : T::BK, ldb, N);
 #pragma unroll
   for (int i = 0; i < T::NA; ++i) {
     if (i < L0 || i >= L1) continue;
@@ -227,10 +237,10 @@ __device__ __forceinline__ void dma_part(const float *__restrict__ A, const floa
     const int idx = idx0 + lane;
     const int ar = idx / T::QP, ak = 4 * ((idx % T::QP) ^ T::aswz(ar));
     uint32_t aoff;
-    if constexpr (ALN)
-      aoff = ((uint32_t)ar * (uint32_t)lda + (uint32_t)ak) * 4u + (uint32_t)k0 * 4u;
-    else
+    if constexpr (SELECT)
       aoff = (k0 + ak < K) ? (uint32_t)((ar * lda + k0 + ak) * 4) : kOutside;
+    else
+      aoff = ((uint32_t)ar * (uint32_t)lda + (uint32_t)ak) * 4u + (uint32_t)k0 * 4u;
     dma16(ra, aoff, lds_addr(As + 4 * idx0));
   }
 #pragma unroll
@@ -240,19 +250,19 @@ __device__ __forceinline__ void dma_part(const float *__restrict__ A, const floa
     const int idx = idx0 + lane;
     const int bk = idx / T::BROW, bn = 4 * (idx % T::BROW);
     uint32_t boff;
-    if constexpr (ALN)
-      boff = ((uint32_t)bk * (uint32_t)ldb + (uint32_t)bn) * 4u + (uint32_t)n0 * 4u;
-    else
+    if constexpr (SELECT)
       boff = (n0 + bn < N) ? (uint32_t)((bk * ldb + n0 + bn) * 4) : kOutside;
+    else
+      boff = ((uint32_t)bk * (uint32_t)ldb + (uint32_t)bn) * 4u + (uint32_t)n0 * 4u;
     dma16(rb, boff, lds_addr(Bs + T::b_at(idx0 / T::BROW, 4 * (idx0 % T::BROW))));
   }
 }
 
-template <class T, bool ALN = false>
+template <class T, bool SELECT, bool WHOLE = false>
 __device__ __forceinline__ void dma_slab(const float *__restrict__ A, const float *__restrict__ B, int64_t M,
                                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t m0, int64_t n0,
                                          int64_t k0, float *As, float *Bs, int wave, int lane) {
-  dma_part<T, ALN, 0, T::NA + T::NB>(A, B, M, N, K, lda, ldb, m0, n0, k0, As, Bs, wave, lane);
+  dma_part<T, SELECT, 0, T::NA + T::NB, WHOLE>(A, B, M, N, K, lda, ldb, m0, n0, k0, As, Bs, wave, lane);
 }
 
 // Wait until at most N vector-memory operations of this wave are in flight
@@ -312,6 +322,24 @@ __device__ __forceinline__ void read_frag(Frag<WTM, WTN> &f, const float *__rest
     for (int j = 0; j < WTN; ++j)
 #pragma unroll
       for (int s = 0; s < 4; ++s) f.b[j][s] = Bs[T::b_at(16 * c + 4 * q + s, wn * 16 * WTN + j * 16 + r)];
+  }
+}
+
+// Zeroes a fragment's A elements at or past K: chunk c of a slab of which
+// `left` k exist. The lane is asked for again here: kept from the entry it
+// would hold a register through the tile loop.
+template <int WTM, int WTN, class T>
+__device__ __forceinline__ void mask_k(Frag<WTM, WTN> &f, int c, int left) {
+  uint32_t lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  const int g = lane >> 4, kq = T::kMF == 32 ? 8 * c + 4 * (lane >> 5) : 16 * c + 4 * (((g & 1) << 1) | (g >> 1));
+  const int n = left - kq;  // elements of this lane's four that exist
+#pragma unroll
+  for (int i = 0; i < WTM; ++i) {
+    f.a[i].x = n > 0 ? f.a[i].x : 0.0f;
+    f.a[i].y = n > 1 ? f.a[i].y : 0.0f;
+    f.a[i].z = n > 2 ? f.a[i].z : 0.0f;
+    f.a[i].w = n > 3 ? f.a[i].w : 0.0f;
   }
 }
 
@@ -406,9 +434,9 @@ __device__ __forceinline__ void k_loop_dma(AccOf<T> (&acc)[WTM][WTN], const floa
   constexpr int BK = T::BK;
   constexpr int C = BK / Mfma<T::kMF>::CK;
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  dma_slab<T>(Ap, Bp, M, N, K, lda, ldb, m0, n0, 0, As, Bs, wv, lane);
+  dma_slab<T, true>(Ap, Bp, M, N, K, lda, ldb, m0, n0, 0, As, Bs, wv, lane);
   if (nslabs > 1) {
-    dma_slab<T>(Ap, Bp, M, N, K, lda, ldb, m0, n0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
+    dma_slab<T, true>(Ap, Bp, M, N, K, lda, ldb, m0, n0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
     vm_barrier<T::NA + T::NB>();
   } else {
     vm_barrier<0>();
@@ -426,7 +454,7 @@ __device__ __forceinline__ void k_loop_dma(AccOf<T> (&acc)[WTM][WTN], const floa
     if (PRIO) __builtin_amdgcn_s_setprio(0);
     vm_barrier<0>();
     if (ks + 2 < nslabs)
-      dma_slab<T>(Ap, Bp, M, N, K, lda, ldb, m0, n0, (ks + 2) * BK, As + fut * T::A_STAGE, Bs + fut * T::B_STAGE,
+      dma_slab<T, true>(Ap, Bp, M, N, K, lda, ldb, m0, n0, (ks + 2) * BK, As + fut * T::A_STAGE, Bs + fut * T::B_STAGE,
                   wv, lane);
     if (ks + 1 < nslabs) read_frag<WTM, WTN, T>(f0, As + nxt * T::A_STAGE, Bs + nxt * T::B_STAGE, 0, wm, wn, lane);
     if (PRIO) __builtin_amdgcn_s_setprio(1);
@@ -658,9 +686,10 @@ __device__ __forceinline__ void gemm_tiles(const float *__restrict__ Ap, const f
 #pragma unroll
       for (int j = 0; j < WTN; ++j) acc[i][j] = AccOf<T>{};
 
-    if constexpr (PATH == kPipeDma)
-      k_loop_dma<WTM, WTN, T, PRIO>(acc, Ap, Bp, M, N, K, lda, ldb, m0, n0, nslabs, As, Bs, wave, wm, wn, lane);
-    else if constexpr (PATH == kPipeRegs)
+    if constexpr (PATH == kPipeDma) {
+      if (nslabs > 0)  // K = 0: no slab to describe
+        k_loop_dma<WTM, WTN, T, PRIO>(acc, Ap, Bp, M, N, K, lda, ldb, m0, n0, nslabs, As, Bs, wave, wm, wn, lane);
+    } else if constexpr (PATH == kPipeRegs)
       k_loop_regs<WTM, WTN, T, PRIO>(acc, Ap, Bp, M, N, K, lda, ldb, m0, n0, nslabs, As, Bs, tid, wm, wn, lane);
     else if constexpr (PATH == kPipePrefetch2)
       k_loop_prefetch2<WTM, WTN, T, PRIO>(acc, Ap, Bp, M, N, K, lda, ldb, m0, n0, nslabs, As, Bs, tid, wm, wn,
@@ -705,14 +734,17 @@ __device__ __forceinline__ void interleave_reads() {
 // chunk's fragment reads are interleaved with the MFMAs of the chunk
 // before them (interleave_reads); the wave priority is raised before the
 // reads, since s_setprio bounds what the scheduler may interleave.
-template <int WTM, int WTN, class T, bool PRIO, bool ALN, int WAIT = 0>
+// MASK: the slab is a tile's last and reaches past K, so its A fragments there
+// are zeroed (left: the k of the slab that exist).
+template <int WTM, int WTN, class T, bool PRIO, bool WHOLE, int WAIT = 0, bool MASK = false>
 __device__ __forceinline__ void flat_step(AccOf<T> (&acc)[WTM][WTN], Frag<WTM, WTN> &f0, Frag<WTM, WTN> &f1, int &cur,
                                           const float *__restrict__ Ap, const float *__restrict__ Bp, int64_t M,
                                           int64_t N, int64_t K, int64_t lda, int64_t ldb, bool dma, int64_t dm0,
                                           int64_t dn0, int64_t dk0, bool read_next, float *As, float *Bs, int wv,
-                                          int wm, int wn, int lane) {
+                                          int wm, int wn, int lane, int left = 0) {
   constexpr int C = T::BK / Mfma<T::kMF>::CK;
   constexpr int kReads = WTM + 2 * WTN;
+  if constexpr (MASK) mask_k<WTM, WTN, T>(f0, 0, left);
   const int nxt = cur == 2 ? 0 : cur + 1;
   const int fut = nxt == 2 ? 0 : nxt + 1;
   const float *sA = As + cur * T::A_STAGE, *sB = Bs + cur * T::B_STAGE;
@@ -733,20 +765,22 @@ __device__ __forceinline__ void flat_step(AccOf<T> (&acc)[WTM][WTN], Frag<WTM, W
     // 8192^3 and 4096^3 level (7347 -> 7328, 926.0 -> 927.0 us); a 2+2+2
     // or 1+2+3 split measured slower at 8192^3 (7413-7416 us).
     constexpr int kL = T::NA + T::NB;
+    if constexpr (MASK) mask_k<WTM, WTN, T>(f1, 1, left);
     if (read_next) read_frag<WTM, WTN, T>(f0, As + nxt * T::A_STAGE, Bs + nxt * T::B_STAGE, 0, wm, wn, lane);
     mfma_frag_s<WTM, WTN, 0, 1>(acc, f1);
     interleave_reads<kReads>();
-    if (dma) dma_part<T, ALN, 0, kL / 2>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
+    if (dma) dma_part<T, false, 0, kL / 2, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
     mfma_frag_s<WTM, WTN, 1, 2>(acc, f1);
-    if (dma) dma_part<T, ALN, kL / 2, kL>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
+    if (dma) dma_part<T, false, kL / 2, kL, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
     mfma_frag_s<WTM, WTN, 2, 4>(acc, f1);
   } else {
-    if (dma) dma_slab<T, ALN>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
+    if (dma) dma_slab<T, false, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
     if (read_next) read_frag<WTM, WTN, T>(f0, As + nxt * T::A_STAGE, Bs + nxt * T::B_STAGE, 0, wm, wn, lane);
   }
 #pragma unroll
   for (int c = 2; c < C; ++c) {
     read_frag<WTM, WTN, T>(f1, sA, sB, c, wm, wn, lane);
+    if constexpr (MASK) mask_k<WTM, WTN, T>(f1, c, left);
     mfma_frag<WTM, WTN>(acc, f1);
   }
   if (PRIO) __builtin_amdgcn_s_setprio(0);
@@ -757,8 +791,9 @@ __device__ __forceinline__ void flat_step(AccOf<T> (&acc)[WTM][WTN], Frag<WTM, W
 // j % 3; slab ks of a tile fetches slab ks+2 of the same tile or, in the
 // tile's last two slabs, slab 0 or 1 of the next. The tile's C stores go
 // out after those fetches. Needs at least two slabs per tile (K > BK) and
-// fewer than 2^31 tiles.
-template <int WTM, int WTN, int BKT, bool PRIO, int WGM = 2, int WGN = 2, int MF = 32, bool ALN = false>
+// fewer than 2^31 tiles. KTAIL: K is no multiple of BK. WHOLE (not with
+// KTAIL): dma_part's.
+template <int WTM, int WTN, int BKT, bool PRIO, int WGM, int WGN, int MF, bool KTAIL, bool WHOLE>
 __device__ __forceinline__ void gemm_tiles_flat(const float *__restrict__ Ap, const float *__restrict__ Bp,
                                                 float *__restrict__ Cp, int64_t M, int64_t N, int64_t K,
                                                 int64_t lda, int64_t ldb, int64_t ldc, float *As, float *Bs) {
@@ -798,8 +833,8 @@ __device__ __forceinline__ void gemm_tiles_flat(const float *__restrict__ Ap, co
 
   int64_t cm0, cn0;
   coords(0, cm0, cn0);
-  dma_slab<T, ALN>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, 0, As, Bs, wv, lane);
-  dma_slab<T, ALN>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
+  dma_slab<T, false, WHOLE>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, 0, As, Bs, wv, lane);
+  dma_slab<T, false, WHOLE>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
   vm_barrier<T::NA + T::NB>();
   Frag<WTM, WTN> f0, f1;
   read_frag<WTM, WTN, T>(f0, As, Bs, 0, wm, wn, lane);
@@ -828,20 +863,23 @@ __device__ __forceinline__ void gemm_tiles_flat(const float *__restrict__ Ap, co
       // min(kStores, 62) are outstanding completes the loads and lets the
       // newest stores drain behind this tile's MFMAs.
       if (t > 0)
-        flat_step<WTM, WTN, T, PRIO, ALN, kStoreSlack>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0,
+        flat_step<WTM, WTN, T, PRIO, WHOLE, kStoreSlack>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0,
                                                        dk0, true, As, Bs, wv, wm, wn, lane);
       else
-        flat_step<WTM, WTN, T, PRIO, ALN>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0, dk0, true, As, Bs,
+        flat_step<WTM, WTN, T, PRIO, WHOLE>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0, dk0, true, As, Bs,
                                      wv, wm, wn, lane);
     }
     for (int64_t ks = 1; ks < ns - 2; ++ks)
-      flat_step<WTM, WTN, T, PRIO, ALN>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, true, cm0, cn0, (ks + 2) * BK,
+      flat_step<WTM, WTN, T, PRIO, WHOLE>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, true, cm0, cn0, (ks + 2) * BK,
                                       true, As, Bs, wv, wm, wn, lane);
     // The last two slabs (the last one only, when ns = 2) fetch the next
     // tile's slabs 0 and 1.
+    // With a partial last slab both mask A's k (all of the first of the two
+    // exist): one copy of the step's code, which is fetched cold.
     for (int64_t ks = ns > 2 ? ns - 2 : 1; ks < ns; ++ks)
-      flat_step<WTM, WTN, T, PRIO, ALN>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, has_next, nm0, nn0,
-                                      (ks + 2 - ns) * BK, ks + 1 < ns || has_next, As, Bs, wv, wm, wn, lane);
+      flat_step<WTM, WTN, T, PRIO, WHOLE, 0, KTAIL>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, has_next, nm0, nn0,
+                                                     (ks + 2 - ns) * BK, ks + 1 < ns || has_next, As, Bs, wv, wm, wn,
+                                                     lane, (int)(K - ks * BK));
     store_tile_buf<WTM, WTN, T>(acc, Cp, M, N, ldc, cm0, cn0, wm, wn, lane);
     cm0 = nm0;
     cn0 = nn0;
@@ -888,11 +926,14 @@ __device__ __forceinline__ void gemm_entry_pipe(const float *__restrict__ Ap, co
   gemm_body<WTM, WTN, BKT, PRIO, PIPE, WGM, WGN, MF>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
 }
 
-// Kernel body of the persistent variant: gemm_tiles_flat when A and B are
-// 16-byte aligned with k and n multiples of 4, K > BK and the tile offsets
-// fit 32 bits (its tail-free form when K and N are whole slabs and tiles);
-// the direct-to-LDS per-tile pipeline (or the generic path) otherwise. Same
-// LDS as gemm_entry_pipe's direct-to-LDS form.
+// Kernel body of the persistent variant: gemm_tiles_flat, at any alignment and
+// any N and K, when no row is shorter than its extent, K > BK and the tile
+// offsets fit 32 bits; the direct-to-LDS per-tile pipeline (or the generic
+// path) otherwise. Same LDS as gemm_entry_pipe's direct-to-LDS form. Shapes
+// whose K or N is no multiple of 4, or whose rows are not 16-byte aligned,
+// took the generic path before (guarded loads an element at a time, no
+// pipeline): 1000x1003x999 55.6 -> 24 us, 2047x2049x2051 360 -> 174,
+// 4000x4001x4002 1462 -> 917, 8191x8190x8189 11308 -> 7444.
 template <int WTM, int WTN, int BKT, bool PRIO, int WGM = 2, int WGN = 2, int MF = 32>
 __device__ __forceinline__ void gemm_entry_flat(const float *__restrict__ Ap, const float *__restrict__ Bp,
                                                 float *__restrict__ Cp, int64_t M, int64_t N, int64_t K, int64_t lda,
@@ -901,19 +942,20 @@ __device__ __forceinline__ void gemm_entry_flat(const float *__restrict__ Ap, co
   using L = LdsNeed<WTM, WTN, BKT, kPipeDma, WGM, WGN, MF>;
   __shared__ __attribute__((aligned(16))) float As[L::A];
   __shared__ __attribute__((aligned(16))) float Bs[L::B];
-  const bool vec = ((K & 3) == 0) && ((lda & 3) == 0) && kh::aligned16(Ap) && ((N & 3) == 0) &&
-                   ((ldb & 3) == 0) && kh::aligned16(Bp);
+  const bool rows = lda >= K && ldb >= N && ldc >= N;
   const bool fits32 = (int64_t)T::BM * lda * 4 < (1ll << 31) && (int64_t)T::BK * ldb * 4 < (1ll << 31) &&
                       (int64_t)T::BM * ldc * 4 < (1ll << 31);
   const int64_t tiles = ((M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN);
-  if (vec && fits32 && K > T::BK && tiles < (1ll << 31)) {
-    // Tail-free slab loads where no slab reaches past K or N: +2-3% at
-    // 8192^3, 4096^3 and 8192x8192x{256,1024} (their offsets stay in
-    // registers; the general form's selects spill them around the loop).
-    if (K % T::BK == 0 && N % T::BN == 0)
-      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, true>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+  if (rows && fits32 && K > T::BK && tiles < (1ll << 31)) {
+    // The 64-wide tiles at one workgroup per CU ran faster with the size of
+    // B's resource computed per slab (1024x1024x8192 151.0 vs 154.9 us), at
+    // two per CU without (3072^3 465 vs 455).
+    if (K % T::BK == 0 && T::BN < 128 && tiles <= KH_GEMM_CUS)
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, false, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+    else if (K % T::BK == 0)
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, false, true>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
     else
-      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, true, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
   } else {
     gemm_body<WTM, WTN, BKT, PRIO, kPipeDma, WGM, WGN, MF>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
   }

@@ -341,3 +341,37 @@ def test_tune_cache_steers_the_launcher(dev, tmp_path):
     finally:
         kh.set_tune_cache(None)
     assert kh.launch_symbol("gemm", shape) == default
+
+
+@pytest.mark.parametrize("sym,threads", [("gemm", 256), ("gemm_small", 512), ("gemm_wide", 512)])
+@pytest.mark.parametrize("m,n,k,grid", [
+    (65, 63, 33, 3),      # one k past a slab, every edge partial
+    (130, 257, 35, 5),    # 3 k past
+    (129, 127, 61, 2),    # a float4 of A with one k left
+    (300, 514, 97, 7),    # several slabs, tiles looped
+    (64, 256, 64, 1),     # whole slabs over odd strides
+    (1, 1, 1001, 1),
+])
+def test_gemm_persistent_any_alignment(dev, sym, threads, m, n, k, grid):
+    """The direct-to-LDS symbols at extents that are no multiple of 4, every
+    operand starting one float past a 16-byte boundary with odd row strides,
+    every pad and the floats around the operands NaN: integer inputs, so the
+    product must be exact bit for bit, and no pad read into it or written."""
+    lda, ldb, ldc = k + 1 + k % 2, n + 3 + n % 2, n + 2 + (n + 1) % 2
+    A, B = O.gemm_int_inputs(m, n, k)
+
+    def padded(x, ld):
+        p = np.full((x.shape[0], ld), np.nan, np.float32)
+        p[:, :x.shape[1]] = x
+        return np.concatenate([[np.float32(np.nan)], p.ravel()])
+
+    dA, dB, dC = up(padded(A, lda)), up(padded(B, ldb)), up(np.full(m * ldc + 1, np.nan, np.float32))
+    args = kh.LaunchArgs().add_memref(dA.ptr + 4, [m, k]).add_memref(dB.ptr + 4, [k, n])
+    args.add_memref(dC.ptr + 4, [m, n])
+    args.slots[5], args.slots[7 + 5], args.slots[14 + 5] = lda, ldb, ldc
+    f = kh.GpuModule(kh.code_object("gemm")).get_function(sym)
+    say(f"{sym} m={m} n={n} k={k} lda={lda} ldb={ldb} ldc={ldc} grid={grid}")
+    kh.kernel_launch(f, (grid, 1, 1), (threads, 1, 1), args)
+    C = down(dC, m * ldc + 1)[1:].reshape(m, ldc)
+    assert np.array_equal(C[:, :n], (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
+    assert np.isnan(C[:, n:]).all()
