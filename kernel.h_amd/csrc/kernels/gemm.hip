@@ -186,180 +186,47 @@ gemm_wide(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(flo
 }
 
 
-// 32x32 tiles with K split over the workgroup's waves (8 at the launcher's
+// Small tiles with K split over the workgroup's waves (8 at the launcher's
 // 512 threads; any 64..512 threads, a multiple of 64, are correct), for
 // launches whose larger tiles leave most CUs idle: 512^3 has 64 tiles of
-// 64x64 for 256 CUs, and 256 tiles of 32x32. Wave w of nw accumulates the
-// products of its K range (contiguous chunks of kc = 8 * ceil(K / (8 nw)))
-// straight from global memory into one v_mfma_f32_32x32x2f32 accumulator,
-// without LDS: lane l (r = l % 32, h = l / 32) loads the float4
-// A[m0 + r][k + 4h .. k + 4h + 3] and the four B[k + 4h + i][n0 + r], so MFMA
-// i of a group of 8 k sums k + i (lanes 0-31) and k + 4 + i (lanes 32-63):
-// every k of the group exactly once. Rows, columns and k past the matrix or
-// chunk edge load a clamped in-range address and are replaced by 0, so the
-// loads carry no branch. The partial tiles meet in LDS, and output register
-// i is summed by wave i % nw in the fixed order w0 + w1 + ... : the result
-// does not depend on timing. Measured against `gemm_small` (64x64 tiles):
-// 512^3 28-30 vs 18.0 TFLOP/s, 512x512x2048 37-41 vs 22, 256^3 6.3-6.5 vs
-// 3.8. Four waves per workgroup reached 22 at 512^3; sixteen spilled, and
-// so did loading 8 groups per batch (6 groups: slower at every shape).
+// 64x64 for 256 CUs, and 256 tiles of 32x32. Each wave accumulates the
+// products of its contiguous K range straight from global memory, without
+// LDS; the partial tiles meet in LDS, where every output is summed in the
+// fixed order w0 + w1 + ... : the result does not depend on timing.
 //
-// Where every tile is whole and every wave's K chunk a whole number of
-// batches (M, N multiples of 32, K of 128, 512 threads: the BASELINE 512^3),
-// the kernel takes a path of its own before the general one (ks_interior):
-// buffer loads with one offset register per operand and lane and the k step
-// in the scalar offset, none of them conditional. In the general path the
-// compiler turns each "clamped load, then select 0" into a branch around the
-// load and waits for it where the branches join, so a wave's loads went out
-// one at a time. Kernel trace, rotated inputs, same bits: 512^3 9.8 -> 6.2
-// us, 512x512x1024 16.4 -> 9.0, 256^3 5.7 -> 4.5; and, in the deep symbol,
-// 512x512x2048 25.6 -> 14.4, 512x512x8192 82 -> 49. Batches of 2 groups,
-// two sets in flight, measured best (4 groups: 6.8 us at 512^3, 8: 7.7;
-// three sets: 6.7).
+// Every load is an unconditional buffer load, at any alignment and extent
+// (ks_any): rows of A past M and rows of B past the wave's K range read 0
+// through the range check, columns of B past N are not stored, and A's k past
+// the range are zeroed in registers in the range's last batch. An earlier
+// form loaded a clamped address and selected 0 for lanes out of range; the
+// compiler turned each such pair into a branch around the load with a wait
+// where the branches join, so a wave's loads went out one at a time.
+//
+// What bounds it: a wave has two batches of loads in flight, and a tile's
+// time is its K range's batches at that latency, or its bytes of A and B at
+// the CU's share of the cache bandwidth. So the tile is chosen to give each
+// CU one workgroup (the launcher: the smallest tile with at most
+// KH_GEMM_CUS tiles). Events around rotated launches, 8 waves each,
+// 16x16 / 32x16 / 32x32 / 32x64 tiles, and the kernel these shapes ran
+// before (in us):
+//   16x4096x4096     17.6 / 19.3 / 23.9 / 38.4   89.7
+//   100x777x555       6.8 /  6.0 /  6.8 /  9.7   21.6
+//   2000x128x8192    84.3 / 70.6 / 48.8 / 73.3   187
+//   333x1000x2000    41.4 / 28.8 / 25.3 / 22.6   40.8 (64x64 tiles)
+//   8192x64x1000     21.1 / 18.9 / 15.5 / 14.6   22.9 (64x64 tiles)
+//   20x100x8000      26.1 / 34.2 / 43.9 / 70.5   107
+// Sixteen waves per workgroup and twice the loads in flight measured level;
+// B in dwordx2 and dwordx4 loads (a lane holding neighbouring columns) 5%
+// slower; 64x16 and 64x32 tiles never best.
 namespace {
 
 using khg::v16f;
+using khg::v4f;
 using kh::u32x4_t;
 constexpr int kKsTile = KH_GEMM_KSPLIT_BM;
 constexpr int kKsMaxWaves = KH_GEMM_KSPLIT_THREADS / 64;
-constexpr int kKsBatch = 4;  // groups of 8 k loaded ahead per batch
-constexpr int kKsFastBatch = 2;  // the same, in ks_interior
+constexpr int kKsFastBatch = 2;  // groups of 8 k loaded ahead per batch in ks_interior
 static_assert(KH_GEMM_KSPLIT_BM == 32 && KH_GEMM_KSPLIT_BN == 32, "one 32x32 MFMA accumulator per wave");
-
-// Loads one group of 8 k for this lane: k is the lane's first k of the
-// group (a multiple of 4 when VEC), K the end of the wave's chunk.
-template <bool VEC>
-__device__ __forceinline__ void ks_load(const float *__restrict__ A, const float *__restrict__ B, int64_t K,
-                                        int64_t lda, int64_t ldb, int64_t arow, int64_t bcol, bool arow_ok,
-                                        bool bcol_ok, int64_t k, float4 &a, float (&b)[4]) {
-  if constexpr (VEC) {
-    const bool ok = arow_ok && k < K;
-    const float4 t = *reinterpret_cast<const float4 *>(A + arow * lda + (k < K ? k : K - 4));
-    a = ok ? t : make_float4(0.f, 0.f, 0.f, 0.f);
-  } else {
-    float t[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int64_t kk = k + i;
-      const float v = A[arow * lda + (kk < K ? kk : K - 1)];
-      t[i] = (arow_ok && kk < K) ? v : 0.0f;
-    }
-    a = make_float4(t[0], t[1], t[2], t[3]);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t kk = k + i;
-    const float v = B[(kk < K ? kk : K - 1) * ldb + bcol];
-    b[i] = (bcol_ok && kk < K) ? v : 0.0f;
-  }
-}
-
-__device__ __forceinline__ void ks_mfma(v16f &acc, const float4 &a, const float (&b)[4]) {
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b[0], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b[1], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b[2], acc, 0, 0, 0);
-  acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b[3], acc, 0, 0, 0);
-}
-
-// NWC: the wave count when known at compile time (the launcher's 512
-// threads), else 0 and the count comes from blockDim. DEEP compiles in the
-// interior-tile path with three batches of loads in flight, for K chunks of
-// at least three batches.
-template <bool VEC, int NWC, bool DEEP>
-__device__ __forceinline__ void gemm_ksplit_body(const float *__restrict__ A, const float *__restrict__ B,
-                                                 float *__restrict__ C, int64_t M, int64_t N, int64_t K,
-                                                 int64_t lda, int64_t ldb, int64_t ldc, int bd, int64_t nblocks,
-                                                 float *red) {
-  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
-  const int nw = NWC > 0 ? NWC : bd / kh::kWave;  // whole waves; a partial last wave takes no k, no output
-  const int r = lane & 31, h = lane >> 5;
-  const int64_t tiles_m = (M + kKsTile - 1) / kKsTile, tiles_n = (N + kKsTile - 1) / kKsTile;
-  const int64_t total = tiles_m * tiles_n;
-  // DEEP chunks are whole batches of 4 groups (32 k).
-  const int64_t kc = DEEP ? 32 * ((K + 32 * nw - 1) / (32 * nw)) : 8 * ((K + 8 * nw - 1) / (8 * nw));
-  const int64_t kb = wave * kc, ke = kb + kc < K ? kb + kc : K;
-  const int64_t groups = ke > kb ? (ke - kb + 7) / 8 : 0;
-  for (int64_t t = blockIdx.x; t < total; t += nblocks) {
-    const int64_t m0 = (t / tiles_n) * kKsTile, n0 = (t % tiles_n) * kKsTile;
-    const bool arow_ok = m0 + r < M, bcol_ok = n0 + r < N;
-    const int64_t arow = arow_ok ? m0 + r : M - 1, bcol = bcol_ok ? n0 + r : N - 1;
-    v16f acc = {};
-    if (DEEP && VEC && m0 + kKsTile <= M && n0 + kKsTile <= N && ke - kb == kc && kc >= 3 * 32 &&
-        31 * lda + 8 <= (1 << 30) && (kc + 8) * ldb + 32 <= (1 << 30)) {
-      // Interior tile, a whole chunk of at least three batches: no clamps,
-      // and three batches of loads in flight (a ring of three register
-      // sets; the tail reloads the last batch and skips its math).
-      const uint32_t aoff = (uint32_t)(r * lda + 4 * h), boff = (uint32_t)(4 * h * ldb + r);
-      const float *abase = A + m0 * lda + kb, *bbase = B + kb * ldb + n0;
-      const int64_t nb = kc / 32;
-      struct Set {
-        float4 a[kKsBatch];
-        float b[kKsBatch][4];
-      };
-      Set f0, f1, f2;
-      auto fload = [&](Set &f, int64_t j) {
-#pragma unroll
-        for (int i = 0; i < kKsBatch; ++i) {
-          f.a[i] = *reinterpret_cast<const float4 *>(abase + (32 * j + 8 * i) + aoff);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) f.b[i][q] = (bbase + (32 * j + 8 * i + q) * ldb)[boff];
-        }
-      };
-      auto fmath = [&](const Set &f) {
-#pragma unroll
-        for (int i = 0; i < kKsBatch; ++i) ks_mfma(acc, f.a[i], f.b[i]);
-      };
-      fload(f0, 0);
-      fload(f1, 1);
-      for (int64_t j = 0; j < nb; j += 3) {
-        fload(f2, j + 2 < nb ? j + 2 : nb - 1);
-        fmath(f0);
-        fload(f0, j + 3 < nb ? j + 3 : nb - 1);
-        if (j + 1 < nb) fmath(f1);
-        fload(f1, j + 4 < nb ? j + 4 : nb - 1);
-        if (j + 2 < nb) fmath(f2);
-      }
-    } else {
-    float4 a0[kKsBatch], a1[kKsBatch];
-    float b0[kKsBatch][4], b1[kKsBatch][4];
-    auto load = [&](float4 (&a)[kKsBatch], float (&b)[kKsBatch][4], int64_t g) {
-#pragma unroll
-      for (int i = 0; i < kKsBatch; ++i) {
-        ks_load<VEC>(A, B, ke, lda, ldb, arow, bcol, arow_ok, bcol_ok, kb + 8 * (g + i) + 4 * h, a[i], b[i]);
-      }
-    };
-    auto math = [&](const float4 (&a)[kKsBatch], const float (&b)[kKsBatch][4]) {
-#pragma unroll
-      for (int i = 0; i < kKsBatch; ++i) ks_mfma(acc, a[i], b[i]);
-    };
-    // Batches of kKsBatch groups, double-buffered: the next batch's loads
-    // are issued before this batch's MFMAs. Groups past `groups` load
-    // clamped addresses and contribute 0.
-    if (groups > 0) load(a0, b0, 0);
-    int64_t g = 0;
-    for (; g + kKsBatch < groups; g += 2 * kKsBatch) {
-      load(a1, b1, g + kKsBatch);
-      math(a0, b0);
-      if (g + 2 * kKsBatch < groups) load(a0, b0, g + 2 * kKsBatch);
-      math(a1, b1);
-    }
-    if (g < groups) math(a0, b0);
-    }
-    // Partial tiles into LDS: red[wave][register][lane].
-#pragma unroll
-    for (int i = 0; i < 16; ++i) red[(wave * 16 + i) * kh::kWave + lane] = acc[i];
-    kh::lds_barrier();
-    if (wave < nw) {
-      for (int i = wave; i < 16; i += nw) {
-        float s = red[i * kh::kWave + lane];
-        for (int w = 1; w < nw; ++w) s += red[(16 * w + i) * kh::kWave + lane];
-        const int64_t gr = m0 + 8 * (i >> 2) + 4 * h + (i & 3), gc = n0 + r;
-        if (gr < M && gc < N) C[gr * ldc + gc] = s;
-      }
-    }
-    kh::lds_barrier();
-  }
-}
 
 // A uniform pointer, forced into scalar registers: its computation may run
 // on the vector ALU (the 64-bit multiply of a row index), and a buffer
@@ -372,12 +239,17 @@ __device__ __forceinline__ T *uniform_ptr(T *p) {
   return reinterpret_cast<T *>(((uint64_t)hi << 32) | lo);
 }
 
-// The K split for launches whose tiles are all whole: M, N multiples of 32,
+// 32x32 tiles for launches whose tiles are all whole: M, N multiples of 32,
 // K of 8 * kKsFastBatch * 8, eight waves, and every buffer span below 2^31
-// bytes, the largest record count a buffer resource holds (ks_interior_ok). The operands and groups are those of gemm_ksplit_body;
-// lane (r, h) reads A from one offset register plus 32 bytes per group (the
-// instruction's immediate) and B from one offset register plus a row step
-// in the scalar offset. Same reduction, so the same bits.
+// bytes, the largest record count a buffer resource holds (ks_interior_ok).
+// One v_mfma_f32_32x32x2f32 accumulator: lane l (r = l % 32, h = l / 32) loads
+// the float4 A[m0 + r][k + 4h .. k + 4h + 3] and the four B[k + 4h + i][n0 + r],
+// so MFMA i of a group of 8 k sums k + i (lanes 0-31) and k + 4 + i (lanes
+// 32-63): every k of the group exactly once. A comes from one offset register
+// plus 32 bytes per group (the instruction's immediate) and B from one offset
+// register plus a row step in the scalar offset. Batches of 2 groups, two
+// sets in flight, measured best (512^3: 6.2 us; 4 groups 6.8, 8 7.7, three
+// sets 6.7).
 __device__ __forceinline__ bool ks_interior_ok(int bd, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                                int64_t ldc, const float *A) {
   constexpr int64_t kLim = int64_t(1) << 29;
@@ -422,7 +294,12 @@ __device__ __forceinline__ void ks_interior(const float *__restrict__ A, const f
     };
     auto math = [&](const Set &s) {
 #pragma unroll
-      for (int i = 0; i < NB; ++i) ks_mfma(acc, s.a[i], s.b[i]);
+      for (int i = 0; i < NB; ++i) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[i].x, s.b[i][0], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[i].y, s.b[i][1], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[i].z, s.b[i][2], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(s.a[i].w, s.b[i][3], acc, 0, 0, 0);
+      }
     };
     // Two sets in flight: batch j + 1's loads go out before batch j's MFMAs.
     load(s0, 0);
@@ -446,55 +323,207 @@ __device__ __forceinline__ void ks_interior(const float *__restrict__ A, const f
   }
 }
 
-}  // namespace
+// The general form: tiles of TM x TN blocks of v_mfma_f32_16x16x4f32. In a
+// batch of 16 k, lane (r = l % 16, g = l / 16) loads the float4
+// A[16 i + r][k + 4g ..] of each row block and the four B[k + 4g + s][16 j + r]
+// of each column block; MFMA step s sums k + 4g + s over the lane groups.
+// NB batches per set of registers, two sets.
+template <int TM, int TN, int NB>
+struct KsSet {
+  float4 a[NB][TM];
+  float b[NB][TN][4];
+};
 
-template <bool DEEP>
-__device__ __forceinline__ void gemm_ksplit_entry(const float *Ap, const float *Bp, float *Cp, int64_t M, int64_t N,
-                                                  int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int bd,
-                                                  int64_t nb, float *red) {
-  const bool vec = ((K & 3) == 0) && ((lda & 3) == 0) && kh::aligned16(Ap);
-  if (bd == KH_GEMM_KSPLIT_THREADS) {
-    if (vec) {
-      gemm_ksplit_body<true, kKsMaxWaves, DEEP>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, bd, nb, red);
-    } else {
-      gemm_ksplit_body<false, kKsMaxWaves, DEEP>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, bd, nb, red);
+__device__ __forceinline__ bool ks_any_ok(int nw, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                          int64_t ldc) {
+  constexpr int64_t kLim = int64_t(1) << 29;  // floats of a 2^31-byte span
+  return nw > 0 && M > 0 && N > 0 && K > 0 && lda >= K && ldb >= N && M <= kLim && N <= kLim &&
+         64 * lda < kLim && (K / nw + 64) * ldb < kLim && ldc < kLim && ((M + 15) >> 4) * ((N + 15) >> 4) < kLim;
+}
+
+template <int TM, int TN, int NB>
+__device__ __forceinline__ void ks_any(const float *__restrict__ A, const float *__restrict__ B,
+                                       float *__restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb,
+                                       int64_t ldc, int nw, int nblocks, float *red) {
+  using Set = KsSet<TM, TN, NB>;
+  constexpr int R = 4 * TM * TN;  // accumulator registers
+  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int r = lane & 15, g = lane >> 4;
+  const int tiles_n = (N + 16 * TN - 1) / (16 * TN), total = ((M + 16 * TM - 1) / (16 * TM)) * tiles_n;
+  // The wave's K range: whole batches but for the last wave's.
+  const int kc = 16 * ((K + 16 * nw - 1) / (16 * nw)), kb = wave * kc, kn = kc < K - kb ? kc : K - kb;
+  uint32_t va[TM], vb[4];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) va[i] = (uint32_t)(((16 * i + r) * lda + 4 * g) * 4);
+#pragma unroll
+  for (int s = 0; s < 4; ++s) vb[s] = (uint32_t)(((4 * g + s) * ldb + r) * 4);
+  for (int pid = blockIdx.x; pid < total; pid += nblocks) {
+    // One tile per workgroup: neighbouring tiles on one XCD (workgroups go to
+    // the 8 XCDs round-robin), so that their rows of A and the two halves of
+    // a line of B meet in one L2.
+    int t = pid;
+    if (nblocks == total) {
+      const int x = pid & 7, per = total >> 3, extra = total & 7;
+      t = x * per + (x < extra ? x : extra) + (pid >> 3);
     }
-  } else if (vec) {
-    gemm_ksplit_body<true, 0, DEEP>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, bd, nb, red);
-  } else {
-    gemm_ksplit_body<false, 0, DEEP>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, bd, nb, red);
+    const int m0 = __builtin_amdgcn_readfirstlane(t / tiles_n) * 16 * TM;
+    const int n0 = __builtin_amdgcn_readfirstlane(t % tiles_n) * 16 * TN;
+    const int rows = M - m0 < 16 * TM ? M - m0 : 16 * TM;
+    v4f acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = v4f{};
+    if (kn > 0 && wave < nw) {
+      const __amdgpu_buffer_rsrc_t ra =
+          kh::span_rsrc(uniform_ptr(A + m0 * lda + kb), (uint32_t)(((rows - 1) * lda + K - kb) * 4));
+      const __amdgpu_buffer_rsrc_t rb =
+          kh::span_rsrc(uniform_ptr(B + kb * ldb + n0), (uint32_t)(((kn - 1) * ldb + N - n0) * 4));
+      auto load = [&](Set &f, int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          // In the vector offset: the range check does not cover the scalar one.
+          const uint32_t ao = (uint32_t)(k0 + 16 * u) * 4u, bo = (uint32_t)((k0 + 16 * u) * ldb) * 4u;
+#pragma unroll
+          for (int i = 0; i < TM; ++i) f.a[u][i] = kh::buf_load4(ra, va[i] + ao);
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              f.b[u][j][s] =
+                  __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rb, vb[s] + bo + 64u * j, 0, 0));
+        }
+      };
+      auto math = [&](Set &f, int k0) __attribute__((always_inline)) {
+        if (k0 + 16 * NB > kn) {
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            const int left = kn - k0 - 16 * u - 4 * g;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+              f.a[u][i] = make_float4(left > 0 ? f.a[u][i].x : 0.0f, left > 1 ? f.a[u][i].y : 0.0f,
+                                      left > 2 ? f.a[u][i].z : 0.0f, left > 3 ? f.a[u][i].w : 0.0f);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+              const float4 a = f.a[u][i];
+              const float av = s == 0 ? a.x : s == 1 ? a.y : s == 2 ? a.z : a.w;
+#pragma unroll
+              for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, f.b[u][j][s], acc[i][j], 0, 0, 0);
+            }
+      };
+      Set s0, s1;
+      load(s0, 0);
+      for (int k = 0; k < kn; k += 32 * NB) {
+        if (k + 16 * NB < kn) load(s1, k + 16 * NB);
+        math(s0, k);
+        if (k + 32 * NB < kn) load(s0, k + 32 * NB);
+        if (k + 16 * NB < kn) math(s1, k + 16 * NB);
+      }
+    }
+    // Partial tiles into LDS: red[wave][register][lane].
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[(wave * R + (i * TN + j) * 4 + q) * kh::kWave + lane] = acc[i][j][q];
+    kh::lds_barrier();
+    if (wave < nw) {
+      for (int x = wave; x < R; x += nw) {
+        float s = red[x * kh::kWave + lane];
+        for (int w = 1; w < nw; ++w) s += red[(R * w + x) * kh::kWave + lane];
+        const int gr = m0 + 16 * (x / (4 * TN)) + 4 * g + (x & 3), gc = n0 + 16 * ((x >> 2) % TN) + r;
+        if (gr < M && gc < N) C[gr * ldc + gc] = s;
+      }
+    }
+    kh::lds_barrier();
   }
 }
 
+// Any strides and spans, an element at a time: launches ks_any_ok turns down.
+// Summed in runs of 1024 k, so that a long K costs no precision.
+__device__ __forceinline__ void ks_plain(const float *__restrict__ A, const float *__restrict__ B,
+                                         float *__restrict__ C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                                         int64_t ldb, int64_t ldc, int64_t threads, int64_t nblocks) {
+  for (int64_t e = (int64_t)blockIdx.x * threads + threadIdx.x; e < M * N; e += nblocks * threads) {
+    const float *a = A + (e / N) * lda, *b = B + e % N;
+    float total = 0.0f;
+    for (int64_t k0 = 0; k0 < K; k0 += 1024) {
+      float s = 0.0f;
+      for (int64_t k = k0; k < K && k < k0 + 1024; ++k) s = fmaf(a[k], b[k * ldb], s);
+      total += s;
+    }
+    C[(e / N) * ldc + e % N] = total;
+  }
+}
+
+}  // namespace
+
 // The arguments the K-split kernels use, loaded in one round (KH_ARGS_READY):
-// at 512^3 the launch is ~10 us, and every serial round trip to
+// at 512^3 the launch is ~6 us, and every serial round trip to
 // kernel-argument memory before the first operand load is part of it.
-#define KH_KSPLIT_ENTRY(DEEP)                                                                                  \
+#define KH_KSPLIT_ARGS()                                                                                       \
   const uint32_t gw = kh::group_size_word(), gz = kh::group_size_z_word(), nb = kh::grid_blocks_x();          \
-  KH_ARGS_READY(A_base, A_off, A_n0, A_n1, A_s0, B_base, B_off, B_n1, B_s0, C_base, C_off, C_s0, gw, gz, nb); \
+  KH_ARGS_READY(A_base, A_off, A_n0, A_n1, A_s0, B_base, B_off, B_n1, B_s0, C_base, C_off, C_s0, gw, gz, nb)
+
+#define KH_KSPLIT_ANY(TM, TN, NB)                                                                              \
+  const int nw = (int)kh::threads_x_of(gw) / kh::kWave; /* a partial last wave takes no k and no output */    \
+  if (ks_any_ok(nw, A_n0, B_n1, A_n1, A_s0, B_s0, C_s0))                                                      \
+    ks_any<TM, TN, NB>(KH_PTR(A), KH_PTR(B), KH_PTR(C), (int)A_n0, (int)B_n1, (int)A_n1, A_s0, B_s0, C_s0,    \
+                       nw, (int)nb, red);                                                                     \
+  else                                                                                                        \
+    ks_plain(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, kh::threads_x_of(gw), nb)
+
+// 32x32 tiles: the whole-tile form where it applies, else the general one.
+#define KH_KSPLIT_32X32(NB)                                                                                    \
+  __shared__ float red[kKsMaxWaves * 16 * 64];                                                                 \
+  KH_KSPLIT_ARGS();                                                                                            \
   if (kh::threads_y_of(gw) == 1 && kh::threads_z_of(gz) == 1 &&                                               \
       ks_interior_ok((int)kh::threads_x_of(gw), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, KH_PTR(A))) {             \
     ks_interior(KH_PTR(A), KH_PTR(B), KH_PTR(C), (int)A_n0, (int)B_n1, (int)A_n1, (int)A_s0, (int)B_s0,       \
                 (int)C_s0, (int)nb, red);                                                                    \
     return;                                                                                                   \
   }                                                                                                           \
-  gemm_ksplit_entry<DEEP>(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0,                \
-                          (int)kh::threads_x_of(gw), nb, red)
+  KH_KSPLIT_ANY(2, 2, NB)
 
 extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
-  __shared__ float red[kKsMaxWaves * 16 * 64];
-  KH_KSPLIT_ENTRY(false);
+  KH_KSPLIT_32X32(1);
 }
 
-// Same tiles and split with the deep-chunk path compiled in: the launcher
-// takes it over `gemm_ksplit` for K >= KH_GEMM_KSPLIT_DEEP_K. A kernel of
-// its own: compiled into `gemm_ksplit`, the extra registers slowed the
-// short-chunk path (512^3: 28 -> 18 TFLOP/s). Measured against it:
-// 512x512x2048 42 vs 37 TFLOP/s, 512x512x8192 54 vs 40; at K = 1024 the two
-// were level.
+// The same with twice the loads in flight in the general form: the launcher
+// takes it over `gemm_ksplit` for K >= KH_GEMM_KSPLIT_DEEP_K (2000x128x8192
+// and 16x8192x8192 within 3% of each other either way).
 extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit_deep(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
-  __shared__ float red[kKsMaxWaves * 16 * 64];
-  KH_KSPLIT_ENTRY(true);
+  KH_KSPLIT_32X32(2);
+}
+
+// Smaller tiles, for fewer rows or columns, and one larger.
+extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
+gemm_ksplit_16x16(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
+  __shared__ float red[kKsMaxWaves * 4 * 64];
+  KH_KSPLIT_ARGS();
+  KH_KSPLIT_ANY(1, 1, 2);
+}
+
+extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
+gemm_ksplit_32x16(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
+  __shared__ float red[kKsMaxWaves * 8 * 64];
+  KH_KSPLIT_ARGS();
+  KH_KSPLIT_ANY(2, 1, 2);
+}
+
+extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
+gemm_ksplit_32x64(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
+  __shared__ float red[kKsMaxWaves * 32 * 64];
+  KH_KSPLIT_ARGS();
+  KH_KSPLIT_ANY(2, 4, 1);
 }

@@ -67,20 +67,22 @@
 #define KH_GEMM_RATE_MID 135
 #define KH_GEMM_RATE_WIDE 137
 #define KH_GEMM_RATE_SMALL 126
-// `gemm_ksplit`: 32x32 tiles, K split over the 8 waves of a 512-thread
-// workgroup. The launcher takes it when its tiles fit one round (at most
-// one workgroup per CU): there the larger tiles leave three CUs in four idle.
-// It also takes it where the 64x64 tiles number fewer than the CUs and
-// every 32x32 tile is whole with K a multiple of KH_GEMM_KSPLIT_INTERIOR_K
-// (the K-split symbols' unconditional-load path), from
+// K split over the 8 waves of a 512-thread workgroup, in tiles of 16x16,
+// 32x16, 32x32 (`gemm_ksplit`, `gemm_ksplit_deep`) and 32x64. The launcher
+// takes the smallest of them with at most KH_GEMM_CUS tiles: more, smaller
+// tiles leave each CU several workgroups that read the same operands again
+// (100x777x555: 343 tiles of 16x16 6.8 us, 196 of 32x16 6.0), fewer, larger
+// ones leave CUs idle (16x4096x4096: 17.6 us in 256 tiles, 23.9 in 128).
+// 32x32 tiles are also taken beyond one round where the 64x64 tiles number
+// fewer than the CUs and every 32x32 tile is whole with K a multiple of
+// KH_GEMM_KSPLIT_INTERIOR_K (the whole-tile form), from
 // KH_GEMM_KSPLIT_MIN_K on; the workgroups then loop over their tiles.
-// Kernel trace, rotated inputs, against the four-wave register-staged
-// 64x64 tiles `gemm_small` then had: 640^3 11.5 vs 18.0 us, 768^3 18.0 vs
-// 21.2, 1024x512x512 10.2 vs 15.2, 256x2048x2048 25.5 vs 50.3,
-// 512x1536x1024 21.5 vs 27.4; level at 768x768x256 and 896^3; at 1024^3
-// (256 tiles of 64x64) level, at 1024x1024x512 slower (17.3 vs 15.9).
-// Against the persistent eight-wave `gemm_small`: 768^3 level (18.0 vs
-// 17.8), 512x512x2048 14.6 vs 40.4.
+// Kernel trace, rotated inputs, against the 64x64 tiles `gemm_small` then
+// had: 640^3 11.5 vs 18.0 us, 1024x512x512 10.2 vs 15.2, 256x2048x2048 25.5
+// vs 50.3; level at 768x768x256 and 896^3; at 1024x1024x512 slower (17.3 vs
+// 15.9). Against the persistent eight-wave `gemm_small`: 768^3 level (18.0
+// vs 17.8), 512x512x2048 14.6 vs 40.4; 32x64 against it: 333x1000x2000 22.6
+// vs 40.8, 513x511x509 8.6 vs 13.8.
 #define KH_GEMM_KSPLIT_BM 32
 #define KH_GEMM_KSPLIT_BN 32
 #define KH_GEMM_KSPLIT_THREADS 512

@@ -187,11 +187,12 @@ struct GemmCandidate {
   // Persistent symbols: workgroups resident per CU (their LDS and
   // registers), so the launcher's grid is one round of them.
   int per_cu = 2;
+  int ks_bm = KH_GEMM_KSPLIT_BM, ks_bn = KH_GEMM_KSPLIT_BN;  // K-split symbols' tiles
   bool ksplit() const { return pipe == kKsplit || pipe == kKsplitDeep; }
-  // K-split: each of the 8 waves holds the whole 32x32 tile for its K range.
+  // K-split: each of the 8 waves holds the whole tile for its K range.
   int waves() const { return ksplit() ? KH_GEMM_KSPLIT_THREADS / 64 : wgm * wgn; }
-  int bm() const { return ksplit() ? KH_GEMM_KSPLIT_BM : mfma * wtm * wgm; }
-  int bn() const { return ksplit() ? KH_GEMM_KSPLIT_BN : mfma * wtn * wgn; }
+  int bm() const { return ksplit() ? ks_bm : mfma * wtm * wgm; }
+  int bn() const { return ksplit() ? ks_bn : mfma * wtn * wgn; }
   // Slabs (K-split: batches of 32 k) in flight ahead of the MFMAs.
   int unroll() const { return pipe == kRegs ? 1 : pipe == kKsplitDeep ? 3 : 2; }
 };
@@ -211,8 +212,18 @@ const GemmCandidate kGemmCandidates[] = {
 constexpr int kGemmCandidateCount = static_cast<int>(sizeof(kGemmCandidates) / sizeof(kGemmCandidates[0]));
 static_assert(kGemmCandidateCount == 7 + KH_GEMM_TUNE_COUNT, "candidate table");
 
+// K-split tiles that only the launcher picks, smallest first.
+const GemmCandidate kKsplitTiles[] = {
+    {"gemm_ksplit_16x16", "gemm", 16, 1, 1, 1, 1, 16, 0, kKsplit, true, 2, 16, 16},
+    {"gemm_ksplit_32x16", "gemm", 16, 1, 1, 2, 1, 16, 0, kKsplit, true, 2, 32, 16},
+    {"gemm_ksplit_32x64", "gemm", 16, 1, 1, 2, 4, 16, 0, kKsplit, true, 2, 32, 64},
+};
+
 const GemmCandidate *find_gemm_candidate(const char *symbol) {
   if (symbol == nullptr) return nullptr;
+  for (const auto &c : kKsplitTiles) {
+    if (std::strcmp(c.symbol, symbol) == 0) return &c;
+  }
   for (const auto &c : kGemmCandidates) {
     if (std::strcmp(c.symbol, symbol) == 0) return &c;
   }
@@ -332,12 +343,20 @@ double gemm_score(int64_t tiles, int64_t round, double rate) {
 }
 
 const char *heuristic_gemm_symbol(int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles64 = ceil_div(m, KH_GEMM_SMALL_BM) * ceil_div(n, KH_GEMM_SMALL_BN);
-  if (ceil_div(m, KH_GEMM_KSPLIT_BM) * ceil_div(n, KH_GEMM_KSPLIT_BN) <= KH_GEMM_CUS ||
-      (tiles64 < KH_GEMM_CUS && m % KH_GEMM_KSPLIT_BM == 0 && n % KH_GEMM_KSPLIT_BN == 0 &&
-       k % KH_GEMM_KSPLIT_INTERIOR_K == 0 && k >= KH_GEMM_KSPLIT_MIN_K)) {
-    return k >= KH_GEMM_KSPLIT_DEEP_K ? "gemm_ksplit_deep" : "gemm_ksplit";
+  // K split (kh_tiles.h): the smallest tile that gives every CU at most one
+  // workgroup; of 32x32 tiles also more, where all are whole and the 64x64
+  // tiles number fewer than the CUs.
+  auto ks_tiles = [&](int64_t bm, int64_t bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
+  const char *ks32 = k >= KH_GEMM_KSPLIT_DEEP_K ? "gemm_ksplit_deep" : "gemm_ksplit";
+  const int64_t tiles64 = ks_tiles(KH_GEMM_SMALL_BM, KH_GEMM_SMALL_BN);
+  if (ks_tiles(16, 16) <= KH_GEMM_CUS) return "gemm_ksplit_16x16";
+  if (ks_tiles(32, 16) <= KH_GEMM_CUS) return "gemm_ksplit_32x16";
+  if (ks_tiles(KH_GEMM_KSPLIT_BM, KH_GEMM_KSPLIT_BN) <= KH_GEMM_CUS) return ks32;
+  if (tiles64 < KH_GEMM_CUS && m % KH_GEMM_KSPLIT_BM == 0 && n % KH_GEMM_KSPLIT_BN == 0 &&
+      k % KH_GEMM_KSPLIT_INTERIOR_K == 0 && k >= KH_GEMM_KSPLIT_MIN_K) {
+    return ks32;
   }
+  if (ks_tiles(32, 64) <= KH_GEMM_CUS) return "gemm_ksplit_32x64";
   const double big = gemm_score(ceil_div(m, KH_GEMM_BM) * ceil_div(n, KH_GEMM_BN), KH_GEMM_ROUND_BIG,
                                 KH_GEMM_RATE_BIG);
   const double mid = gemm_score(ceil_div(m, KH_GEMM_MID_BM) * ceil_div(n, KH_GEMM_MID_BN), KH_GEMM_ROUND_MID,

@@ -375,3 +375,64 @@ def test_gemm_persistent_any_alignment(dev, sym, threads, m, n, k, grid):
     C = down(dC, m * ldc + 1)[1:].reshape(m, ldc)
     assert np.array_equal(C[:, :n], (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
     assert np.isnan(C[:, n:]).all()
+
+
+@pytest.mark.parametrize("sym", ["gemm_ksplit", "gemm_ksplit_deep", "gemm_ksplit_16x16", "gemm_ksplit_32x16",
+                                 "gemm_ksplit_32x64"])
+@pytest.mark.parametrize("m,n,k,grid,block", [
+    (1, 1, 1, 1, 512),        # one k for the first wave, none for the others
+    (17, 15, 16, 2, 512),     # one whole batch
+    (33, 65, 129, 7, 512),    # edges of every tile; nine waves' worth of k for eight
+    (16, 64, 640, 4, 512),    # whole tiles of some symbols, whole batches
+    (50, 130, 1023, 500, 512),  # a partial last batch; more workgroups than tiles
+    (50, 130, 1023, 3, 192),  # three waves, tiles looped
+    (31, 31, 47, 1, 64),      # one wave
+])
+def test_gemm_ksplit_any_shape(dev, sym, m, n, k, grid, block):
+    """Every K-split symbol over odd strides and addresses, pads NaN, inputs
+    small integers (exact whatever the order); a last column of A next to a
+    row of infinities in the pads of the following row must not leak."""
+    lda, ldb, ldc = k + 3, n + 1, n + 2
+    A, B = O.gemm_int_inputs(m, n, k)
+    Ap = np.full((m, lda), np.inf, np.float32)
+    Ap[:, :k] = A
+    Bp = np.full((k, ldb), np.nan, np.float32)
+    Bp[:, :n] = B
+    one = np.full(1, np.nan, np.float32)
+    dA, dB = up(np.concatenate([one, Ap.ravel()])), up(np.concatenate([one, Bp.ravel()]))
+    dC = up(np.full(m * ldc + 1, -7.0, np.float32))
+    args = kh.LaunchArgs().add_memref(dA.ptr + 4, [m, k]).add_memref(dB.ptr + 4, [k, n])
+    args.add_memref(dC.ptr + 4, [m, n])
+    args.slots[5], args.slots[7 + 5], args.slots[14 + 5] = lda, ldb, ldc
+    f = kh.GpuModule(kh.code_object("gemm")).get_function(sym)
+    say(f"{sym} m={m} n={n} k={k} grid={grid} block={block}")
+    kh.kernel_launch(f, (grid, 1, 1), (block, 1, 1), args)
+    C = down(dC, m * ldc + 1)[1:].reshape(m, ldc)
+    assert np.array_equal(C[:, :n], (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
+    assert np.all(C[:, n:] == -7.0)
+
+
+@pytest.mark.parametrize("m,n,k,symbol", [
+    (16, 4096, 4096, "gemm_ksplit_16x16"), (17, 4096, 4096, "gemm_ksplit_32x16"),
+    (100, 777, 555, "gemm_ksplit_32x16"), (333, 1000, 2000, "gemm_ksplit_32x64"),
+    (1, 1, 1, "gemm_ksplit_16x16"), (8192, 16, 500, "gemm_ksplit_32x16"),
+])
+def test_gemm_ksplit_tile_choice(dev, m, n, k, symbol):
+    assert kh.launch_symbol("gemm", f"m={m},n={n},k={k}") == symbol
+    A, B = O.gemm_int_inputs(m, n, k)
+    C = _gemm(A, B, m, n, k)
+    assert np.array_equal(C, (A.astype(np.float64) @ B.astype(np.float64)).astype(np.float32))
+
+
+def test_gemm_ksplit_broadcast_rows(dev):
+    # Rows of A and B all the same memory (stride 0): the element form.
+    m, n, k = 20, 30, 100
+    A, B = O.gemm_int_inputs(1, n, k)
+    dA, dB, dC = up(A), up(B[:1]), empty(m * n)
+    args = kh.LaunchArgs().add_memref(dA, [m, k]).add_memref(dB, [k, n]).add_memref(dC, [m, n])
+    args.slots[5] = args.slots[7 + 5] = 0
+    f = kh.GpuModule(kh.code_object("gemm")).get_function("gemm_ksplit")
+    say("gemm_ksplit broadcast rows")
+    kh.kernel_launch(f, (4, 1, 1), (512, 1, 1), args)
+    want = np.repeat(A.astype(np.float64), m, 0) @ np.repeat(B[:1].astype(np.float64), k, 0)
+    assert np.array_equal(down(dC, m * n).reshape(m, n), want.astype(np.float32))
