@@ -348,6 +348,290 @@ __device__ __forceinline__ void attention_slice(const float *__restrict__ Qg, co
   }
 }
 
+// ---------------------------------------------------------------------------
+// Keys split over the waves of a workgroup (`attention_split`): every wave
+// holds the same 16 TQ query rows and runs the online softmax over its own
+// range of keys, K and V straight from global memory; the waves' (m, l, O)
+// meet in LDS at the end. No tile is shared, so there are no barriers in the
+// loop.
+//
+// For launches whose 128-row tiles leave much of the chip idle, where one
+// wave's serial chain of key tiles is the time: with 128 rows per workgroup,
+// batch 1, 8 heads, 777 keys is 56 workgroups, a wave on 224 of 1024 SIMDs
+// with 13 tiles of 4.4 us each. What bounds it then is the MFMAs of the
+// waves there are (a step of 32 queries x 32 keys is 1.7 us of them and takes
+// 2.2), and the start and the merge, about 5 us. Events around rotated
+// launches, attention / attention_split (32 rows) / attention_split16, us:
+//   b1 h8  s777      58.6 / 20.8 / 22.3      b1 h1  s64      8.3 /  7.0 / 5.1
+//   b1 h16 s1024     71.1 / 40.6 / 45.9      b1 h1  s4096  266   / 73.6 / 46.9
+//   b4 h16 s256      22.3 / 15.9 / 18.3      b3 h12 s1100  149   / 101  / 114
+//   b4 h16 s512      39.8 / 44.5 / 51.2      b4 h16 s1024  133   / 145  / 163
+// Eight waves per workgroup measured level or slower.
+//
+// MFMA formulation, v_mfma_f32_16x16x4f32, per 16 keys (lane r = l % 16,
+// g = l / 16):
+//   S^T = K Q^T        A: K[key r][16c + 4g + st], one float4 per c; B: Q
+//                      likewise. The result's lane holds query r and keys
+//                      4g .. 4g + 3.
+//   O^T += V^T P^T     B = the P registers as the first product left them:
+//                      step st sums keys 4g + st over the lane groups. A:
+//                      V[key 4g + st][4r + dt], one float4 per step, so that
+//                      row r of block dt is head-dim element 4r + dt and a
+//                      lane ends with whole float4s of O.
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr int SK = 32;       // keys per step
+constexpr int LDO = D + 4;   // merged O in LDS: [wave][query][d], padded rows
+
+// The maximum over the four lanes of a query (l, l ^ 16, l ^ 32, l ^ 48): two
+// register swaps between lane rows, no LDS round trip.
+__device__ __forceinline__ float across_max(float v) {
+  const uint32_t u = __float_as_uint(v);
+  auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const uint32_t w = __float_as_uint(m);
+  auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
+template <int TQ>
+__device__ __forceinline__ void attention_split_tile(__amdgpu_buffer_rsrc_t rq, __amdgpu_buffer_rsrc_t rk,
+                                                     __amdgpu_buffer_rsrc_t rv, __amdgpu_buffer_rsrc_t ro, int qs,
+                                                     int ks, int vs, int os, int seq, int q0, int nw, int wave,
+                                                     int lane, float *ml, float *Ob) {
+  constexpr int NQ = 16 * TQ;
+  const int r = lane & 15, g = lane >> 4;
+  const float qscale = kh::kLog2e * 0.125f;
+  const int steps = (seq + SK - 1) / SK, per = (steps + nw - 1) / nw;
+  const int t0 = wave * per, t1 = t0 + per < steps ? t0 + per : steps;
+  float4 q[TQ][4], k[2][4], v[2][4];
+  v4f o[TQ][4];
+  float m[TQ], l[TQ];
+  // Offsets are a lane term, plus a step's term kept opaque: left to itself
+  // the compiler carries an induction register for every load of the loop.
+  const uint32_t ko = (uint32_t)((r * ks + 4 * g) * 4), vo = (uint32_t)((4 * g * vs + 4 * r) * 4);
+  auto load_k = [&](int t) __attribute__((always_inline)) {
+    uint32_t at = (uint32_t)(t * SK * ks) * 4u;
+    asm volatile("" : "+s"(at));
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const uint32_t off = ko + (at + (uint32_t)(16 * b * ks) * 4u);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) k[b][c] = kh::buf_load4(rk, off + 64u * c);
+    }
+  };
+  auto load_v = [&](int t) __attribute__((always_inline)) {
+    uint32_t at = (uint32_t)(t * SK * vs) * 4u;
+    asm volatile("" : "+s"(at));
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+        v[b][st] = kh::buf_load4(rv, vo + (at + (uint32_t)((16 * b + st) * vs) * 4u));
+  };
+  load_k(t0);
+#pragma unroll
+  for (int i = 0; i < TQ; ++i)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) q[i][c] = kh::buf_load4(rq, (uint32_t)(((q0 + 16 * i + r) * qs + 16 * c + 4 * g) * 4));
+  load_v(t0);
+#pragma unroll
+  for (int i = 0; i < TQ; ++i) {
+    m[i] = kNegBig;
+    l[i] = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[i][dt] = v4f{};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      q[i][c] = make_float4(q[i][c].x * qscale, q[i][c].y * qscale, q[i][c].z * qscale, q[i][c].w * qscale);
+  }
+  auto scores = [&](v4f (&s)[TQ][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TQ; ++i)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) s[i][b] = v4f{};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int i = 0; i < TQ; ++i)
+            s[i][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(comp(k[b][c], st), comp(q[i][c], st), s[i][b], 0, 0, 0);
+  };
+  auto softmax = [&](v4f (&s)[TQ][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TQ; ++i) {
+      float mt = m[i];
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mt = fmaxf(mt, s[i][b][j]);
+      mt = across_max(mt);
+      const float alpha = kh::exp2_hw(m[i] - mt);
+      m[i] = mt;
+      float ls = 0.0f;
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          s[i][b][j] = kh::exp2_hw(s[i][b][j] - mt);
+          ls += s[i][b][j];
+        }
+      l[i] = l[i] * alpha + ls;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[i][dt][j] *= alpha;
+    }
+  };
+  auto accumulate = [&](v4f (&s)[TQ][2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int st = 0; st < 4; ++st)
+#pragma unroll
+        for (int i = 0; i < TQ; ++i)
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt)
+            o[i][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(comp(v[b][st], dt), s[i][b][st], o[i][dt], 0, 0, 0);
+  };
+  // One step: the next step's S^T, while whose MFMAs run this one's softmax
+  // takes the vector ALU, then this one's P V. Each load goes out as soon as
+  // its registers' last readers have been issued (K past the last key reads 0
+  // and is not used); only vector and scalar arithmetic moves across those
+  // points. Unrolled by two: copying the scores instead cost 8%.
+  auto step = [&](int t, v4f (&sc)[TQ][2], v4f (&sn)[TQ][2]) __attribute__((always_inline)) {
+    scores(sn);
+    load_k(t + 2);
+    __builtin_amdgcn_sched_barrier(0x6);
+    softmax(sc);
+    accumulate(sc);
+    load_v(t + 1);
+    __builtin_amdgcn_sched_barrier(0x6);
+  };
+  // The range's last step, the only one that can reach past the last key.
+  auto finish = [&](int t, v4f (&s)[TQ][2]) __attribute__((always_inline)) {
+    if ((t + 1) * SK > seq) {
+#pragma unroll
+      for (int i = 0; i < TQ; ++i)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (t * SK + 16 * b + 4 * g + j >= seq) s[i][b][j] = -__builtin_inff();
+    }
+    softmax(s);
+    accumulate(s);
+  };
+  v4f sa[TQ][2], sb[TQ][2];
+  if (t0 < t1) {
+    scores(sa);
+    load_k(t0 + 1);
+    int t = t0;
+    for (; t + 2 < t1; t += 2) {
+      step(t, sa, sb);
+      step(t + 1, sb, sa);
+    }
+    if (t + 1 < t1) {
+      step(t, sa, sb);
+      finish(t + 1, sb);
+    } else {
+      finish(t, sa);
+    }
+  }
+  // Merge: each wave scales its O to the common maximum, then every thread
+  // sums its share of the outputs over the waves.
+#pragma unroll
+  for (int i = 0; i < TQ; ++i) {
+    l[i] += __shfl_xor(l[i], 16, kh::kWave);
+    l[i] += __shfl_xor(l[i], 32, kh::kWave);
+    if (g == 0) {
+      ml[(wave * NQ + 16 * i + r) * 2] = m[i];
+      ml[(wave * NQ + 16 * i + r) * 2 + 1] = l[i];
+    }
+  }
+  kh::lds_barrier();
+#pragma unroll
+  for (int i = 0; i < TQ; ++i) {
+    float mm = m[i];
+    for (int w = 0; w < nw; ++w) mm = fmaxf(mm, ml[(w * NQ + 16 * i + r) * 2]);
+    const float f = kh::exp2_hw(m[i] - mm);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *reinterpret_cast<float4 *>(Ob + (wave * NQ + 16 * i + r) * LDO + 16 * g + 4 * j) =
+          make_float4(o[i][0][j] * f, o[i][1][j] * f, o[i][2][j] * f, o[i][3][j] * f);
+  }
+  kh::lds_barrier();
+  for (int e = threadIdx.x; e < NQ * (D / 4); e += nw * kh::kWave) {
+    const int qr = e >> 4, d4 = e & 15;
+    float mm = ml[qr * 2];
+    for (int w = 1; w < nw; ++w) mm = fmaxf(mm, ml[(w * NQ + qr) * 2]);
+    float lt = 0.0f;
+    float4 a = make_float4(0, 0, 0, 0);
+    for (int w = 0; w < nw; ++w) {
+      lt += ml[(w * NQ + qr) * 2 + 1] * kh::exp2_hw(ml[(w * NQ + qr) * 2] - mm);
+      const float4 b = *reinterpret_cast<const float4 *>(Ob + (w * NQ + qr) * LDO + 4 * d4);
+      a = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+    }
+    const float inv = 1.0f / lt;
+    const u32x4 u = {__float_as_uint(a.x * inv), __float_as_uint(a.y * inv), __float_as_uint(a.z * inv),
+                     __float_as_uint(a.w * inv)};
+    const uint32_t off = (uint32_t)(((q0 + qr) * os + 4 * d4) * 4);
+    __builtin_amdgcn_raw_buffer_store_b128(u, ro, q0 + qr < seq ? off : kh::kOutside, 0, 0);
+  }
+  kh::lds_barrier();
+}
+
+// The template's contract (attention.cpp:109-120 refuses other shapes): four
+// [batch, heads, seq, 64] tensors with contiguous head_dim rows. Anything else
+// is refused by filling O (as its descriptor describes it) with NaN, never by
+// computing from memory the descriptors do not cover. Evaluated without
+// short-circuit branches (& and |, not && and ||): the compiler then issues
+// every descriptor load in one round at the start instead of one round per
+// branch.
+__device__ __forceinline__ void attention_refuse(float *__restrict__ Op, int64_t n0, int64_t n1, int64_t n2,
+                                                 int64_t n3, int64_t s0, int64_t s1, int64_t s2, int64_t s3,
+                                                 uint32_t gxy, uint32_t bcx) {
+  const int64_t total = n0 * n1 * n2 * n3;
+  const int64_t tx = kh::threads_x_of(gxy), ty = kh::threads_y_of(gxy), tz = kh::threads_z_of(kh::group_size_z_word());
+  const int64_t gy = kh::grid_blocks_y(), gz = kh::grid_blocks_z();
+  const int64_t threads = tx * ty * tz;
+  const int64_t flat = ((int64_t)threadIdx.z * ty + threadIdx.y) * tx + threadIdx.x;
+  const int64_t block = ((int64_t)blockIdx.z * gy + blockIdx.y) * bcx + blockIdx.x;
+  const int64_t step = threads * bcx * gy * gz;
+  for (int64_t e = block * threads + flat; e < total; e += step) {
+    int64_t r = e;
+    const int64_t i3 = r % n3;
+    r /= n3;
+    const int64_t i2 = r % n2;
+    r /= n2;
+    Op[(r / n1) * s0 + (r % n1) * s1 + i2 * s2 + i3 * s3] = __builtin_nanf("");
+  }
+}
+
+// Pointers, extents and the refusal above, the check's loads, the base
+// pointers and the launch geometry in one round.
+#define KH_ATTN_CHECK(...)                                                                                     \
+  const float *__restrict__ Qp = KH_PTR(Q);                                                                    \
+  const float *__restrict__ Kp = KH_PTR(K);                                                                    \
+  const float *__restrict__ Vp = KH_PTR(V);                                                                    \
+  float *__restrict__ Op = KH_PTR(O);                                                                          \
+  const int64_t heads = Q_n1, seq = Q_n2;                                                                      \
+  const bool same = (K_n0 == Q_n0) & (V_n0 == Q_n0) & (O_n0 == Q_n0) & (K_n1 == heads) & (V_n1 == heads) &     \
+                    (O_n1 == heads) & (K_n2 == seq) & (V_n2 == seq) & (O_n2 == seq);                           \
+  const bool d64 = (Q_n3 == D) & (K_n3 == D) & (V_n3 == D) & (O_n3 == D);                                      \
+  const bool rows = ((Q_s3 == 1) | (Q_n3 <= 1)) & ((K_s3 == 1) | (K_n3 <= 1)) & ((V_s3 == 1) | (V_n3 <= 1)) &  \
+                    ((O_s3 == 1) | (O_n3 <= 1));                                                               \
+  const int ok = same & d64 & rows __VA_ARGS__;                                                                \
+  const uint32_t gxy = kh::group_size_word(), bcx = kh::grid_blocks_x();                                       \
+  KH_ARGS_READY(ok, Q_base, Q_off, K_base, K_off, V_base, V_off, O_base, O_off, gxy, bcx);                     \
+  if (!ok) {                                                                                                   \
+    attention_refuse(Op, O_n0, O_n1, O_n2, O_n3, O_s0, O_s1, O_s2, O_s3, gxy, bcx);                            \
+    return;                                                                                                    \
+  }
+
 }  // namespace
 
 // Registers capped for two waves per SIMD (two workgroups per CU, as LDS
@@ -356,47 +640,7 @@ __device__ __forceinline__ void attention_slice(const float *__restrict__ Qg, co
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 attention(KH_MEMREF4(const float, Q), KH_MEMREF4(const float, K), KH_MEMREF4(const float, V),
           KH_MEMREF4(float, O)) {
-  const float *__restrict__ Qp = KH_PTR(Q);
-  const float *__restrict__ Kp = KH_PTR(K);
-  const float *__restrict__ Vp = KH_PTR(V);
-  float *__restrict__ Op = KH_PTR(O);
-  const int64_t heads = Q_n1, seq = Q_n2;
-  // The template's contract (attention.cpp:109-120 refuses other shapes):
-  // four [batch, heads, seq, 64] tensors with contiguous head_dim rows.
-  // Anything else is refused by filling O (as its descriptor describes it)
-  // with NaN, never by computing from memory the descriptors do not cover.
-  // Evaluated without short-circuit branches (& and |, not && and ||): the
-  // compiler then issues every descriptor load in one round at the start
-  // instead of one round per branch.
-  const bool same = (K_n0 == Q_n0) & (V_n0 == Q_n0) & (O_n0 == Q_n0) & (K_n1 == heads) & (V_n1 == heads) &
-                    (O_n1 == heads) & (K_n2 == seq) & (V_n2 == seq) & (O_n2 == seq);
-  const bool d64 = (Q_n3 == D) & (K_n3 == D) & (V_n3 == D) & (O_n3 == D);
-  const bool rows = ((Q_s3 == 1) | (Q_n3 <= 1)) & ((K_s3 == 1) | (K_n3 <= 1)) & ((V_s3 == 1) | (V_n3 <= 1)) &
-                    ((O_s3 == 1) | (O_n3 <= 1));
-  const int ok = same & d64 & rows;
-  // The check's loads, the base pointers and the launch geometry in one round.
-  const uint32_t gxy = kh::group_size_word(), bcx = kh::grid_blocks_x();
-  KH_ARGS_READY(ok, Q_base, Q_off, K_base, K_off, V_base, V_off, O_base, O_off, gxy, bcx);
-  if (!ok) {
-    const int64_t total = O_n0 * O_n1 * O_n2 * O_n3;
-    const int64_t tx = kh::threads_x_of(gxy), ty = kh::threads_y_of(gxy), tz = kh::threads_z_of(kh::group_size_z_word());
-    const int64_t gy = kh::grid_blocks_y(), gz = kh::grid_blocks_z();
-    const int64_t threads = tx * ty * tz;
-    const int64_t flat = ((int64_t)threadIdx.z * ty + threadIdx.y) * tx + threadIdx.x;
-    const int64_t block = ((int64_t)blockIdx.z * gy + blockIdx.y) * bcx + blockIdx.x;
-    const int64_t step = threads * bcx * gy * gz;
-    for (int64_t e = block * threads + flat; e < total; e += step) {
-      int64_t r = e;
-      const int64_t i3 = r % O_n3;
-      r /= O_n3;
-      const int64_t i2 = r % O_n2;
-      r /= O_n2;
-      const int64_t i1 = r % O_n1;
-      const int64_t i0 = r / O_n1;
-      Op[i0 * O_s0 + i1 * O_s1 + i2 * O_s2 + i3 * O_s3] = __builtin_nanf("");
-    }
-    return;
-  }
+  KH_ATTN_CHECK()
   // Which slice and query tiles this workgroup takes: slice (blockIdx.z,
   // blockIdx.y), query tiles blockIdx.x, + gridDim.x, ... (any grid). Under
   // the launcher's grid (one workgroup per 128-row query tile of each
@@ -440,4 +684,70 @@ attention(KH_MEMREF4(const float, Q), KH_MEMREF4(const float, K), KH_MEMREF4(con
   else
     attention_slice<false>(Qg, Kg, Vg, Og, Q_s2, K_s2, V_s2, O_s2, seq, (int)kh::threads_x_of(gxy), q0, qstep, Ks,
                            Vt);
+}
+
+// One workgroup of attention_split{,16}: query tile qt of a slice. Under the
+// launcher's grid (one workgroup per tile of each slice) each XCD takes a
+// contiguous range of the flat index, so that the tiles of a slice share an
+// L2 (see attention). Any strides of at least 64 floats, any alignment, spans
+// below 2^31 bytes, 64..256 threads; other launches are refused.
+template <int TQ>
+__device__ __forceinline__ void attention_split_slice(const float *__restrict__ Qp, const float *__restrict__ Kp,
+                                                      const float *__restrict__ Vp, float *__restrict__ Op,
+                                                      const int64_t (&sq)[3], const int64_t (&sk)[3],
+                                                      const int64_t (&sv)[3], const int64_t (&so)[3], int64_t batch,
+                                                      int64_t heads, int seq, int bd, uint32_t bcx, float *ml,
+                                                      float *Ob) {
+  const int nw = bd / kh::kWave, lane = kh::lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int tiles = (seq + 16 * TQ - 1) / (16 * TQ);
+  const uint32_t bcy = kh::grid_blocks_y(), bcz = kh::grid_blocks_z();
+  int64_t hb = blockIdx.y, bb = blockIdx.z;
+  int qt = blockIdx.x, qstep = bcx;
+  if ((int64_t)bcx == tiles && bcy == heads && bcz == batch && heads * batch * tiles < (1ll << 31)) {
+    const uint32_t L = (blockIdx.z * bcy + blockIdx.y) * bcx + blockIdx.x, total = bcx * bcy * bcz;
+    const uint32_t x = L & 7, per = total >> 3, extra = total & 7;
+    const uint32_t id = x * per + (x < extra ? x : extra) + (L >> 3), slice = id / tiles;
+    qt = id % tiles;
+    qstep = tiles;  // one tile per workgroup
+    hb = slice % heads;
+    bb = slice / heads;
+  }
+  if (hb >= heads || bb >= batch) return;
+  auto slice_rsrc = [&](const float *p, const int64_t (&st)[3]) __attribute__((always_inline)) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p + bb * st[0] + hb * st[1]);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return kh::span_rsrc(reinterpret_cast<const float *>(((uint64_t)hi << 32) | lo),
+                         (uint32_t)(((seq - 1) * st[2] + D) * 4));
+  };
+  const __amdgpu_buffer_rsrc_t rq = slice_rsrc(Qp, sq), rk = slice_rsrc(Kp, sk), rv = slice_rsrc(Vp, sv),
+                               ro = slice_rsrc(Op, so);
+  for (; qt < tiles; qt += qstep)
+    attention_split_tile<TQ>(rq, rk, rv, ro, (int)sq[2], (int)sk[2], (int)sv[2], (int)so[2], seq, qt * 16 * TQ, nw,
+                             wave, lane, ml, Ob);
+}
+
+#define KH_ATTN_SPLIT_BODY(TQ)                                                                                 \
+  constexpr int kWaves = KH_ATTN_SPLIT_THREADS / kh::kWave;                                                    \
+  __shared__ __attribute__((aligned(16))) float ml[kWaves * 16 * TQ * 2];                                      \
+  __shared__ __attribute__((aligned(16))) float Ob[kWaves * 16 * TQ * LDO];                                    \
+  KH_ATTN_CHECK(&(Q_s2 >= D) & (K_s2 >= D) & (V_s2 >= D) & (O_s2 >= D) & (seq > 0) &                           \
+                ((seq + 4 * SK) * (Q_s2 | K_s2 | V_s2 | O_s2) < (1ll << 29)) &                                 \
+                (kh::threads_x_of(kh::group_size_word()) % kh::kWave == 0))                                    \
+  const int64_t sq[3] = {Q_s0, Q_s1, Q_s2}, sk[3] = {K_s0, K_s1, K_s2}, sv[3] = {V_s0, V_s1, V_s2},            \
+                so[3] = {O_s0, O_s1, O_s2};                                                                    \
+  attention_split_slice<TQ>(Qp, Kp, Vp, Op, sq, sk, sv, so, Q_n0, heads, (int)seq,                             \
+                            (int)kh::threads_x_of(gxy), bcx, ml, Ob)
+
+extern "C" __global__ void __launch_bounds__(KH_ATTN_SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+attention_split(KH_MEMREF4(const float, Q), KH_MEMREF4(const float, K), KH_MEMREF4(const float, V),
+                KH_MEMREF4(float, O)) {
+  KH_ATTN_SPLIT_BODY(2);
+}
+
+extern "C" __global__ void __launch_bounds__(KH_ATTN_SPLIT_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+attention_split16(KH_MEMREF4(const float, Q), KH_MEMREF4(const float, K), KH_MEMREF4(const float, V),
+                  KH_MEMREF4(float, O)) {
+  KH_ATTN_SPLIT_BODY(1);
 }

@@ -413,6 +413,26 @@ RowPlan row_plan(bool softmax, int64_t cols) {
   return {block, cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
 }
 
+// How attention spreads (batch, heads, seq) over the chip (kh_tiles.h).
+struct AttentionPlan {
+  const char *symbol;
+  int64_t rows;  // query rows per workgroup
+};
+
+AttentionPlan attention_plan(int64_t batch, int64_t heads, int64_t seq) {
+  // Past this the split kernels' 32-bit offsets do not reach.
+  if (batch > 65535 || heads > 65535 || seq > (int64_t(1) << 22)) return {"attention", KH_ATTN_BLOCK_Q};
+  auto us = [&](int64_t rows, int64_t keys, int64_t waves, double step, double start) {
+    const int64_t rounds = ceil_div(batch * heads * ceil_div(seq, rows), KH_GEMM_CUS);
+    return static_cast<double>(rounds * ceil_div(ceil_div(seq, keys), waves)) * step + start;
+  };
+  const double whole = us(KH_ATTN_BLOCK_Q, 64, 1, KH_ATTN_STEP_US, KH_ATTN_START_US);
+  const double split = us(32, 32, 4, KH_ATTN_SPLIT_STEP_US, KH_ATTN_SPLIT_START_US);
+  const double split16 = us(16, 32, 4, KH_ATTN_SPLIT16_STEP_US, KH_ATTN_SPLIT16_START_US);
+  if (whole <= split && whole <= split16) return {"attention", KH_ATTN_BLOCK_Q};
+  return split <= split16 ? AttentionPlan{"attention_split", 32} : AttentionPlan{"attention_split16", 16};
+}
+
 // Launcher-owned geometry per template (see each kernel's header comment).
 int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block) {
   block = {256, 1, 1};
@@ -460,7 +480,7 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
       return khrt::fail(KHRT_E_INVALID, "attention: the kernel is pinned to head_dim = 64 (got head_dim = " +
                                             std::to_string(d) + ")");
     }
-    grid = {static_cast<unsigned>(ceil_div(seq, KH_ATTN_BLOCK_Q)), static_cast<unsigned>(h),
+    grid = {static_cast<unsigned>(ceil_div(seq, attention_plan(b, h, seq).rows)), static_cast<unsigned>(h),
             static_cast<unsigned>(b)};
   } else {
     return unknown_template(name);
@@ -476,6 +496,12 @@ const char *launch_symbol(const Template *t, const Shape &s) {
   if (n == "softmax" || n == "layernorm") {
     auto it = s.find("cols");
     if (it != s.end()) return row_plan(n == "softmax", it->second).symbol;
+  }
+  if (n == "attention") {
+    auto b = s.find("batch"), h = s.find("heads"), q = s.find("seq");
+    if (b != s.end() && h != s.end() && q != s.end()) {
+      return attention_plan(b->second, h->second, q->second).symbol;
+    }
   }
   if (n == "gemm") {
     auto m = s.find("m"), nn = s.find("n"), k = s.find("k");

@@ -208,3 +208,73 @@ def test_attention_reference_geometry_and_negative_control(dev):
     g, ref, bh, qi = _check(Q, K, V, got, b, h, s)
     wrong = O.ref_attention_rows(Q, K, V, s, D, bh, qi, scaled=False)
     assert O.attention_violation(g, wrong) > 2e-3
+
+
+@pytest.mark.parametrize("b,h,s,symbol", [
+    (1, 1, 1, "attention_split16"),     # one key: three waves without any
+    (1, 1, 31, "attention_split16"), (2, 3, 33, "attention_split16"), (1, 3, 97, "attention_split16"),
+    (1, 5, 129, "attention_split16"),   # two steps for the first waves, none for the last
+    (1, 8, 777, "attention_split"), (3, 7, 500, "attention_split16"), (2, 8, 1000, "attention_split"),
+    (4, 16, 256, "attention_split"),
+])
+def test_attention_split_launches(dev, b, h, s, symbol):
+    """Launches the 128-row tiles would leave idle: every row. N(0,1) inputs:
+    scores in log2 units below ~10 in magnitude carry 64 products' rounding
+    (~2^-21 of them) into exponents, so weights and outputs (|o| <= ~4) are
+    good to a few 1e-6."""
+    assert kh.launch_symbol("attention", f"batch={b},heads={h},seq={s},head_dim={D}") == symbol
+    n = b * h * s * D
+    Q, K, V = (O.normal(n, 31 + i, 0.0, 1.0) for i in range(3))
+    O.set_threads(8)
+    g, ref, _, _ = _check(Q, K, V, _attention(Q, K, V, b, h, s), b, h, s)
+    assert np.max(np.abs(g - ref)) <= 1e-5
+
+
+@pytest.mark.parametrize("symbol,rows", [("attention_split", 32), ("attention_split16", 16)])
+@pytest.mark.parametrize("s,threads,grid", [(70, 256, None), (200, 64, None), (200, 192, 2)])
+def test_attention_split_strides(dev, symbol, rows, s, threads, grid):
+    """Q, K, V and O each with an odd row pitch of its own and an odd start,
+    pads of NaN in the inputs and a sentinel in O; fewer waves and fewer
+    workgroups than the launcher's."""
+    b, h = 2, 3
+    pitch = {"Q": 65, "K": 67, "V": 71, "O": 69}
+    n = b * h * s * D
+    host = {"Q": O.normal(n, 41, 0.0, 1.0), "K": O.normal(n, 42, 0.0, 1.0), "V": O.normal(n, 43, 0.0, 1.0)}
+    bufs, args = {}, kh.LaunchArgs()
+    for i, name in enumerate("QKVO"):
+        p = np.full((b * h * s, pitch[name]), -7.0 if name == "O" else np.nan, np.float32)
+        if name != "O":
+            p[:, :D] = host[name].reshape(-1, D)
+        bufs[name] = up(np.concatenate([np.full(1, -7.0, np.float32), p.ravel()]))
+        args.add_memref(bufs[name].ptr + 4, [b, h, s, D])
+        w = pitch[name]
+        args.slots[11 * i + 7:11 * i + 11] = [h * s * w, s * w, w, 1]
+    f = kh.GpuModule(kh.code_object("attention")).get_function(symbol)
+    say(f"{symbol} pitches {pitch} s={s} threads={threads} grid={grid}")
+    kh.kernel_launch(f, (grid or (s + rows - 1) // rows, h, b), (threads, 1, 1), args)
+    out = down(bufs["O"], 1 + b * h * s * pitch["O"])[1:].reshape(-1, pitch["O"])
+    assert np.all(out[:, D:] == -7.0)
+    g, ref, _, _ = _check(host["Q"], host["K"], host["V"],
+                          np.ascontiguousarray(out[:, :D]).reshape(b * h, s, D), b, h, s)
+    assert np.max(np.abs(g - ref)) <= 1e-5
+
+
+@pytest.mark.parametrize("symbol", ["attention_split", "attention_split16"])
+@pytest.mark.parametrize("bad", ["head_dim32", "row_stride"])
+def test_attention_split_refuses(dev, symbol, bad):
+    # Another head_dim, or rows closer than their 64 floats: O becomes NaN and
+    # nothing past it is touched.
+    b, h, s, guard = 1, 2, 64, 256
+    d = 32 if bad == "head_dim32" else D
+    n = b * h * s * d
+    bufs = [empty(n + guard, 1.0) for _ in range(4)]
+    args = kh.LaunchArgs()
+    for x in bufs:
+        args.add_memref(x, [b, h, s, d])
+    if bad == "row_stride":
+        args.slots[11 + 9] = 0  # K: every key the same row
+    f = kh.GpuModule(kh.code_object("attention")).get_function(symbol)
+    say(f"{symbol} refusal {bad}")
+    kh.launch_raw(f, (2, h, b), (256, 1, 1), args)
+    out = down(bufs[3], n + guard)
+    assert np.all(np.isnan(out[:n])) and np.all(out[n:] == 1.0)
