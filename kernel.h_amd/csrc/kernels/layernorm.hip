@@ -204,11 +204,11 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
 }
 
 // One row per workgroup of nt threads, V float4 per thread (cols <= 4 V nt),
-// as many threads as hold the row at V = 4: every load of the row in flight,
-// one read and one write per element (gamma and beta come from L2). The wave
+// as many threads as hold the row: every load of the row in flight, one read
+// and one write per element (gamma and beta come from L2). The wave
 // per row that took such rows a float at a time, in three sweeps, was bound
 // by that one wave's load latency: 2048x5000 76.6 -> 17.1 us (4.8 TB/s),
-// 512x32001 508 -> 29, 1024x3001 35.0 -> 5.4, 16x65536 602 -> 14.4. More
+// 512x32001 508 -> 26, 1024x3001 35.0 -> 5.4, 16x65536 602 -> 14.4. More
 // threads than the row needs were slower (512x12000 8.3 us at 768, 11.2 at
 // 1024; 16384x4096 88.5 at 256, 103 at 512).
 template <int V>

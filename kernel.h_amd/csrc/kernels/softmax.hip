@@ -167,9 +167,10 @@ __device__ __forceinline__ void softmax_row_regs(const float *__restrict__ xr, f
 // The max and the sum each cross the waves through LDS; the maximum is the
 // whole row's before any exponential, so that every element's exponent
 // carries the same rounding of m * log2e and it cancels in the quotient. As
-// many threads as hold the row at V = 4 (fewer, larger threads measured level,
-// more were slower: 512x12000 7.8 us at 384-768 threads, 10.5 at 1024): one
-// read and one write per element with every load of the row in flight. The
+// many threads as hold the row (more were slower: 512x12000 7.8 us at 384-768
+// threads, 10.5 at 1024): one read and one write per element with every load
+// of the row in flight, and where the workgroup is small enough a second one
+// on the CU to fill its reductions. The
 // wave per row that took such rows a float at a time, twice, was bound by
 // that one wave's load latency: 256x32001 301.6 -> 14.1 us (4.6 TB/s),
 // 2048x6000 66.3 -> 18.9, 16x65536 285 -> 10.6.

@@ -398,18 +398,25 @@ struct RowPlan {
   int64_t rows_per_block;
 };
 
-RowPlan row_plan(bool softmax, int64_t cols) {
+RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   const char *narrow = softmax ? "softmax" : "layernorm", *wide = softmax ? "softmax_wide" : "layernorm_wide",
              *block = softmax ? "softmax_block" : "layernorm_block";
   if (cols <= KH_ROW16_COLS) return {narrow, 256, 16};
   if (cols <= 1024) return {narrow, 256, 4};
   if (cols <= 2048) return {wide, 256, 4};
   // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
-  // per thread.
+  // per thread: the fewest that need at most 768 threads, so that a CU's 2048
+  // hold two workgroups and one's loads fill the other's reductions and
+  // stores. Rotated launches, softmax / layernorm: 300x13000 9.5 / 10.5 us at
+  // 832 threads, 7.0 / 7.6 at 448; 1024x16000 26.7 / 28.5 at 1024, 23.6 / 25.6
+  // at 512; 512x32001 27.7 / 28.7 at 1024, 24.7 / 25.7 at 512. At 768 and
+  // below the two splits are within 4% (2000x10000, 4000x12000). With a CU for
+  // every row there is no second workgroup, and 16 float4 gain nothing over 8
+  // (256x32001: 14.2 us at 1024 threads, 14.4 at 512).
   auto threads = [&](int v) { return static_cast<unsigned>(64 * ceil_div(ceil_div(cols, 4), 64 * v)); };
   if (cols <= 4096) return {wide, threads(4), 1};
-  if (cols <= 4096 * 4) return {narrow, threads(4), 1};
-  if (cols <= 4096 * 8) return {narrow, threads(8), 1};
+  if (threads(4) <= 768) return {narrow, threads(4), 1};
+  if (threads(8) <= 768 || (threads(8) <= 1024 && rows <= KH_GEMM_CUS)) return {narrow, threads(8), 1};
   return {block, cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
 }
 
@@ -452,7 +459,7 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
     if (!need(s, "rows", rows) || !need(s, "cols", cols)) {
       return khrt::fail(KHRT_E_INVALID, t + ": shape attributes 'rows' and 'cols' are required and must be positive");
     }
-    const RowPlan p = row_plan(t == "softmax", cols);
+    const RowPlan p = row_plan(t == "softmax", rows, cols);
     block.x = p.threads;
     grid.x = clamp_grid(ceil_div(rows, p.rows_per_block));
   } else if (t == "scan" || t == "scan_totals") {
@@ -494,8 +501,8 @@ int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block
 const char *launch_symbol(const Template *t, const Shape &s) {
   const std::string n = t->name;
   if (n == "softmax" || n == "layernorm") {
-    auto it = s.find("cols");
-    if (it != s.end()) return row_plan(n == "softmax", it->second).symbol;
+    auto r = s.find("rows"), c = s.find("cols");
+    if (r != s.end() && c != s.end()) return row_plan(n == "softmax", r->second, c->second).symbol;
   }
   if (n == "attention") {
     auto b = s.find("batch"), h = s.find("heads"), q = s.find("seq");
