@@ -14,10 +14,13 @@
 #include "kh_tiles.h"
 
 #include <algorithm>
+#include <array>
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <fstream>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <string>
@@ -72,15 +75,24 @@ const KernelResources kResources[] = {
 #include "kh_resources.inc"
 };
 
+enum Kind { kVecadd, kGemm, kSoftmax, kLayernorm, kScan, kScanTotals, kFusedGelu, kAttention };
+
 struct Template {
   const char *name;  // template name == kernel symbol
   const char *co;    // code object holding the symbol
+  Kind kind;         // its index here
 };
 
 // Registry order follows the reference's registration (registry.cpp:23-36).
 const Template kTemplates[] = {
-    {"vecadd", "vecadd"}, {"gemm", "gemm"},         {"softmax", "softmax"},       {"layernorm", "layernorm"},
-    {"scan", "scan"},     {"scan_totals", "scan"}, {"fused_gelu", "fused_gelu"}, {"attention", "attention"},
+    {"vecadd", "vecadd", kVecadd},
+    {"gemm", "gemm", kGemm},
+    {"softmax", "softmax", kSoftmax},
+    {"layernorm", "layernorm", kLayernorm},
+    {"scan", "scan", kScan},
+    {"scan_totals", "scan", kScanTotals},
+    {"fused_gelu", "fused_gelu", kFusedGelu},
+    {"attention", "attention", kAttention},
 };
 
 const CodeObject *find_co(const char *name) {
@@ -440,89 +452,105 @@ AttentionPlan attention_plan(int64_t batch, int64_t heads, int64_t seq) {
   return split <= split16 ? AttentionPlan{"attention_split", 32} : AttentionPlan{"attention_split16", 16};
 }
 
-// Launcher-owned geometry per template (see each kernel's header comment).
-int geometry(const char *name, const Shape &s, khrt_dim3 &grid, khrt_dim3 &block) {
-  block = {256, 1, 1};
-  grid = {1, 1, 1};
-  int64_t n = 0, rows = 0, cols = 0, m = 0, k = 0, b = 0, h = 0, seq = 0, d = 0;
-  const std::string t = name;
-  if (t == "vecadd" || t == "fused_gelu") {
-    if (!need(s, "n", n)) {
-      if (t == "fused_gelu" && need(s, "rows", rows) && need(s, "cols", cols)) {
-        n = rows * cols;
+// Extents of a template's shape, in the order its entry point takes them:
+// n; rows, cols; m, n, k; batch, heads, seq, head_dim.
+using Dims = std::array<int64_t, 4>;
+
+// Dims of a parsed shape, or the error that names what is missing.
+int dims_of(const Template &tpl, const Shape &s, Dims &d) {
+  const std::string t = tpl.name;
+  if (tpl.kind == kVecadd || tpl.kind == kFusedGelu) {
+    if (!need(s, "n", d[0])) {
+      if (tpl.kind == kFusedGelu && need(s, "rows", d[0]) && need(s, "cols", d[1])) {
+        d[0] *= d[1];
       } else {
         return khrt::fail(KHRT_E_INVALID, t + ": shape attribute 'n' is required and must be positive");
       }
     }
-    grid.x = clamp_grid(ceil_div(ceil_div(n, 4), 256LL * KH_EW_UNROLL));
-  } else if (t == "softmax" || t == "layernorm") {
-    if (!need(s, "rows", rows) || !need(s, "cols", cols)) {
+  } else if (tpl.kind == kSoftmax || tpl.kind == kLayernorm) {
+    if (!need(s, "rows", d[0]) || !need(s, "cols", d[1])) {
       return khrt::fail(KHRT_E_INVALID, t + ": shape attributes 'rows' and 'cols' are required and must be positive");
     }
-    const RowPlan p = row_plan(t == "softmax", rows, cols);
-    block.x = p.threads;
-    grid.x = clamp_grid(ceil_div(rows, p.rows_per_block));
-  } else if (t == "scan" || t == "scan_totals") {
-    if (!need(s, "n", n)) return khrt::fail(KHRT_E_INVALID, t + ": shape attribute 'n' is required and must be positive");
-    if (t == "scan") {
-      block.x = n <= KH_SCAN_SMALL_N ? KH_SCAN_SMALL_THREADS : KH_SCAN_THREADS;
-      grid.x = clamp_grid(ceil_div(n, int64_t(KH_SCAN_PER_THREAD) * (block.x - 64)));
-    } else {
-      grid.x = clamp_grid(std::min<int64_t>(ceil_div(ceil_div(n, 256) + 1, 256), 1024));
-    }
-  } else if (t == "gemm") {
-    if (!need(s, "m", m) || !need(s, "n", n) || !need(s, "k", k)) {
+  } else if (tpl.kind == kScan || tpl.kind == kScanTotals) {
+    if (!need(s, "n", d[0])) return khrt::fail(KHRT_E_INVALID, t + ": shape attribute 'n' is required and must be positive");
+  } else if (tpl.kind == kGemm) {
+    if (!need(s, "m", d[0]) || !need(s, "n", d[1]) || !need(s, "k", d[2])) {
       return khrt::fail(KHRT_E_INVALID, "gemm: shape attributes 'm', 'n' and 'k' are required and must be positive");
     }
-    const GemmCandidate &c = gemm_choice(m, n, k);
-    grid.x = clamp_grid(candidate_grid(c, m, n));
-    block.x = static_cast<unsigned>(64 * c.waves());
-  } else if (t == "attention") {
-    if (!need(s, "batch", b) || !need(s, "heads", h) || !need(s, "seq", seq) || !need(s, "head_dim", d)) {
+  } else {
+    if (!need(s, "batch", d[0]) || !need(s, "heads", d[1]) || !need(s, "seq", d[2]) || !need(s, "head_dim", d[3])) {
       return khrt::fail(KHRT_E_INVALID,
                         "attention: shape attributes 'batch', 'heads', 'seq' and 'head_dim' are required and "
                         "must be positive");
     }
-    if (d != 64) {
-      return khrt::fail(KHRT_E_INVALID, "attention: the kernel is pinned to head_dim = 64 (got head_dim = " +
-                                            std::to_string(d) + ")");
-    }
-    grid = {static_cast<unsigned>(ceil_div(seq, attention_plan(b, h, seq).rows)), static_cast<unsigned>(h),
-            static_cast<unsigned>(b)};
-  } else {
-    return unknown_template(name);
   }
   return 0;
 }
 
-// Symbol the launcher runs for a template at a shape. Every symbol of a
-// template takes the same arguments and computes the same result; the
-// variants differ in which register paths they compile in (row_plan).
-const char *launch_symbol(const Template *t, const Shape &s) {
-  const std::string n = t->name;
-  if (n == "softmax" || n == "layernorm") {
-    auto r = s.find("rows"), c = s.find("cols");
-    if (r != s.end() && c != s.end()) return row_plan(n == "softmax", r->second, c->second).symbol;
-  }
-  if (n == "attention") {
-    auto b = s.find("batch"), h = s.find("heads"), q = s.find("seq");
-    if (b != s.end() && h != s.end() && q != s.end()) {
-      return attention_plan(b->second, h->second, q->second).symbol;
+// What the launcher runs for a template at a shape: the symbol (every symbol
+// of a template takes the same arguments and computes the same result), its
+// code object and the launch geometry (see each kernel's header comment).
+struct Plan {
+  const char *symbol;
+  const char *co;
+  khrt_dim3 grid, block;
+};
+
+int make_plan(const Template &tpl, const Dims &d, Plan &p) {
+  p = Plan{tpl.name, tpl.co, {1, 1, 1}, {256, 1, 1}};
+  switch (tpl.kind) {
+    case kVecadd:
+    case kFusedGelu:
+      p.grid.x = clamp_grid(ceil_div(ceil_div(d[0], 4), 256LL * KH_EW_UNROLL));
+      return 0;
+    case kSoftmax:
+    case kLayernorm: {
+      const RowPlan r = row_plan(tpl.kind == kSoftmax, d[0], d[1]);
+      p.symbol = r.symbol;
+      p.block.x = r.threads;
+      p.grid.x = clamp_grid(ceil_div(d[0], r.rows_per_block));
+      return 0;
+    }
+    case kScan:
+      p.block.x = d[0] <= KH_SCAN_SMALL_N ? KH_SCAN_SMALL_THREADS : KH_SCAN_THREADS;
+      p.grid.x = clamp_grid(ceil_div(d[0], int64_t(KH_SCAN_PER_THREAD) * (p.block.x - 64)));
+      return 0;
+    case kScanTotals:
+      p.grid.x = clamp_grid(std::min<int64_t>(ceil_div(ceil_div(d[0], 256) + 1, 256), 1024));
+      return 0;
+    case kGemm: {
+      const GemmCandidate &c = gemm_choice(d[0], d[1], d[2]);
+      p.symbol = c.symbol;
+      p.co = c.co;
+      p.grid.x = clamp_grid(candidate_grid(c, d[0], d[1]));
+      p.block.x = static_cast<unsigned>(64 * c.waves());
+      return 0;
+    }
+    case kAttention: {
+      if (d[3] != 64) {
+        return khrt::fail(KHRT_E_INVALID, "attention: the kernel is pinned to head_dim = 64 (got head_dim = " +
+                                              std::to_string(d[3]) + ")");
+      }
+      const AttentionPlan a = attention_plan(d[0], d[1], d[2]);
+      p.symbol = a.symbol;
+      p.grid = {static_cast<unsigned>(ceil_div(d[2], a.rows)), static_cast<unsigned>(d[1]),
+                static_cast<unsigned>(d[0])};
+      return 0;
     }
   }
-  if (n == "gemm") {
-    auto m = s.find("m"), nn = s.find("n"), k = s.find("k");
-    if (m != s.end() && nn != s.end() && k != s.end()) return gemm_choice(m->second, nn->second, k->second).symbol;
-  }
-  return t->name;
+  return unknown_template(tpl.name);
 }
 
-// Code object holding the symbol the launcher runs for a template.
-const char *launch_co(const Template *t, const char *symbol) {
-  if (std::strcmp(t->name, "gemm") == 0) {
-    if (const GemmCandidate *c = find_gemm_candidate(symbol)) return c->co;
-  }
-  return t->co;
+// The plan of a shape given as text.
+int plan_of(const char *name, const char *shape, Plan &p) {
+  const Template *t = find_template(name);
+  if (t == nullptr) return unknown_template(name);
+  Shape s;
+  std::string why;
+  if (!kernelh::parse_shape_text(shape, s, &why)) return khrt::fail(KHRT_E_INVALID, "malformed shape: expected " + why);
+  Dims d{};
+  if (int rc = dims_of(*t, s, d)) return rc;
+  return make_plan(*t, d, p);
 }
 
 // Workgroups of `block` threads of `fn` resident on the whole device at
@@ -556,28 +584,108 @@ int64_t resident_workgroups(void *fn, unsigned block) {
   return resident;
 }
 
-// Packs, verifies and launches template `name`.
-int launch_template(const char *name, khrt::LaunchArgs &args, const Shape &shape, void *stream) {
-  const Template *t = find_template(name);
-  if (t == nullptr) return unknown_template(name);
-  khrt_dim3 grid, block;
-  if (int rc = geometry(name, shape, grid, block)) return rc;
-  void *fn = nullptr;
-  const char *symbol = launch_symbol(t, shape);
-  if (int rc = get_function(launch_co(t, symbol), symbol, &fn)) return rc;
-  if (std::strcmp(name, "scan") == 0) {
+// Functions launched before: what a launch of `symbol` with `threads` threads
+// on `device` needs besides its arguments. The verifier's other rules (shared
+// memory, threads, wave multiple, occupancy) depend on nothing else, and the
+// embedded modules stay loaded for the process's life, so once a launch has
+// passed it only the grid is left to check. Entries are only ever appended,
+// whole, under the mutex; readers see them through the count. A full table
+// only means that further functions verify every launch.
+struct Ready {
+  const char *symbol;
+  int device;
+  unsigned threads;
+  void *fn;
+  int64_t resident;  // workgroups on the device at once (scan; 0: not asked)
+  int64_t max_grid[3];
+};
+constexpr int kMaxReady = 512;
+Ready g_ready[kMaxReady];
+std::atomic<int> g_nready{0};
+std::mutex g_ready_mu;
+
+const Ready *find_ready(const char *symbol, int device, unsigned threads) {
+  const int n = g_nready.load(std::memory_order_acquire);
+  for (int i = 0; i < n; ++i) {
+    const Ready &r = g_ready[i];
+    if (r.symbol == symbol && r.threads == threads && r.device == device) return &r;
+  }
+  return nullptr;
+}
+
+void add_ready(const Ready &r) {
+  std::lock_guard<std::mutex> lock(g_ready_mu);
+  const int n = g_nready.load(std::memory_order_relaxed);
+  if (n == kMaxReady || find_ready(r.symbol, r.device, r.threads) != nullptr) return;
+  g_ready[n] = r;
+  g_nready.store(n + 1, std::memory_order_release);
+}
+
+// Kernel parameters of a template call on the stack: the memref descriptors
+// of LaunchArgs, contiguous row-major with offset 0.
+class StackArgs {
+ public:
+  void add_memref(const void *ptr, std::initializer_list<int64_t> shape) {
+    const uint64_t p = static_cast<uint64_t>(reinterpret_cast<uintptr_t>(ptr));
+    const size_t rank = shape.size();
+    uint64_t *s = slots_ + count_;
+    s[0] = s[1] = p;
+    s[2] = 0;
+    uint64_t stride = 1;
+    for (size_t i = rank; i-- > 0;) {
+      s[3 + i] = static_cast<uint64_t>(shape.begin()[i]);
+      s[3 + rank + i] = stride;
+      stride *= static_cast<uint64_t>(shape.begin()[i]);
+    }
+    count_ += 3 + 2 * rank;
+  }
+  void **params() {
+    for (size_t i = 0; i < count_; ++i) params_[i] = &slots_[i];
+    return params_;
+  }
+  size_t count() const { return count_; }
+
+ private:
+  static constexpr size_t kMax = 44;  // attention: four of rank 4
+  uint64_t slots_[kMax];
+  void *params_[kMax];
+  size_t count_ = 0;
+};
+
+// Verifies and launches template `kind` at extents `d`.
+int launch_template(Kind kind, StackArgs &args, const Dims &d, void *stream) {
+  Plan p;
+  if (int rc = make_plan(kTemplates[kind], d, p)) return rc;
+  if (int rc = khrt::ensure_device()) return rc;
+  const int dev = khrt::current_device();
+  const Ready *known = find_ready(p.symbol, dev, p.block.x);
+  Ready r;
+  if (known != nullptr) {
+    r = *known;
+  } else {
+    r = Ready{p.symbol, dev, p.block.x, nullptr, 0, {0, 0, 0}};
+    if (int rc = get_function(p.co, p.symbol, &r.fn)) return rc;
+    if (kind == kScan) r.resident = resident_workgroups(r.fn, p.block.x);
+    khrt_device_limits live;
+    if (int rc = khrt_live_limits(&live)) return rc;
+    for (int i = 0; i < 3; ++i) r.max_grid[i] = live.max_grid_dim[i];
+  }
+  if (kind == kScan && r.resident > 0) {
     // The look-back scan is persistent: one resident wave of workgroups
     // loops over tiles, so launch no more workgroups than fit at once, and
     // as many as give every workgroup the same number of tiles (grid.x is
     // the tile count here): 4370 tiles at n = 2^26 run as 18 full rounds of
     // 243 workgroups, not 17 rounds of 256 and an 18th of 18 tiles, during
     // which HBM idles.
-    if (const int64_t resident = resident_workgroups(fn, block.x); resident > 0) {
-      const int64_t tiles = grid.x, rounds = ceil_div(tiles, resident);
-      grid.x = static_cast<unsigned>(ceil_div(tiles, rounds));
-    }
+    const int64_t tiles = p.grid.x, rounds = ceil_div(tiles, r.resident);
+    p.grid.x = static_cast<unsigned>(ceil_div(tiles, rounds));
   }
-  return khrt::verified_launch(fn, grid, block, 0, stream, args.params(), args.count());
+  if (known != nullptr && p.grid.x <= r.max_grid[0] && p.grid.y <= r.max_grid[1] && p.grid.z <= r.max_grid[2]) {
+    return khrt_launch_raw(r.fn, p.grid, p.block, 0, stream, args.params());
+  }
+  if (int rc = khrt::verified_launch(r.fn, p.grid, p.block, 0, stream, args.params(), args.count())) return rc;
+  if (known == nullptr) add_ready(r);
+  return 0;
 }
 
 int bad(const char *what) { return khrt::fail(KHRT_E_INVALID, what); }
@@ -618,25 +726,20 @@ int khrt_template_resources(const char *name, khrt_kernel_resources *out) {
 
 int khrt_template_geometry(const char *name, const char *shape, khrt_dim3 *grid, khrt_dim3 *block) {
   if (grid == nullptr || block == nullptr || shape == nullptr) return bad("khrt_template_geometry: null argument");
-  if (find_template(name) == nullptr) return unknown_template(name);
-  Shape s;
-  std::string why;
-  if (!kernelh::parse_shape_text(shape, s, &why)) return khrt::fail(KHRT_E_INVALID, "malformed shape: expected " + why);
-  return geometry(name, s, *grid, *block);
+  Plan p;
+  if (int rc = plan_of(name, shape, p)) return rc;
+  *grid = p.grid;
+  *block = p.block;
+  return 0;
 }
 
 int khrt_template_launch_symbol(const char *name, const char *shape, char *out, size_t cap) {
   if (shape == nullptr || out == nullptr || cap == 0) return bad("khrt_template_launch_symbol: null argument");
-  const Template *t = find_template(name);
-  if (t == nullptr) return unknown_template(name);
-  Shape s;
-  std::string why;
-  if (!kernelh::parse_shape_text(shape, s, &why)) return khrt::fail(KHRT_E_INVALID, "malformed shape: expected " + why);
-  khrt_dim3 grid, block;
-  if (int rc = geometry(name, s, grid, block)) return rc;  // the same shape checks as a launch
-  const std::string sym = launch_symbol(t, s);
-  if (sym.size() + 1 > cap) return bad("khrt_template_launch_symbol: output buffer too small");
-  std::memcpy(out, sym.c_str(), sym.size() + 1);
+  Plan p;
+  if (int rc = plan_of(name, shape, p)) return rc;  // the same shape checks as a launch
+  const size_t len = std::strlen(p.symbol);
+  if (len + 1 > cap) return bad("khrt_template_launch_symbol: output buffer too small");
+  std::memcpy(out, p.symbol, len + 1);
   return 0;
 }
 
@@ -742,42 +845,42 @@ int khrt_fill_f32(void *dst, float value, size_t count, void *stream) {
 int kh_vecadd(const float *a, const float *b, float *c, int64_t n, void *stream) {
   if (n <= 0) return bad("vecadd: n must be positive");
   if (!a || !b || !c) return bad("vecadd: null buffer");
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(a, {n});
   args.add_memref(b, {n});
   args.add_memref(c, {n});
-  return launch_template("vecadd", args, {{"n", n}}, stream);
+  return launch_template(kVecadd, args, {n}, stream);
 }
 
 int kh_fused_gelu(const float *x, float *tmp, float *out, int64_t n, void *stream) {
   if (n <= 0) return bad("fused_gelu: n must be positive");
   if (!x || !out) return bad("fused_gelu: null buffer");
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(x, {n});
   args.add_memref(tmp, {n});
   args.add_memref(out, {n});
-  return launch_template("fused_gelu", args, {{"n", n}}, stream);
+  return launch_template(kFusedGelu, args, {n}, stream);
 }
 
 int kh_softmax(const float *x, float *y, int64_t rows, int64_t cols, void *stream) {
   if (rows <= 0 || cols <= 0) return bad("softmax: rows and cols must be positive");
   if (!x || !y) return bad("softmax: null buffer");
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(x, {rows, cols});
   args.add_memref(y, {rows, cols});
-  return launch_template("softmax", args, {{"rows", rows}, {"cols", cols}}, stream);
+  return launch_template(kSoftmax, args, {rows, cols}, stream);
 }
 
 int kh_layernorm(const float *x, const float *gamma, const float *beta, float *y, int64_t rows, int64_t cols,
                  void *stream) {
   if (rows <= 0 || cols <= 0) return bad("layernorm: rows and cols must be positive");
   if (!x || !gamma || !beta || !y) return bad("layernorm: null buffer");
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(x, {rows, cols});
   args.add_memref(gamma, {cols});
   args.add_memref(beta, {cols});
   args.add_memref(y, {rows, cols});
-  return launch_template("layernorm", args, {{"rows", rows}, {"cols", cols}}, stream);
+  return launch_template(kLayernorm, args, {rows, cols}, stream);
 }
 
 int kh_scan(const float *x, float *y, float *y_lo, float *totals_hi, float *totals_lo, int64_t n, void *stream) {
@@ -789,13 +892,13 @@ int kh_scan(const float *x, float *y, float *y_lo, float *totals_hi, float *tota
   // floats of each;
   // the kernel establishes it on first use and keeps it valid across calls.
   const int64_t T = ceil_div(n, 256);
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(x, {n});
   args.add_memref(y, {n});
   args.add_memref(y_lo, {n});
   args.add_memref(totals_hi, {T});
   args.add_memref(totals_lo, {T});
-  return launch_template("scan", args, {{"n", n}}, stream);
+  return launch_template(kScan, args, {n}, stream);
 }
 
 int kh_scan_totals(const float *totals_hi, const float *totals_lo, float *off_hi, float *off_lo, float *off_lo2,
@@ -803,7 +906,7 @@ int kh_scan_totals(const float *totals_hi, const float *totals_lo, float *off_hi
   if (n <= 0) return bad("scan_totals: n must be positive");
   if (!totals_hi || !totals_lo || !off_hi || !off_lo || !off_lo2 || !y) return bad("scan_totals: null buffer");
   const int64_t T = ceil_div(n, 256);
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(totals_hi, {T});
   args.add_memref(totals_lo, {T});
   args.add_memref(off_hi, {T});
@@ -811,17 +914,17 @@ int kh_scan_totals(const float *totals_hi, const float *totals_lo, float *off_hi
   args.add_memref(off_lo2, {T});
   args.add_memref(y, {n});
   args.add_memref(y_lo, {n});
-  return launch_template("scan_totals", args, {{"n", n}}, stream);
+  return launch_template(kScanTotals, args, {n}, stream);
 }
 
 int kh_gemm(const float *A, const float *B, float *C, int64_t m, int64_t n, int64_t k, void *stream) {
   if (m <= 0 || n <= 0 || k <= 0) return bad("gemm: m, n and k must be positive");
   if (!A || !B || !C) return bad("gemm: null buffer");
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(A, {m, k});
   args.add_memref(B, {k, n});
   args.add_memref(C, {m, n});
-  return launch_template("gemm", args, {{"m", m}, {"n", n}, {"k", k}}, stream);
+  return launch_template(kGemm, args, {m, n, k}, stream);
 }
 
 int kh_attention(const float *Q, const float *K, const float *V, float *O, int64_t batch, int64_t heads, int64_t seq,
@@ -829,13 +932,12 @@ int kh_attention(const float *Q, const float *K, const float *V, float *O, int64
   if (batch <= 0 || heads <= 0 || seq <= 0 || head_dim <= 0) return bad("attention: all extents must be positive");
   if (!Q || !K || !V || !O) return bad("attention: null buffer");
   if (heads > 65535 || batch > 65535) return bad("attention: heads and batch must be <= 65535 (grid y/z)");
-  khrt::LaunchArgs args;
+  StackArgs args;
   args.add_memref(Q, {batch, heads, seq, head_dim});
   args.add_memref(K, {batch, heads, seq, head_dim});
   args.add_memref(V, {batch, heads, seq, head_dim});
   args.add_memref(O, {batch, heads, seq, head_dim});
-  return launch_template("attention", args,
-                         {{"batch", batch}, {"heads", heads}, {"seq", seq}, {"head_dim", head_dim}}, stream);
+  return launch_template(kAttention, args, {batch, heads, seq, head_dim}, stream);
 }
 
 // Streaming roofline kernels: 32 workgroups of 256 per CU, grid-strided.

@@ -570,3 +570,28 @@ def test_bench_row_work(kernel, shape, value, flops):
 def test_bench_row_work_needs_the_kernels_dims():
     with pytest.raises(kh.KhrtError, match="no bench row for kernel 'softmax'"):
         kh.bench_row_work("softmax", "n=1024")
+
+
+# ------------------------------------------------------------------ template calls from Python
+
+@pytest.mark.parametrize("bad", [b"\0" * 64, "text", np.zeros(4, np.float32), (ctypes.c_float * 4)(), 1.5j])
+def test_template_calls_take_only_device_pointers(bad):
+    # Host objects that ctypes would pass as a pointer are refused before the
+    # library is entered, in every position.
+    for call in (lambda: kh.vecadd(bad, 16, 16, 4), lambda: kh.gemm(16, bad, 16, 1, 1, 1),
+                 lambda: kh.softmax(16, 16, 1, 1, bad), lambda: kh.scan(16, 16, bad, 16, 16, 4),
+                 lambda: kh.attention(16, 16, 16, bad, 1, 1, 1, 64)):
+        with pytest.raises((TypeError, ValueError, ctypes.ArgumentError)):
+            call()
+
+
+@pytest.mark.parametrize("null", [0, None, np.int64(0)])
+def test_template_calls_null_buffers(null):
+    # Integers of any kind and None reach the entry point, which names the
+    # missing buffer; extents are checked first.
+    for call, what in ((lambda: kh.vecadd(null, null, null, 4), "vecadd: null buffer"),
+                       (lambda: kh.layernorm(null, null, null, null, 1, 1, null), "layernorm: null buffer"),
+                       (lambda: kh.fused_gelu(null, null, null, 0), "fused_gelu: n must be positive"),
+                       (lambda: kh.attention(null, null, null, null, 1, 1, 1, 64), "attention: null buffer")):
+        with pytest.raises(kh.KhrtError, match=what):
+            call()
