@@ -209,22 +209,23 @@ __device__ __forceinline__ uint32_t lds_addr(const float *p) { return (uint32_t)
 // is row-major within a group. Callers fetch slabs with k0 < K (or k0 = 0
 // when K = 0, which reads nothing). `wave` must be wave-uniform.
 //
-// SELECT: float4s past K (A) or N (B) are sent to an offset outside the
-// resource and read 0; for K and N multiples of 4. Without it nothing is
-// selected: a float4 at or past K or N carries what follows in memory (the
-// next row, or 0 past the matrix). Columns of B past N only feed columns of C
-// that are not stored, rows of B past K read 0 through the range check, and
-// the caller zeroes A's k past K in the fragments (mask_k). Each offset is
-// then a loop-invariant 32-bit term plus a wave-uniform one (k0 for A, n0 for
-// B), which keeps the offsets of every load of a slab in registers even where
-// the tile's accumulators leave few: 8192^3 142.8 -> 146.8 TFLOP/s.
+// SEL: float4s past K (kSelA, for K a multiple of 4) and past N (kSelAB, and
+// N too) are sent to an offset outside the resource and read 0. What is not
+// selected carries what follows in memory (the next row, or 0 past the
+// matrix). Columns of B past N only feed columns of C that are not stored,
+// rows of B past K read 0 through the range check, and A's k past K are the
+// caller's to zero in the fragments (mask_k). An offset without a select is a
+// loop-invariant 32-bit term plus a wave-uniform one (k0 for A, n0 for B),
+// which keeps the offsets of every load of a slab in registers even where the
+// tile's accumulators leave few: 8192^3 142.8 -> 146.8 TFLOP/s.
 //
 // WHOLE: every slab the caller fetches has BK rows of B, so the resource's
 // size is the same for all of them (else it is computed per slab).
 //
 // dma_part issues loads L0..L1-1 of a slab (A's NA, then B's NB), so that a
 // slab's loads can be spread between MFMAs; dma_slab issues all of them.
-template <class T, bool SELECT, int L0, int L1, bool WHOLE = false>
+constexpr int kSelNone = 0, kSelA = 1, kSelAB = 2;
+template <class T, int SEL, int L0, int L1, bool WHOLE = false>
 __device__ __forceinline__ void dma_part(const float *__restrict__ A, const float *__restrict__ B, int64_t M,
                                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t m0, int64_t n0,
                                          int64_t k0, float *As, float *Bs, int wave, int lane) {
@@ -237,10 +238,8 @@ __device__ __forceinline__ void dma_part(const float *__restrict__ A, const floa
     const int idx = idx0 + lane;
     const int ar = idx / T::QP, ak = 4 * ((idx % T::QP) ^ T::aswz(ar));
     uint32_t aoff;
-    if constexpr (SELECT)
-      aoff = (k0 + ak < K) ? (uint32_t)((ar * lda + k0 + ak) * 4) : kOutside;
-    else
-      aoff = ((uint32_t)ar * (uint32_t)lda + (uint32_t)ak) * 4u + (uint32_t)k0 * 4u;
+    aoff = ((uint32_t)ar * (uint32_t)lda + (uint32_t)ak) * 4u + (uint32_t)k0 * 4u;
+    if constexpr (SEL != kSelNone) aoff = ((uint32_t)ak < (uint32_t)(K - k0)) ? aoff : kOutside;
     dma16(ra, aoff, lds_addr(As + 4 * idx0));
   }
 #pragma unroll
@@ -250,7 +249,7 @@ __device__ __forceinline__ void dma_part(const float *__restrict__ A, const floa
     const int idx = idx0 + lane;
     const int bk = idx / T::BROW, bn = 4 * (idx % T::BROW);
     uint32_t boff;
-    if constexpr (SELECT)
+    if constexpr (SEL == kSelAB)
       boff = (n0 + bn < N) ? (uint32_t)((bk * ldb + n0 + bn) * 4) : kOutside;
     else
       boff = ((uint32_t)bk * (uint32_t)ldb + (uint32_t)bn) * 4u + (uint32_t)n0 * 4u;
@@ -258,11 +257,11 @@ __device__ __forceinline__ void dma_part(const float *__restrict__ A, const floa
   }
 }
 
-template <class T, bool SELECT, bool WHOLE = false>
+template <class T, int SEL, bool WHOLE = false>
 __device__ __forceinline__ void dma_slab(const float *__restrict__ A, const float *__restrict__ B, int64_t M,
                                          int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t m0, int64_t n0,
                                          int64_t k0, float *As, float *Bs, int wave, int lane) {
-  dma_part<T, SELECT, 0, T::NA + T::NB, WHOLE>(A, B, M, N, K, lda, ldb, m0, n0, k0, As, Bs, wave, lane);
+  dma_part<T, SEL, 0, T::NA + T::NB, WHOLE>(A, B, M, N, K, lda, ldb, m0, n0, k0, As, Bs, wave, lane);
 }
 
 // Wait until at most N vector-memory operations of this wave are in flight
@@ -434,9 +433,9 @@ __device__ __forceinline__ void k_loop_dma(AccOf<T> (&acc)[WTM][WTN], const floa
   constexpr int BK = T::BK;
   constexpr int C = BK / Mfma<T::kMF>::CK;
   const int wv = __builtin_amdgcn_readfirstlane(wave);
-  dma_slab<T, true>(Ap, Bp, M, N, K, lda, ldb, m0, n0, 0, As, Bs, wv, lane);
+  dma_slab<T, kSelAB>(Ap, Bp, M, N, K, lda, ldb, m0, n0, 0, As, Bs, wv, lane);
   if (nslabs > 1) {
-    dma_slab<T, true>(Ap, Bp, M, N, K, lda, ldb, m0, n0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
+    dma_slab<T, kSelAB>(Ap, Bp, M, N, K, lda, ldb, m0, n0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
     vm_barrier<T::NA + T::NB>();
   } else {
     vm_barrier<0>();
@@ -454,7 +453,7 @@ __device__ __forceinline__ void k_loop_dma(AccOf<T> (&acc)[WTM][WTN], const floa
     if (PRIO) __builtin_amdgcn_s_setprio(0);
     vm_barrier<0>();
     if (ks + 2 < nslabs)
-      dma_slab<T, true>(Ap, Bp, M, N, K, lda, ldb, m0, n0, (ks + 2) * BK, As + fut * T::A_STAGE, Bs + fut * T::B_STAGE,
+      dma_slab<T, kSelAB>(Ap, Bp, M, N, K, lda, ldb, m0, n0, (ks + 2) * BK, As + fut * T::A_STAGE, Bs + fut * T::B_STAGE,
                   wv, lane);
     if (ks + 1 < nslabs) read_frag<WTM, WTN, T>(f0, As + nxt * T::A_STAGE, Bs + nxt * T::B_STAGE, 0, wm, wn, lane);
     if (PRIO) __builtin_amdgcn_s_setprio(1);
@@ -736,7 +735,7 @@ __device__ __forceinline__ void interleave_reads() {
 // reads, since s_setprio bounds what the scheduler may interleave.
 // MASK: the slab is a tile's last and reaches past K, so its A fragments there
 // are zeroed (left: the k of the slab that exist).
-template <int WTM, int WTN, class T, bool PRIO, bool WHOLE, int WAIT = 0, bool MASK = false>
+template <int WTM, int WTN, class T, bool PRIO, int SEL, bool WHOLE, int WAIT = 0, bool MASK = false>
 __device__ __forceinline__ void flat_step(AccOf<T> (&acc)[WTM][WTN], Frag<WTM, WTN> &f0, Frag<WTM, WTN> &f1, int &cur,
                                           const float *__restrict__ Ap, const float *__restrict__ Bp, int64_t M,
                                           int64_t N, int64_t K, int64_t lda, int64_t ldb, bool dma, int64_t dm0,
@@ -769,12 +768,12 @@ __device__ __forceinline__ void flat_step(AccOf<T> (&acc)[WTM][WTN], Frag<WTM, W
     if (read_next) read_frag<WTM, WTN, T>(f0, As + nxt * T::A_STAGE, Bs + nxt * T::B_STAGE, 0, wm, wn, lane);
     mfma_frag_s<WTM, WTN, 0, 1>(acc, f1);
     interleave_reads<kReads>();
-    if (dma) dma_part<T, false, 0, kL / 2, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
+    if (dma) dma_part<T, SEL, 0, kL / 2, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
     mfma_frag_s<WTM, WTN, 1, 2>(acc, f1);
-    if (dma) dma_part<T, false, kL / 2, kL, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
+    if (dma) dma_part<T, SEL, kL / 2, kL, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
     mfma_frag_s<WTM, WTN, 2, 4>(acc, f1);
   } else {
-    if (dma) dma_slab<T, false, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
+    if (dma) dma_slab<T, SEL, WHOLE>(Ap, Bp, M, N, K, lda, ldb, dm0, dn0, dk0, dA, dB, wv, lane);
     if (read_next) read_frag<WTM, WTN, T>(f0, As + nxt * T::A_STAGE, Bs + nxt * T::B_STAGE, 0, wm, wn, lane);
   }
 #pragma unroll
@@ -791,14 +790,18 @@ __device__ __forceinline__ void flat_step(AccOf<T> (&acc)[WTM][WTN], Frag<WTM, W
 // j % 3; slab ks of a tile fetches slab ks+2 of the same tile or, in the
 // tile's last two slabs, slab 0 or 1 of the next. The tile's C stores go
 // out after those fetches. Needs at least two slabs per tile (K > BK) and
-// fewer than 2^31 tiles. KTAIL: K is no multiple of BK. WHOLE (not with
-// KTAIL): dma_part's.
-template <int WTM, int WTN, int BKT, bool PRIO, int WGM, int WGN, int MF, bool KTAIL, bool WHOLE>
+// fewer than 2^31 tiles. KTAIL: what zeroes A's k past K, when K is no multiple
+// of BK: selects in every load (K a multiple of 4), or masks in the last two
+// slabs of a tile (mask_k), which cost more per tile and less per slab.
+// WHOLE (without a tail): dma_part's.
+constexpr int kTailNone = 0, kTailQuads = 1, kTailMask = 2;
+template <int WTM, int WTN, int BKT, bool PRIO, int WGM, int WGN, int MF, int KTAIL, bool WHOLE>
 __device__ __forceinline__ void gemm_tiles_flat(const float *__restrict__ Ap, const float *__restrict__ Bp,
                                                 float *__restrict__ Cp, int64_t M, int64_t N, int64_t K,
                                                 int64_t lda, int64_t ldb, int64_t ldc, float *As, float *Bs) {
   using T = Tile<WTM, WTN, BKT, true, WGM, WGN, MF>;
   constexpr int BK = T::BK;
+  constexpr int SEL = KTAIL == kTailQuads ? kSelA : kSelNone;
   constexpr int kStores = WTM * WTN * (MF == 32 ? 16 : 4);  // store_tile_buf's stores per lane
   constexpr int kStoreSlack = kStores < 62 ? kStores : 62;
   const int tid = threadIdx.x;
@@ -833,8 +836,8 @@ __device__ __forceinline__ void gemm_tiles_flat(const float *__restrict__ Ap, co
 
   int64_t cm0, cn0;
   coords(0, cm0, cn0);
-  dma_slab<T, false, WHOLE>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, 0, As, Bs, wv, lane);
-  dma_slab<T, false, WHOLE>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
+  dma_slab<T, SEL, WHOLE>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, 0, As, Bs, wv, lane);
+  dma_slab<T, SEL, WHOLE>(Ap, Bp, M, N, K, lda, ldb, cm0, cn0, BK, As + T::A_STAGE, Bs + T::B_STAGE, wv, lane);
   vm_barrier<T::NA + T::NB>();
   Frag<WTM, WTN> f0, f1;
   read_frag<WTM, WTN, T>(f0, As, Bs, 0, wm, wn, lane);
@@ -863,21 +866,21 @@ __device__ __forceinline__ void gemm_tiles_flat(const float *__restrict__ Ap, co
       // min(kStores, 62) are outstanding completes the loads and lets the
       // newest stores drain behind this tile's MFMAs.
       if (t > 0)
-        flat_step<WTM, WTN, T, PRIO, WHOLE, kStoreSlack>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0,
+        flat_step<WTM, WTN, T, PRIO, SEL, WHOLE, kStoreSlack>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0,
                                                        dk0, true, As, Bs, wv, wm, wn, lane);
       else
-        flat_step<WTM, WTN, T, PRIO, WHOLE>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0, dk0, true, As, Bs,
+        flat_step<WTM, WTN, T, PRIO, SEL, WHOLE>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, dma, dm0, dn0, dk0, true, As, Bs,
                                      wv, wm, wn, lane);
     }
     for (int64_t ks = 1; ks < ns - 2; ++ks)
-      flat_step<WTM, WTN, T, PRIO, WHOLE>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, true, cm0, cn0, (ks + 2) * BK,
+      flat_step<WTM, WTN, T, PRIO, SEL, WHOLE>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, true, cm0, cn0, (ks + 2) * BK,
                                       true, As, Bs, wv, wm, wn, lane);
     // The last two slabs (the last one only, when ns = 2) fetch the next
     // tile's slabs 0 and 1.
     // With a partial last slab both mask A's k (all of the first of the two
     // exist): one copy of the step's code, which is fetched cold.
     for (int64_t ks = ns > 2 ? ns - 2 : 1; ks < ns; ++ks)
-      flat_step<WTM, WTN, T, PRIO, WHOLE, 0, KTAIL>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, has_next, nm0, nn0,
+      flat_step<WTM, WTN, T, PRIO, SEL, WHOLE, 0, KTAIL == kTailMask>(acc, f0, f1, cur, Ap, Bp, M, N, K, lda, ldb, has_next, nm0, nn0,
                                                      (ks + 2 - ns) * BK, ks + 1 < ns || has_next, As, Bs, wv, wm, wn,
                                                      lane, (int)(K - ks * BK));
     store_tile_buf<WTM, WTN, T>(acc, Cp, M, N, ldc, cm0, cn0, wm, wn, lane);
@@ -951,11 +954,17 @@ __device__ __forceinline__ void gemm_entry_flat(const float *__restrict__ Ap, co
     // B's resource computed per slab (1024x1024x8192 151.0 vs 154.9 us), at
     // two per CU without (3072^3 465 vs 455).
     if (K % T::BK == 0 && T::BN < 128 && tiles <= KH_GEMM_CUS)
-      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, false, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, kTailNone, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
     else if (K % T::BK == 0)
-      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, false, true>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, kTailNone, true>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+    // Selects against masks, 64-wide tiles two per CU: 2500x2500 with K = 112
+    // 23.7 vs 24.6 us, 300 45.1 vs 45.7, 404 56.2 vs 56.3, 500 67.3 vs 67.0; one
+    // tile per CU or the 128-wide ones: 2048x2048x400 32.5 vs 32.0,
+    // 2000x2000x2004 129.1 vs 125.8, 4096x4096x100 37.2 vs 37.4.
+    else if (K % 4 == 0 && K <= 12 * T::BK)
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, kTailQuads, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
     else
-      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, true, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
+      gemm_tiles_flat<WTM, WTN, BKT, PRIO, WGM, WGN, MF, kTailMask, false>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
   } else {
     gemm_body<WTM, WTN, BKT, PRIO, kPipeDma, WGM, WGN, MF>(Ap, Bp, Cp, M, N, K, lda, ldb, ldc, As, Bs);
   }

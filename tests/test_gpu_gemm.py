@@ -349,6 +349,10 @@ def test_tune_cache_steers_the_launcher(dev, tmp_path):
     (130, 257, 35, 5),    # 3 k past
     (129, 127, 61, 2),    # a float4 of A with one k left
     (300, 514, 97, 7),    # several slabs, tiles looped
+    (129, 127, 36, 2),    # k a multiple of 4: one float4 past a slab,
+    (300, 514, 100, 7),   # tiles looped,
+    (65, 63, 380, 3),     # the longest such k that is selected in the loads
+    (65, 63, 388, 3),     # and the shortest that is masked
     (64, 256, 64, 1),     # whole slabs over odd strides
     (1, 1, 1001, 1),
 ])
