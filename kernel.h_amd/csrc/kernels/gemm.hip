@@ -12,11 +12,10 @@
 //     MFMA accumulator blocks. Five such symbols, all correct for every
 //     shape; the launcher scores each by its full-occupancy rate times how
 //     busy its last round of workgroups would be (kh_tiles.h) and takes the
-//     best, unless the launch has at most 256 tiles of 32x32, or fewer
-//     than 256 tiles of 64x64 that are all whole with K a multiple of 128
-//     (then `gemm_ksplit` / `gemm_ksplit_deep`, at the end of this file,
-//     split K over 8 waves instead); a tune cache, when set, overrides the
-//     choice:
+//     best, unless the launch has at most 256 tiles of 32x64, or fewer
+//     than 256 tiles of 64x64 with whole 32x32 tiles and K a multiple of 128
+//     (then a `gemm_ksplit*`, at the end of this file, splits K over 8
+//     waves instead); a tune cache, when set, overrides the choice:
 //       `gemm`        128x256 tiles (64x128 per wave, 128 accumulator registers
 //                     per lane), 16-deep K slabs: the least LDS and L2 traffic
 //                     per MFMA (8192^3, 4096^3, 8192x8192x256); persistent
@@ -58,7 +57,8 @@
 //     direct-to-LDS symbols' slab loads are unconditional at any alignment and
 //     extent: a dwordx4 buffer load needs 4-byte alignment only and is
 //     range-checked dword by dword, and what it carries past K is zeroed in
-//     the fragments of a tile's last slab. The register-staged ones' are
+//     the fragments of a tile's last slabs (or, for short K that is a multiple
+//     of 4, selected away in the loads). The register-staged ones' are
 //     branch-free buffer loads for aligned operands with k, n multiples of 4,
 //     whose range checks zero-fill the tails (the guarded per-element form of
 //     the generic path made the compiler split every load into branches and
