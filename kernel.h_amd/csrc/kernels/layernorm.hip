@@ -208,7 +208,7 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
 // and one write per element (gamma and beta come from L2). The wave
 // per row that took such rows a float at a time, in three sweeps, was bound
 // by that one wave's load latency: 2048x5000 76.6 -> 17.1 us (4.8 TB/s),
-// 512x32001 508 -> 26, 1024x3001 35.0 -> 5.4, 16x65536 602 -> 14.4. More
+// 512x32001 508 -> 26, 1024x3001 35.0 -> 5.4, 16x65536 602 -> 13.4. More
 // threads than the row needs were slower (512x12000 8.3 us at 768, 11.2 at
 // 1024; 16384x4096 88.5 at 256, 103 at 512).
 template <int V>
@@ -331,7 +331,7 @@ __device__ __forceinline__ void layernorm_all(const float *__restrict__ X, const
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
   const int64_t r0 = (int64_t)blockIdx.x * waves_per_block + wave;
   const int64_t rstep = waves_per_block * nb;
-  const int c = (int)(cols < KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
+  const int c = (int)(cols <= KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
   static_assert(kStageCols == 4 * 4 * kh::kWave, "the narrow symbol stages every column its widest wave path holds");
   if (S == kNarrow && c <= KH_ROW16_COLS && xs >= cols && ys >= cols && (xs | ys) < (1 << 26)) {
     if (c <= 64)

@@ -173,7 +173,7 @@ __device__ __forceinline__ void softmax_row_regs(const float *__restrict__ xr, f
 // on the CU to fill its reductions. The
 // wave per row that took such rows a float at a time, twice, was bound by
 // that one wave's load latency: 256x32001 301.6 -> 14.1 us (4.6 TB/s),
-// 2048x6000 66.3 -> 18.9, 16x65536 285 -> 10.6.
+// 2048x6000 66.3 -> 18.9, 16x65536 285 -> 9.5.
 template <int V>
 __device__ __forceinline__ void softmax_row_block(const float *__restrict__ xr, float *__restrict__ yr, int cols,
                                                   int nt, int lane, int wave, float (&red)[2][kh::kMaxWaves]) {
@@ -283,7 +283,7 @@ __device__ __forceinline__ void softmax_rows(const float *__restrict__ X, float 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);  // uniform: scalar row loop
   const int64_t nwaves = waves_per_block * nb;
   const int64_t w0 = (int64_t)blockIdx.x * waves_per_block + wave;
-  const int c = (int)(cols < KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
+  const int c = (int)(cols <= KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
   if (S == kNarrow && c <= KH_ROW16_COLS && xs >= cols && ys >= cols && (xs | ys) < (1 << 26)) {
     for (int64_t r = 4 * w0; r < rows; r += 4 * nwaves) {
       if (c <= 64)

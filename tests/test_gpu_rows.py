@@ -194,8 +194,8 @@ def test_rows_blocks_of_partial_waves(dev, template, cols):
 # Edges of softmax's row paths: 16 lanes (one, two, four float4 each), a wave,
 # a workgroup of 4, 8 and 16 float4 per thread, two sweeps; one column either
 # side of each and widths that leave 1-3 floats in the last float4.
-SOFTMAX_EDGES = [1, 3, 63, 64, 65, 127, 129, 254, 256, 257, 511, 513, 1023, 1025, 2047, 2049, 4095, 4097, 16383,
-                 16385, 32767, 32769, 65535, 65537]
+SOFTMAX_EDGES = [1, 3, 63, 64, 65, 127, 129, 254, 256, 257, 511, 513, 1023, 1025, 2047, 2048, 2049, 4095, 4096, 4097,
+                 12288, 12289, 16383, 16385, 24576, 24577, 32767, 32768, 32769, 65535, 65536, 65537]
 
 
 @pytest.mark.parametrize("cols", SOFTMAX_EDGES)
@@ -296,3 +296,24 @@ def test_layernorm_padded_rows_any_symbol(dev, symbol, cols, block):
     out = down(dy, rows * ys).reshape(rows, ys)
     assert np.all(out[:, cols:] == -7.0)
     assert np.max(np.abs(out[:, :cols] - O.ref_layernorm(x, g, b, rows, cols))) <= 1e-5
+
+
+@pytest.mark.parametrize("template", ["softmax", "layernorm"])
+@pytest.mark.parametrize("cols", [5000, 12289, 24577, 32768, 65535, 65536])
+def test_row_is_read_whole_before_it_is_written(dev, template, cols):
+    # Up to 65536 columns a workgroup holds the row in registers, so an output
+    # that overlaps the input further on is the one beside it; a second sweep
+    # over the row would read what the first chunk's outputs replaced.
+    shift = 16384 if cols > 16384 else 1024
+    x = O.normal(cols, 0x0E1A, 0.0, 4.0)
+    g, b = O.uniform(cols, 0x1A7F, 0.5, 1.5), O.uniform(cols, 0x1A80, -0.1, 0.1)
+    buf = up(np.concatenate([x, np.zeros(shift, np.float32)]))
+    say(f"{template} rows=1 cols={cols}, y {shift} floats into x")
+    if template == "softmax":
+        ref = _softmax(x, 1, cols)
+        kh.softmax(buf.ptr, buf.ptr + 4 * shift, 1, cols)
+    else:
+        ref = _layernorm(x, g, b, 1, cols)
+        dg, db = up(g), up(b)
+        kh.layernorm(buf.ptr, dg, db, buf.ptr + 4 * shift, 1, cols)
+    assert np.array_equal(down(buf, shift + cols)[shift:], ref.ravel())
