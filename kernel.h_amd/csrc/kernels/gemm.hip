@@ -447,8 +447,109 @@ __device__ __forceinline__ void ks_any(const float *__restrict__ A, const float 
   }
 }
 
-// Any strides and spans, an element at a time: launches ks_any_ok turns down.
-// Summed in runs of 1024 k, so that a long K costs no precision.
+// The same with 64-bit addresses, at any strides and spans: launches ks_any_ok
+// turns down (K from 2^23, a wave's share of B past 2^31 bytes, rows that
+// overlap). Its callers take tiles one block wide, whose addresses fit beside
+// the registers of the other forms (two blocks and more took 140-210). Rows past
+// M and columns past N load the last one's, which is in range, and are not
+// stored; k past the wave's range only occur in its last partial batch, where
+// the loads are clamped and both operands zeroed. So the loop has no conditional
+// load, and what bounds it is, as there, two batches in flight per wave:
+// 1x1x(2^23 + 64) 21 ms, 4x64x(2^23 + 1) 35, 20x1000x1000000 4.1. An element per
+// thread, one load after another, took 519 ms for the first.
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int TM, int TN>
+__device__ __forceinline__ void ks_wide(const float *__restrict__ A, const float *__restrict__ B,
+                                        float *__restrict__ C, int64_t M, int64_t N, int64_t K, int64_t lda,
+                                        int64_t ldb, int64_t ldc, int nw, int64_t nblocks, float *red) {
+  using Set = KsSet<TM, TN, 1>;
+  constexpr int R = 4 * TM * TN;  // accumulator registers
+  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int r = lane & 15, g = lane >> 4;
+  const int64_t tiles_n = (N + 16 * TN - 1) / (16 * TN), total = ((M + 16 * TM - 1) / (16 * TM)) * tiles_n;
+  const int64_t kc = 16 * ((K + 16 * nw - 1) / (16 * nw)), kb = wave * kc, ke = kb + kc < K ? kb + kc : K;
+  for (int64_t t = blockIdx.x; t < total; t += nblocks) {
+    const int64_t m0 = (t / tiles_n) * 16 * TM, n0 = (t % tiles_n) * 16 * TN;
+    v4f acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = v4f{};
+    if (wave < nw && kb < ke) {
+      const float *pa[TM], *pb[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) pa[i] = A + (m0 + 16 * i + r < M ? m0 + 16 * i + r : M - 1) * lda + 4 * g;
+#pragma unroll
+      for (int j = 0; j < TN; ++j) pb[j] = B + (n0 + 16 * j + r < N ? n0 + 16 * j + r : N - 1) + 4 * g * ldb;
+      auto load = [&](Set &f, int64_t k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const f4_any a = *reinterpret_cast<const f4_any *>(pa[i] + k0);
+          f.a[0][i] = make_float4(a.x, a.y, a.z, a.w);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) f.b[0][j][s] = pb[j][(k0 + s) * ldb];
+      };
+      auto math = [&](const Set &f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < TM; ++i) {
+            const float4 a = f.a[0][i];
+            const float av = s == 0 ? a.x : s == 1 ? a.y : s == 2 ? a.z : a.w;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, f.b[0][j][s], acc[i][j], 0, 0, 0);
+          }
+      };
+      const int64_t whole = kb + (ke - kb) / 16 * 16;  // whole batches
+      Set s0, s1;
+      if (kb < whole) load(s0, kb);
+      for (int64_t k = kb; k < whole; k += 32) {
+        if (k + 16 < whole) load(s1, k + 16);
+        math(s0);
+        if (k + 32 < whole) load(s0, k + 32);
+        if (k + 16 < whole) math(s1);
+      }
+      if (whole < ke) {
+        const int64_t left = ke - whole - 4 * g;  // of this lane's four k
+        float *const fa = reinterpret_cast<float *>(s0.a[0]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const int64_t k = s < left ? whole + s : ke - 1 - 4 * g;
+#pragma unroll
+          for (int i = 0; i < TM; ++i) fa[4 * i + s] = s < left ? pa[i][k] : 0.0f;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) s0.b[0][j][s] = s < left ? pb[j][k * ldb] : 0.0f;
+        }
+        math(s0);
+      }
+    }
+    // Partial tiles into LDS, summed in the order of the waves, as in ks_any.
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[(wave * R + (i * TN + j) * 4 + q) * kh::kWave + lane] = acc[i][j][q];
+    kh::lds_barrier();
+    if (wave < nw) {
+      for (int x = wave; x < R; x += nw) {
+        float s = red[x * kh::kWave + lane];
+        for (int w = 1; w < nw; ++w) s += red[(R * w + x) * kh::kWave + lane];
+        const int64_t gr = m0 + 16 * (x / (4 * TN)) + 4 * g + (x & 3), gc = n0 + 16 * ((x >> 2) % TN) + r;
+        if (gr < M && gc < N) C[gr * ldc + gc] = s;
+      }
+    }
+    kh::lds_barrier();
+  }
+}
+
+// Blocks without a whole wave: an element per thread. Summed in runs of 1024
+// k, so that a long K costs no precision.
 __device__ __forceinline__ void ks_plain(const float *__restrict__ A, const float *__restrict__ B,
                                          float *__restrict__ C, int64_t M, int64_t N, int64_t K, int64_t lda,
                                          int64_t ldb, int64_t ldc, int64_t threads, int64_t nblocks) {
@@ -478,6 +579,8 @@ __device__ __forceinline__ void ks_plain(const float *__restrict__ A, const floa
   if (ks_any_ok(nw, A_n0, B_n1, A_n1, A_s0, B_s0, C_s0))                                                      \
     ks_any<TM, TN, NB>(KH_PTR(A), KH_PTR(B), KH_PTR(C), (int)A_n0, (int)B_n1, (int)A_n1, A_s0, B_s0, C_s0,    \
                        nw, (int)nb, red);                                                                     \
+  else if (nw > 0)                                                                                            \
+    ks_wide<TM, 1>(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, nw, nb, red);         \
   else                                                                                                        \
     ks_plain(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, kh::threads_x_of(gw), nb)
 

@@ -440,3 +440,46 @@ def test_gemm_ksplit_broadcast_rows(dev):
     kh.kernel_launch(f, (4, 1, 1), (512, 1, 1), args)
     want = np.repeat(A.astype(np.float64), m, 0) @ np.repeat(B[:1].astype(np.float64), k, 0)
     assert np.array_equal(down(dC, m * n).reshape(m, n), want.astype(np.float32))
+
+
+def test_gemm_long_k_costs_what_its_length_does(dev):
+    # One output of 2^23 products and more: past the K-split kernels' 32-bit
+    # offsets, where the time must still follow the length.
+    import time
+    k0 = 1 << 23
+    times = {}
+    for k in (k0 - 64, k0 + 64):
+        dA, dB, dC = kh.Buffer(4 * k), kh.Buffer(4 * k), empty(1)
+        dA.fill(0.5)
+        dB.fill(0.25)
+        say(f"gemm m=1 n=1 k={k}")
+        for i in range(2):  # the second call is timed
+            kh.synchronize()
+            t = time.perf_counter()
+            kh.gemm(dA, dB, dC, 1, 1, k)
+            kh.synchronize()
+            times[k] = time.perf_counter() - t
+        assert down(dC, 1)[0] == k * 0.125  # multiples of 1/8 below 2^24 of them: exact in any order
+    print(times)
+    assert times[k0 + 64] <= 8 * times[k0 - 64]
+
+
+@pytest.mark.parametrize("sym", ["gemm_ksplit", "gemm_ksplit_deep", "gemm_ksplit_16x16", "gemm_ksplit_32x16",
+                                 "gemm_ksplit_32x64"])
+@pytest.mark.parametrize("m,n,k,block", [
+    (1, 1, 1, 512), (17, 33, 16, 512), (33, 65, 129, 512), (40, 70, 515, 192), (5, 3, 47, 64), (16, 16, 0, 512),
+    (20, 30, 61, 32),  # less than a wave
+])
+def test_gemm_ksplit_overlapping_rows(dev, sym, m, n, k, block):
+    """Rows of A and B one float apart, whatever their length: the form with
+    64-bit addresses, at the edges of its tiles and batches. Whole numbers."""
+    host = np.resize(np.array([1, -2, 3, 0, 2, -1, 4, -3, 2, 1, -4], np.float32), 1 + max(m, k) + max(k, n))
+    dA, dB, dC = up(host), up(host[::-1]), empty(m * n)
+    args = kh.LaunchArgs().add_memref(dA.ptr + 4, [m, k]).add_memref(dB, [k, n]).add_memref(dC, [m, n])
+    args.slots[5] = args.slots[7 + 5] = 1
+    f = kh.GpuModule(kh.code_object("gemm")).get_function(sym)
+    say(f"{sym} overlapping rows m={m} n={n} k={k} block={block}")
+    kh.launch_raw(f, (3, 1, 1), (block, 1, 1), args)
+    A = np.array([host[1 + i:1 + i + k] for i in range(m)], np.float64).reshape(m, k)
+    B = np.array([host[::-1][i:i + n] for i in range(k)], np.float64).reshape(k, n)
+    assert np.array_equal(down(dC, m * n).reshape(m, n), (A @ B).astype(np.float32))
