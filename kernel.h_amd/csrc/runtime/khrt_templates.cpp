@@ -219,23 +219,16 @@ const GemmCandidate kGemmCandidates[] = {
     {"gemm_wide", "gemm", 16, 4, 2, 2, 4, 32, 1, kPersistent, true, 1},
     {"gemm_ksplit", "gemm", 32, 1, 1, 1, 1, 8, 0, kKsplit, true},
     {"gemm_ksplit_deep", "gemm", 32, 1, 1, 1, 1, 8, 0, kKsplitDeep, true},
-    KH_GEMM_TUNE_CONFIGS(KH_TUNE_CANDIDATE)};
-#undef KH_TUNE_CANDIDATE
-constexpr int kGemmCandidateCount = static_cast<int>(sizeof(kGemmCandidates) / sizeof(kGemmCandidates[0]));
-static_assert(kGemmCandidateCount == 7 + KH_GEMM_TUNE_COUNT, "candidate table");
-
-// K-split tiles that only the launcher picks, smallest first.
-const GemmCandidate kKsplitTiles[] = {
     {"gemm_ksplit_16x16", "gemm", 16, 1, 1, 1, 1, 16, 0, kKsplit, true, 2, 16, 16},
     {"gemm_ksplit_32x16", "gemm", 16, 1, 1, 2, 1, 16, 0, kKsplit, true, 2, 32, 16},
     {"gemm_ksplit_32x64", "gemm", 16, 1, 1, 2, 4, 16, 0, kKsplit, true, 2, 32, 64},
-};
+    KH_GEMM_TUNE_CONFIGS(KH_TUNE_CANDIDATE)};
+#undef KH_TUNE_CANDIDATE
+constexpr int kGemmCandidateCount = static_cast<int>(sizeof(kGemmCandidates) / sizeof(kGemmCandidates[0]));
+static_assert(kGemmCandidateCount == 10 + KH_GEMM_TUNE_COUNT, "candidate table");
 
 const GemmCandidate *find_gemm_candidate(const char *symbol) {
   if (symbol == nullptr) return nullptr;
-  for (const auto &c : kKsplitTiles) {
-    if (std::strcmp(c.symbol, symbol) == 0) return &c;
-  }
   for (const auto &c : kGemmCandidates) {
     if (std::strcmp(c.symbol, symbol) == 0) return &c;
   }

@@ -404,7 +404,7 @@ def test_elf_image_size_refuses_what_is_not_a_code_object():
 # ------------------------------------------------------------------ GEMM candidates / tune space
 
 _PRODUCT_GEMM = ["gemm", "gemm_mid", "gemm_small", "gemm_small_pf2", "gemm_wide", "gemm_ksplit",
-                 "gemm_ksplit_deep"]
+                 "gemm_ksplit_deep", "gemm_ksplit_16x16", "gemm_ksplit_32x16", "gemm_ksplit_32x64"]
 
 
 def _notes(co):
@@ -450,6 +450,19 @@ def test_gemm_candidate_table():
             assert c["bm"] == c["wave_grid_m"] * c["wave_tile_m"] and c["bn"] == c["wave_grid_n"] * c["wave_tile_n"]
             assert c["wave_tile_m"] % c["mfma"] == 0 and c["wave_tile_n"] % c["mfma"] == 0
             assert c["waves"] == c["wave_grid_m"] * c["wave_grid_n"]
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (16, 4096, 4096), (17, 4096, 4096), (100, 777, 555), (333, 1000, 2000), (1, 1, 1), (8192, 16, 500),
+    (512, 512, 512), (512, 512, 8192), (760, 768, 768), (1024, 1024, 1024), (2048, 2048, 2048), (8192, 8192, 8192),
+])
+def test_tuning_covers_what_the_launcher_picks(m, n, k):
+    # `kernelh tune` evaluates this list and its best overrides the launcher,
+    # so a symbol missing from it would be tuned away.
+    sym = kh.launch_symbol("gemm", f"m={m},n={n},k={k}")
+    own = {c["symbol"]: c for c in kh.gemm_candidates() if c["product"]}
+    assert sym in own
+    assert kh.gemm_candidate_geometry(sym, m, n, k) == kh.geometry("gemm", f"m={m},n={n},k={k}")
 
 
 @pytest.mark.parametrize("symbol,m,n,k,grid,block", [

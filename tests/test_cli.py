@@ -186,16 +186,16 @@ def test_tune_usage_and_refusals(tmp_path):
 
 @pytest.mark.gpu
 def test_tune_evaluates_candidates_and_caches(dev, tmp_path):
-    print("[gpu-case] kernelh tune gemm m=n=k=512, 10 candidates", flush=True)
+    print("[gpu-case] kernelh tune gemm m=n=k=512, 12 candidates", flush=True)
     cache = str(tmp_path / "cache.json")
     shape = "m=512,n=512,k=512"
-    args = ("tune", "--shape", shape, "--out", str(tmp_path), "--max-candidates", "10",
+    args = ("tune", "--shape", shape, "--out", str(tmp_path), "--max-candidates", "12",
             "--timeout", "60", "--cache", cache)
     r = run(*args)
     assert r.returncode == 0, r.stdout
     assert "best config: gemm" in r.stdout and "tune ok" in r.stdout
     rows = list(csv.DictReader(open(tmp_path / "tune-results.csv")))
-    assert len(rows) == 10
+    assert len(rows) == 12
     assert list(rows[0].keys())[:11] == ["kernel", "shape", "bm", "bn", "bk", "waves", "unroll", "vec", "ms_median",
                                           "accepted", "reason"]
     assert all(row["accepted"] == "true" and row["reason"] == "ok" for row in rows), rows
@@ -207,7 +207,7 @@ def test_tune_evaluates_candidates_and_caches(dev, tmp_path):
     assert (by["gemm"]["bm"], by["gemm"]["bn"], by["gemm"]["waves"], by["gemm"]["unroll"]) == ("128", "256", "4", "2")
     assert (by["gemm_mid"]["unroll"], by["gemm_ksplit"]["waves"], by["gemm_ksplit_deep"]["unroll"]) == ("1", "8", "3")
     assert {row["vec"] for row in rows} == {"4"}  # k, n multiples of 4: dwordx4 loads
-    assert all(row["product"] == ("1" if i < 7 else "0") for i, row in enumerate(rows))
+    assert all(row["product"] == ("1" if i < 10 else "0") for i, row in enumerate(rows))
     best = min(rows, key=lambda row: float(row["ms_median"]))["symbol"]
     assert f"best config: {best} " in r.stdout
     r2 = run(*args)
