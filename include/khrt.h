@@ -257,8 +257,8 @@ typedef struct khrt_gemm_candidate {
   int32_t waves;          /* wave64s per workgroup */
   int32_t wave_grid_m, wave_grid_n;  /* waves along m and n (K-split: 1 x 1) */
   int32_t wave_tile_m, wave_tile_n;  /* C elements per wave */
-  int32_t bm, bn, bk;     /* C tile per workgroup; K slab depth (K-split: k group) */
-  int32_t unroll;         /* slabs (K-split: 32-k batches) in flight ahead of the MFMAs */
+  int32_t bm, bn, bk;     /* C tile per workgroup; K slab depth (K-split: k per MFMA group) */
+  int32_t unroll;         /* slabs (K-split: sets of loads) in flight ahead of the MFMAs */
   int32_t prio;           /* waves raise their priority while issuing MFMAs */
   int32_t persistent;     /* grid = min(tiles, two per CU); workgroups loop over tiles */
   int32_t k_split;        /* the workgroup's waves split K, summed in a fixed order */

@@ -205,8 +205,8 @@ struct GemmCandidate {
   int waves() const { return ksplit() ? KH_GEMM_KSPLIT_THREADS / 64 : wgm * wgn; }
   int bm() const { return ksplit() ? ks_bm : mfma * wtm * wgm; }
   int bn() const { return ksplit() ? ks_bn : mfma * wtn * wgn; }
-  // Slabs (K-split: batches of 32 k) in flight ahead of the MFMAs.
-  int unroll() const { return pipe == kRegs ? 1 : pipe == kKsplitDeep ? 3 : 2; }
+  // Slabs (K-split: register sets of loads) in flight ahead of the MFMAs.
+  int unroll() const { return pipe == kRegs ? 1 : 2; }
 };
 
 #define KH_TUNE_CANDIDATE(PART, MF, WGM, WGN, WTM, WTN, BK, PRIO, PIPE, SYM) \

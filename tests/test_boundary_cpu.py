@@ -427,6 +427,8 @@ def test_gemm_candidate_table():
     assert [c["symbol"] for c in cands[:np_]] == _PRODUCT_GEMM
     assert all(c["product"] == 1 for c in cands[:np_]) and not any(c["product"] for c in cands[np_:])
     assert len({c["symbol"] for c in cands}) == len(cands)
+    # The K-split forms hold two register sets of loads, whatever their size.
+    assert {c["unroll"] for c in cands if c["k_split"]} == {2}
     space = cands[np_:]
     # The reference's axes (autotuner.hpp:36-41) all vary over the space,
     # re-pruned for MFMA tiles: both MFMA shapes, 4 and 8 waves, BM/BN in

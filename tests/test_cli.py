@@ -202,10 +202,10 @@ def test_tune_evaluates_candidates_and_caches(dev, tmp_path):
     assert all(float(row["ms_median"]) > 0 for row in rows)
     # The launcher's own symbols come first, with their real axes: the
     # persistent 128x256 `gemm` (4 waves, two slabs ahead), the K-split
-    # symbols (8 waves; the deep one three batches ahead).
+    # symbols (8 waves; two sets of loads in registers).
     by = {row["symbol"]: row for row in rows}
     assert (by["gemm"]["bm"], by["gemm"]["bn"], by["gemm"]["waves"], by["gemm"]["unroll"]) == ("128", "256", "4", "2")
-    assert (by["gemm_mid"]["unroll"], by["gemm_ksplit"]["waves"], by["gemm_ksplit_deep"]["unroll"]) == ("1", "8", "3")
+    assert (by["gemm_mid"]["unroll"], by["gemm_ksplit"]["waves"], by["gemm_ksplit_deep"]["unroll"]) == ("1", "8", "2")
     assert {row["vec"] for row in rows} == {"4"}  # k, n multiples of 4: dwordx4 loads
     assert all(row["product"] == ("1" if i < 10 else "0") for i, row in enumerate(rows))
     best = min(rows, key=lambda row: float(row["ms_median"]))["symbol"]
