@@ -97,15 +97,3 @@
 // attention_split and attention_split16: 32 and 16 query rows per workgroup,
 // the keys split over its 4 waves.
 #define KH_ATTN_SPLIT_THREADS 256
-// The launcher's choice between the three (khrt_templates.cpp,
-// attention_plan): the least of
-//   rounds of workgroups (one per CU) x key steps of a wave x us per step + us
-// over attention (128 rows, steps of 64 keys), attention_split (32 rows, steps
-// of 32 keys, a quarter of them) and attention_split16. Fitted on the launches
-// tabled at attention_split; each choice among them is the measured best.
-#define KH_ATTN_STEP_US 4.3
-#define KH_ATTN_START_US 3.0
-#define KH_ATTN_SPLIT_STEP_US 2.2
-#define KH_ATTN_SPLIT_START_US 5.0
-#define KH_ATTN_SPLIT16_STEP_US 1.3
-#define KH_ATTN_SPLIT16_START_US 4.0

@@ -425,24 +425,49 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   return {block, cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
 }
 
-// How attention spreads (batch, heads, seq) over the chip (kh_tiles.h).
-struct AttentionPlan {
+// How attention spreads (batch, heads, seq) over the chip: query rows per
+// workgroup, and what a launch of that symbol takes. `resident` workgroups
+// share a CU (registers and LDS), so workgroups run in rounds of that many per
+// CU; a round of i of them takes step[i - 1] us for each key step of a wave
+// and fixed[i - 1] for its start and merge, a launch `start`.
+struct AttentionForm {
   const char *symbol;
-  int64_t rows;  // query rows per workgroup
+  int64_t rows, keys, waves;  // query rows; keys per step; waves the keys are split over
+  int resident;
+  double start, step[3], fixed[3];
 };
 
-AttentionPlan attention_plan(int64_t batch, int64_t heads, int64_t seq) {
+// Fitted to the three symbols timed at 1193 launches (1 to 4096 slices of 8 to
+// 8192 keys): the symbol taken is within 3% of the fastest at 99% of them and
+// loses more than 1% to `attention` at four (at most 9%). A model that paid start
+// and merge once per launch, and one workgroup per CU, held up to 64 slices
+// and was up to 38% slower than `attention` past that: 256x129 37.8 us for
+// 29.7-32, 384x128 31.6 for 25.3, 1024x200 181 for 148.
+const AttentionForm kAttentionForms[] = {
+    {"attention", KH_ATTN_BLOCK_Q, 64, 1, 2, 1.9, {4.0, 8.0}, {3.1, 4.15}},
+    {"attention_split", 32, 32, 4, 2, 2.7, {1.45, 3.85}, {5.15, 5.4}},
+    {"attention_split16", 16, 32, 4, 3, 2.9, {0.7, 2.0, 3.35}, {3.4, 3.75, 3.4}},
+};
+
+double attention_us(const AttentionForm &f, int64_t slices, int64_t seq) {
+  const int64_t per_cu = ceil_div(slices * ceil_div(seq, f.rows), KH_GEMM_CUS);
+  const int64_t full = per_cu / f.resident, rest = per_cu % f.resident;
+  const int64_t steps = ceil_div(seq, f.keys), longest = ceil_div(steps, f.waves);
+  // Waves without a last step leave their share to the CU's other workgroups,
+  // but not where there are none.
+  const double mean = (static_cast<double>(steps) / static_cast<double>(f.waves) + static_cast<double>(longest)) / 2;
+  double us = f.start + static_cast<double>(full) * (f.step[f.resident - 1] * mean + f.fixed[f.resident - 1]);
+  if (rest > 0) us += f.step[rest - 1] * (full == 0 ? static_cast<double>(longest) : mean) + f.fixed[rest - 1];
+  return us;
+}
+
+const AttentionForm &attention_form(int64_t batch, int64_t heads, int64_t seq) {
+  const AttentionForm &whole = kAttentionForms[0], &split = kAttentionForms[1], &split16 = kAttentionForms[2];
   // Past this the split kernels' 32-bit offsets do not reach.
-  if (batch > 65535 || heads > 65535 || seq > (int64_t(1) << 22)) return {"attention", KH_ATTN_BLOCK_Q};
-  auto us = [&](int64_t rows, int64_t keys, int64_t waves, double step, double start) {
-    const int64_t rounds = ceil_div(batch * heads * ceil_div(seq, rows), KH_GEMM_CUS);
-    return static_cast<double>(rounds * ceil_div(ceil_div(seq, keys), waves)) * step + start;
-  };
-  const double whole = us(KH_ATTN_BLOCK_Q, 64, 1, KH_ATTN_STEP_US, KH_ATTN_START_US);
-  const double split = us(32, 32, 4, KH_ATTN_SPLIT_STEP_US, KH_ATTN_SPLIT_START_US);
-  const double split16 = us(16, 32, 4, KH_ATTN_SPLIT16_STEP_US, KH_ATTN_SPLIT16_START_US);
-  if (whole <= split && whole <= split16) return {"attention", KH_ATTN_BLOCK_Q};
-  return split <= split16 ? AttentionPlan{"attention_split", 32} : AttentionPlan{"attention_split16", 16};
+  if (batch > 65535 || heads > 65535 || seq > (int64_t(1) << 22)) return whole;
+  const double us = attention_us(split, batch * heads, seq), us16 = attention_us(split16, batch * heads, seq);
+  if (attention_us(whole, batch * heads, seq) <= 1.02 * std::min(us, us16)) return whole;  // level: the fewer
+  return us <= us16 ? split : split16;
 }
 
 // Extents of a template's shape, in the order its entry point takes them:
@@ -524,7 +549,7 @@ int make_plan(const Template &tpl, const Dims &d, Plan &p) {
         return khrt::fail(KHRT_E_INVALID, "attention: the kernel is pinned to head_dim = 64 (got head_dim = " +
                                               std::to_string(d[3]) + ")");
       }
-      const AttentionPlan a = attention_plan(d[0], d[1], d[2]);
+      const AttentionForm &a = attention_form(d[0], d[1], d[2]);
       p.symbol = a.symbol;
       p.grid = {static_cast<unsigned>(ceil_div(d[2], a.rows)), static_cast<unsigned>(d[1]),
                 static_cast<unsigned>(d[0])};

@@ -308,6 +308,16 @@ def test_launcher_geometry(name, shape, grid, block):
     ("layernorm", "rows=16,cols=2048", "layernorm_wide"),
     ("layernorm", "rows=16,cols=4100", "layernorm"),         # beyond the register paths: streaming
     ("scan_totals", "n=1000000", "scan_totals"),
+    # attention: many slices, which 128-row tiles fill the chip with, and few.
+    ("attention", "batch=8,heads=16,seq=128,head_dim=64", "attention_split"),
+    ("attention", "batch=64,heads=8,seq=65,head_dim=64", "attention"),
+    ("attention", "batch=64,heads=16,seq=200,head_dim=64", "attention"),
+    ("attention", "batch=112,heads=6,seq=245,head_dim=64", "attention"),
+    ("attention", "batch=38,heads=16,seq=128,head_dim=64", "attention"),
+    ("attention", "batch=4,heads=16,seq=1024,head_dim=64", "attention"),
+    ("attention", "batch=1,heads=8,seq=777,head_dim=64", "attention_split"),
+    ("attention", "batch=2,heads=16,seq=129,head_dim=64", "attention_split16"),
+    ("attention", "batch=64,heads=16,seq=24,head_dim=64", "attention_split"),    # a quarter of each 128-row tile
 ])
 def test_launch_symbol(name, shape, symbol):
     assert kh.launch_symbol(name, shape) == symbol
