@@ -87,6 +87,7 @@ static_assert(Tile<2, 2, 32, false>::BM == KH_GEMM_MID_BM && Tile<2, 2, 32, fals
               "launcher tile size");
 static_assert(Tile<1, 2, 32, true, 4, 2, 16>::BM == KH_GEMM_SMALL_BM &&
                   Tile<1, 2, 32, true, 4, 2, 16>::BN == KH_GEMM_SMALL_BN &&
+                  Tile<1, 2, 32, true, 4, 2, 16>::BK == KH_GEMM_SMALL_BK &&
                   Tile<1, 2, 32, true, 4, 2, 16>::NT == KH_GEMM_SMALL_THREADS &&
                   Tile<2, 2, 32, false, 2, 2, 16>::BM == KH_GEMM_SMALL_BM &&
                   Tile<2, 2, 32, false, 2, 2, 16>::BN == KH_GEMM_SMALL_BN,

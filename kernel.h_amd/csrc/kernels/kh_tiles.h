@@ -35,6 +35,7 @@
 #define KH_GEMM_MID_BN 128
 #define KH_GEMM_SMALL_BM 64
 #define KH_GEMM_SMALL_BN 64
+#define KH_GEMM_SMALL_BK 32
 // `gemm_small` runs eight waves (512 threads), two workgroups per CU.
 #define KH_GEMM_SMALL_THREADS 512
 // `gemm_wide`: 128x128 tiles on eight waves (512 threads), one workgroup per

@@ -361,7 +361,10 @@ const char *heuristic_gemm_symbol(int64_t m, int64_t n, int64_t k) {
       k % KH_GEMM_KSPLIT_INTERIOR_K == 0 && k >= KH_GEMM_KSPLIT_MIN_K) {
     return ks32;
   }
-  if (ks_tiles(32, 64) <= KH_GEMM_CUS) return "gemm_ksplit_32x64";
+  // Past a slab of the 64x64 tiles only: their merge of eight waves' partial
+  // tiles costs more than a single slab's products (448x640, K of 1 to 32: 4.5 us
+  // against 4.0 in `gemm_small`; K = 33: 4.6 against 4.9).
+  if (k > KH_GEMM_SMALL_BK && ks_tiles(32, 64) <= KH_GEMM_CUS) return "gemm_ksplit_32x64";
   const double big = gemm_score(ceil_div(m, KH_GEMM_BM) * ceil_div(n, KH_GEMM_BN), KH_GEMM_ROUND_BIG,
                                 KH_GEMM_RATE_BIG);
   const double mid = gemm_score(ceil_div(m, KH_GEMM_MID_BM) * ceil_div(n, KH_GEMM_MID_BN), KH_GEMM_ROUND_MID,

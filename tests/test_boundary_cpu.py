@@ -303,6 +303,9 @@ def test_launcher_geometry(name, shape, grid, block):
     ("gemm", "m=256,n=2048,k=2048", "gemm_ksplit_deep"),
     ("gemm", "m=1024,n=1024,k=512", "gemm_small"),           # 256 tiles of 64x64
     ("gemm", "m=760,n=768,k=768", "gemm_small"),             # an edge tile in m
+    ("gemm", "m=448,n=640,k=32", "gemm_small"),              # one slab: no K to split
+    ("gemm", "m=448,n=640,k=33", "gemm_ksplit_32x64"),
+    ("gemm", "m=290,n=1295,k=19", "gemm_small"),
     ("softmax", "rows=4096,cols=1024", "softmax"),
     ("softmax", "rows=16384,cols=4096", "softmax_wide"),
     ("layernorm", "rows=16,cols=2048", "layernorm_wide"),
