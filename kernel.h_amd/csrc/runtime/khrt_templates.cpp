@@ -353,14 +353,19 @@ const char *heuristic_gemm_symbol(int64_t m, int64_t n, int64_t k) {
   // tiles number fewer than the CUs.
   auto ks_tiles = [&](int64_t bm, int64_t bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
   const char *ks32 = k >= KH_GEMM_KSPLIT_DEEP_K ? "gemm_ksplit_deep" : "gemm_ksplit";
+  const bool whole = m % KH_GEMM_KSPLIT_BM == 0 && n % KH_GEMM_KSPLIT_BN == 0 && k % KH_GEMM_KSPLIT_INTERIOR_K == 0;
   const int64_t tiles64 = ks_tiles(KH_GEMM_SMALL_BM, KH_GEMM_SMALL_BN);
-  if (ks_tiles(16, 16) <= KH_GEMM_CUS) return "gemm_ksplit_16x16";
-  if (ks_tiles(32, 16) <= KH_GEMM_CUS) return "gemm_ksplit_32x16";
+  // Whole 32x32 tiles move 16 k a batch and wave, the smaller tiles 32, so that
+  // an odd multiple of 128 leaves each of their waves half a batch of padding.
+  // One 32x16 tile per CU against a 32x32 one on half of them, K = 128: 4.0 vs
+  // 3.2 us, 384 5.3 vs 4.6, 640 6.3 vs 5.8, 1408 10.4 vs 9.4, 1920 13.2 vs 11.8
+  // (256, 512 and 1024 level; 2048 and past it the smaller, 512x256x4096 22.0 vs
+  // 23.8). A 16x16 tile wins but at K = 128: 3.3-3.5 vs 2.9-3.2 us (256 3.4 vs 3.9).
+  const bool half = whole && k % (2 * KH_GEMM_KSPLIT_INTERIOR_K) != 0;
+  if (ks_tiles(16, 16) <= KH_GEMM_CUS) return half && k == KH_GEMM_KSPLIT_INTERIOR_K ? ks32 : "gemm_ksplit_16x16";
+  if (ks_tiles(32, 16) <= KH_GEMM_CUS) return half && k < KH_GEMM_KSPLIT_DEEP_K ? ks32 : "gemm_ksplit_32x16";
   if (ks_tiles(KH_GEMM_KSPLIT_BM, KH_GEMM_KSPLIT_BN) <= KH_GEMM_CUS) return ks32;
-  if (tiles64 < KH_GEMM_CUS && m % KH_GEMM_KSPLIT_BM == 0 && n % KH_GEMM_KSPLIT_BN == 0 &&
-      k % KH_GEMM_KSPLIT_INTERIOR_K == 0 && k >= KH_GEMM_KSPLIT_MIN_K) {
-    return ks32;
-  }
+  if (tiles64 < KH_GEMM_CUS && whole && k >= KH_GEMM_KSPLIT_MIN_K) return ks32;
   // Past a slab of the 64x64 tiles only: their merge of eight waves' partial
   // tiles costs more than a single slab's products (448x640, K of 1 to 32: 4.5 us
   // against 4.0 in `gemm_small`; K = 33: 4.6 against 4.9).

@@ -303,6 +303,12 @@ def test_launcher_geometry(name, shape, grid, block):
     ("gemm", "m=256,n=2048,k=2048", "gemm_ksplit_deep"),
     ("gemm", "m=1024,n=1024,k=512", "gemm_small"),           # 256 tiles of 64x64
     ("gemm", "m=760,n=768,k=768", "gemm_small"),             # an edge tile in m
+    ("gemm", "m=64,n=64,k=128", "gemm_ksplit"),              # whole 32x32 tiles, half a batch of the smaller ones
+    ("gemm", "m=64,n=64,k=256", "gemm_ksplit_16x16"),
+    ("gemm", "m=64,n=60,k=128", "gemm_ksplit_16x16"),
+    ("gemm", "m=256,n=512,k=384", "gemm_ksplit"),
+    ("gemm", "m=256,n=512,k=512", "gemm_ksplit_32x16"),
+    ("gemm", "m=256,n=512,k=2176", "gemm_ksplit_32x16"),
     ("gemm", "m=448,n=640,k=32", "gemm_small"),              # one slab: no K to split
     ("gemm", "m=448,n=640,k=33", "gemm_ksplit_32x64"),
     ("gemm", "m=290,n=1295,k=19", "gemm_small"),
