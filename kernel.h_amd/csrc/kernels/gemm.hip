@@ -602,9 +602,9 @@ gemm_ksplit(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(f
   KH_KSPLIT_32X32(1);
 }
 
-// The same with twice the loads in flight in the general form: the launcher
-// takes it over `gemm_ksplit` for K >= KH_GEMM_KSPLIT_DEEP_K (2000x128x8192
-// and 16x8192x8192 within 3% of each other either way).
+// The same with twice the loads in flight in the general form, for long K over
+// operands the L2s do not hold (the rule and what it rests on:
+// KH_GEMM_KSPLIT_DEEP_FLOATS).
 extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit_deep(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
   KH_KSPLIT_32X32(2);

@@ -89,9 +89,17 @@
 #define KH_GEMM_KSPLIT_THREADS 512
 #define KH_GEMM_KSPLIT_INTERIOR_K 128
 #define KH_GEMM_KSPLIT_MIN_K 256
-// From this K on, the launcher takes `gemm_ksplit_deep` (three batches of
-// loads in flight per wave) for the same launches.
+// `gemm_ksplit_deep` (twice the loads in flight in the form for tiles that are
+// not all whole) is taken from this K on, for operands of at least so many
+// floats: past what the L2s hold, where each load takes longer. Events around
+// rotated launches, gemm_ksplit / gemm_ksplit_deep:
+//   300x520x7001      5.7 M floats  46.2 / 49.7    500x500x8191   8.2 M  52.6 / 52.1
+//   500x500x9999     10.0           63.4 / 64.2    500x500x12001 12.0    77.5 / 74.6
+//   100x2000x9999    21.0           66.8 / 69.0    500x500x16001 16.0   103.8 / 98.5
+//   1500x150x16001   26.4            124 / 109     8000x30x5001  40.2    54.8 / 48.3
+// Where all are whole the two run the same code.
 #define KH_GEMM_KSPLIT_DEEP_K 2048
+#define KH_GEMM_KSPLIT_DEEP_FLOATS (1 << 24)
 
 // Attention: query rows per workgroup (4 wavefronts x 32 rows).
 #define KH_ATTN_BLOCK_Q 128

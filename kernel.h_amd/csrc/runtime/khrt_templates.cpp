@@ -352,8 +352,10 @@ const char *heuristic_gemm_symbol(int64_t m, int64_t n, int64_t k) {
   // workgroup; of 32x32 tiles also more, where all are whole and the 64x64
   // tiles number fewer than the CUs.
   auto ks_tiles = [&](int64_t bm, int64_t bn) { return ceil_div(m, bm) * ceil_div(n, bn); };
-  const char *ks32 = k >= KH_GEMM_KSPLIT_DEEP_K ? "gemm_ksplit_deep" : "gemm_ksplit";
   const bool whole = m % KH_GEMM_KSPLIT_BM == 0 && n % KH_GEMM_KSPLIT_BN == 0 && k % KH_GEMM_KSPLIT_INTERIOR_K == 0;
+  const bool deep = k >= KH_GEMM_KSPLIT_DEEP_K &&
+                    (whole || static_cast<double>(m + n) * static_cast<double>(k) >= KH_GEMM_KSPLIT_DEEP_FLOATS);
+  const char *ks32 = deep ? "gemm_ksplit_deep" : "gemm_ksplit";
   const int64_t tiles64 = ks_tiles(KH_GEMM_SMALL_BM, KH_GEMM_SMALL_BN);
   // Whole 32x32 tiles move 16 k a batch and wave, the smaller tiles 32, so that
   // an odd multiple of 128 leaves each of their waves half a batch of padding.

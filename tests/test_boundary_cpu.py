@@ -303,6 +303,8 @@ def test_launcher_geometry(name, shape, grid, block):
     ("gemm", "m=256,n=2048,k=2048", "gemm_ksplit_deep"),
     ("gemm", "m=1024,n=1024,k=512", "gemm_small"),           # 256 tiles of 64x64
     ("gemm", "m=760,n=768,k=768", "gemm_small"),             # an edge tile in m
+    ("gemm", "m=500,n=500,k=7001", "gemm_ksplit"),           # operands the L2s hold
+    ("gemm", "m=1500,n=150,k=16001", "gemm_ksplit_deep"),
     ("gemm", "m=64,n=64,k=128", "gemm_ksplit"),              # whole 32x32 tiles, half a batch of the smaller ones
     ("gemm", "m=64,n=64,k=256", "gemm_ksplit_16x16"),
     ("gemm", "m=64,n=60,k=128", "gemm_ksplit_16x16"),
