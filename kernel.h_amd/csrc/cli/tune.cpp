@@ -258,7 +258,8 @@ void usage_tune(std::ostream &os) {
      << "(gemm_tune_space.py): MFMA 32x32 or 16x16 wave tiles, 4 or 8 waves, BM/BN in\n"
      << "{64,128,256}, BK in {16,32}, unroll 1 or 2 (register-staged, direct-to-LDS\n"
      << "three stages, or two slabs ahead), MFMA wave priority; vec is 4 (dwordx4)\n"
-     << "when k and n are multiples of 4, else 1. The space is precompiled; it is\n"
+     << "when k and n are multiples of 4 and, for the persistent and K-split symbols,\n"
+     << "at other extents too, else 1. The space is precompiled; it is\n"
      << "evaluated whole unless --sample/--refine-budget ask for the sampled search.\n"
      << "Point the runtime at the cache\n"
      << "(KHRT_TUNE_CACHE=<path> or khrt_set_tune_cache) and kh_gemm runs the\n"
@@ -542,10 +543,15 @@ int run_tune(int argc, char **argv) {
     }
   }
 
-  // vec: floats per global load the candidate issues at this shape: float4
-  // (dwordx4) when k (and, except for the K-split symbols, which read B a
-  // column at a time, n) are multiples of 4, else the guarded scalar path.
-  const int vec_tiles = (k % 4 == 0 && n % 4 == 0) ? 4 : 1, vec_ksplit = (k % 4 == 0) ? 4 : 1;
+  // vec: floats per load of A the candidate issues at this shape. K-split
+  // symbols and, past one slab and below 32-bit tile offsets, the persistent ones
+  // load float4s (dwordx4) at any extent; the others where k and n are
+  // multiples of 4, else an element at a time.
+  auto vec = [&](const Candidate &c) {
+    constexpr int64_t kSpan = int64_t(1) << 29;  // floats
+    const bool any = c.k_split || (c.persistent && k > c.bk && c.bm * k < kSpan && c.bk * n < kSpan && c.bm * n < kSpan);
+    return any || (k % 4 == 0 && n % 4 == 0) ? 4 : 1;
+  };
   std::ostringstream csv;
   csv << "kernel,shape,bm,bn,bk,waves,unroll,vec,ms_median,accepted,reason,symbol,mfma,wave_grid,wave_tile,"
          "pipeline,prio,product,gflops\n";
@@ -553,7 +559,7 @@ int run_tune(int argc, char **argv) {
   for (const Result &r : results) {
     const Candidate &c = *r.c;
     csv << kernel << "," << csv_escape(shape_text) << "," << c.bm << "," << c.bn << "," << c.bk << "," << c.waves
-        << "," << c.unroll << "," << (c.k_split ? vec_ksplit : vec_tiles) << "," << r.ms << ","
+        << "," << c.unroll << "," << vec(c) << "," << r.ms << ","
         << (r.accepted ? "true" : "false") << "," << csv_escape(r.reason) << "," << c.symbol << "," << c.mfma << "x"
         << c.mfma << "," << c.wave_grid_m << "x" << c.wave_grid_n << "," << c.wave_tile_m << "x" << c.wave_tile_n
         << "," << c.pipeline << "," << c.prio << "," << c.product << "," << r.gflops << "\n";

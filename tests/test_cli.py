@@ -250,13 +250,17 @@ def test_tune_sampled_search(dev, tmp_path):
 
 @pytest.mark.gpu
 def test_tune_vec_column_follows_the_shape(dev, tmp_path):
-    # k not a multiple of 4: every candidate takes its guarded scalar loads.
-    print("[gpu-case] kernelh tune gemm m=100,n=100,k=33, 2 candidates", flush=True)
-    r = run("tune", "--shape", "m=100,n=100,k=33", "--out", str(tmp_path), "--max-candidates", "2",
+    # k no multiple of 4: the persistent symbols (past one slab: 16 deep in
+    # `gemm`, 32 in `gemm_small` and `gemm_wide`) and the K-split ones still
+    # load float4s, the register-staged ones an element at a time.
+    print("[gpu-case] kernelh tune gemm m=100,n=100,k=31, 8 candidates", flush=True)
+    r = run("tune", "--shape", "m=100,n=100,k=31", "--out", str(tmp_path), "--max-candidates", "8",
             "--cache", str(tmp_path / "c.json"))
     assert r.returncode == 0, r.stdout
     rows = list(csv.DictReader(open(tmp_path / "tune-results.csv")))
-    assert [row["vec"] for row in rows] == ["1", "1"]
+    assert {row["symbol"]: row["vec"] for row in rows} == {
+        "gemm": "4", "gemm_mid": "1", "gemm_small": "1", "gemm_small_pf2": "1", "gemm_wide": "1",
+        "gemm_ksplit": "4", "gemm_ksplit_deep": "4", "gemm_ksplit_16x16": "4"}
     assert all(row["accepted"] == "true" for row in rows), rows
 
 
