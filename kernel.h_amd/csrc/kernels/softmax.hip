@@ -257,11 +257,11 @@ __device__ __forceinline__ void softmax_row_serial(const float *__restrict__ xr,
                                                    int64_t cols) {
   float m = -__builtin_inff();
   for (int64_t c = 0; c < cols; ++c) m = fmaxf(m, xr[c]);
-  const float mb = -m * kh::kLog2e;
+  // The maximum is subtracted first, so that rows of any size do (shift_extreme).
   float s = 0.0f;
-  for (int64_t c = 0; c < cols; ++c) s += kh::exp2_hw(fmaf(xr[c], kh::kLog2e, mb));
+  for (int64_t c = 0; c < cols; ++c) s += kh::exp2_hw((xr[c] - m) * kh::kLog2e);
   const float inv = 1.0f / s;
-  for (int64_t c = 0; c < cols; ++c) yr[c] = kh::exp2_hw(fmaf(xr[c], kh::kLog2e, mb)) * inv;
+  for (int64_t c = 0; c < cols; ++c) yr[c] = kh::exp2_hw((xr[c] - m) * kh::kLog2e) * inv;
 }
 
 // Which register paths a symbol compiles in: the kernel's register

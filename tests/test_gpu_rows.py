@@ -233,6 +233,24 @@ def test_softmax_extreme_rows(dev, cols):
     assert np.nanmax(np.abs(got - ref)) <= 1e-6
 
 
+@pytest.mark.parametrize("cols", [40, 100, 250])
+def test_softmax_extreme_rows_partial_wave_blocks(dev, cols):
+    # The same rows in blocks that are not whole waves, a thread per row.
+    low = np.finfo(np.float32).min
+    x = O.normal(7 * cols, 0xE28, 0.0, 1.0).reshape(7, cols)
+    x[0], x[1], x[2], x[3, : cols // 2], x[4, 0], x[5, : cols // 2] = low, 3e38, -np.inf, low, np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        e = np.exp(x.astype(np.float64) - np.max(x.astype(np.float64), axis=1, keepdims=True))
+        ref = e / e.sum(axis=1, keepdims=True)
+    dx, dy = up(x.ravel()), empty(7 * cols)
+    args = kh.LaunchArgs().add_memref(dx, [7, cols]).add_memref(dy, [7, cols])
+    say(f"softmax extreme rows, cols={cols}, block={cols}")
+    kh.launch_raw(kh.template_function("softmax"), (7, 1, 1), (cols, 1, 1), args)
+    got = down(dy, 7 * cols).reshape(7, cols)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.nanmax(np.abs(got - ref)) <= 1e-6
+
+
 @pytest.mark.parametrize("symbol", ["softmax", "softmax_wide", "softmax_block"])
 @pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
 @pytest.mark.parametrize("block", [64, 256])
