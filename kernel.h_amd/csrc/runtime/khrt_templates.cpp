@@ -419,6 +419,7 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   if (cols <= KH_ROW16_COLS) return {narrow, 256, 16};
   if (cols <= 1024) return {narrow, 256, 4};
   if (cols <= 2048) return {wide, 256, 4};
+  if (cols > KH_ROW_BLOCK_MAX) return {block, 1024, 1};
   // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
   // per thread: the fewest that need at most 768 threads, so that a CU's 2048
   // hold two workgroups and one's loads fill the other's reductions and
@@ -432,7 +433,7 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   if (cols <= 4096) return {wide, threads(4), 1};
   if (threads(4) <= 768) return {narrow, threads(4), 1};
   if (threads(8) <= 768 || (threads(8) <= 1024 && rows <= KH_GEMM_CUS)) return {narrow, threads(8), 1};
-  return {block, cols <= KH_ROW_BLOCK_MAX ? threads(16) : 1024, 1};
+  return {block, threads(16), 1};
 }
 
 // How attention spreads (batch, heads, seq) over the chip: query rows per

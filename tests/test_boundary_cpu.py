@@ -285,6 +285,22 @@ def test_launcher_geometry(name, shape, grid, block):
     assert kh.geometry(name, shape) == (grid, block)
 
 
+@pytest.mark.parametrize("name", ["softmax", "layernorm"])
+@pytest.mark.parametrize("rows,cols,suffix,grid,threads", [
+    (5, 256, "", 1, 256), (5, 1024, "", 2, 256), (5, 1025, "_wide", 2, 256), (5, 2048, "_wide", 2, 256),
+    (5, 2049, "_wide", 5, 192), (5, 4096, "_wide", 5, 256),
+    # 4, 8 and 16 float4 per thread, at most 768 threads; up to a CU for every row 8 to 1024.
+    (5, 4097, "", 5, 320), (5, 12288, "", 5, 768), (5, 12289, "", 5, 448), (5, 24576, "", 5, 768),
+    (256, 24577, "", 256, 832), (256, 32768, "", 256, 1024), (257, 24577, "_block", 257, 448),
+    (257, 32768, "_block", 257, 512), (5, 32769, "_block", 5, 576), (5, 65536, "_block", 5, 1024),
+    (5, 65537, "_block", 5, 1024), (1, 1 << 36, "_block", 1, 1024), (1, (1 << 63) - 1, "_block", 1, 1024),
+])
+def test_row_plan(name, rows, cols, suffix, grid, threads):
+    shape = f"rows={rows},cols={cols}"
+    assert kh.launch_symbol(name, shape) == name + suffix
+    assert kh.geometry(name, shape) == ((grid, 1, 1), (threads, 1, 1))
+
+
 @pytest.mark.parametrize("name,shape,symbol", [
     ("gemm", "m=8192,n=8192,k=8192", "gemm"),
     ("gemm", "m=8192,n=8192,k=256", "gemm"),
