@@ -9,7 +9,8 @@
 // traffic per element. What holds a row depends on its width:
 //
 //   cols <= 256            16 lanes, four rows per wavefront (rows16)
-//   cols <= 2048           one wavefront (row_regs; the wide symbol past 1024)
+//   cols <= 2048           one wavefront (row_regs; softmax_wave up to 512, the
+//                          wide symbol past 1024)
 //   cols <= 65536          one workgroup (row_block)
 //   beyond                 one workgroup in two sweeps (row_stream)
 //
@@ -264,6 +265,24 @@ __device__ __forceinline__ void softmax_row_serial(const float *__restrict__ xr,
   for (int64_t c = 0; c < cols; ++c) yr[c] = kh::exp2_hw((xr[c] - m) * kh::kLog2e) * inv;
 }
 
+// Any width in one wavefront, for launches of softmax_wave past what its
+// registers hold: an online (max, sum) per lane, merged, then a second sweep.
+__device__ __forceinline__ void softmax_row_wave(const float *__restrict__ xr, float *__restrict__ yr, int64_t cols,
+                                                 int lane) {
+  const float ninf = -__builtin_inff();
+  float m = ninf, s = 0.0f;
+  for (int64_t c = lane; c < cols; c += kh::kWave) {
+    const float x = xr[c], mn = fmaxf(m, x);
+    const float ref = mn == ninf ? 0.0f : mn;  // nothing but -inf so far: every term is 0
+    s = s * kh::exp2_hw((m - ref) * kh::kLog2e) + kh::exp2_hw((x - ref) * kh::kLog2e);
+    m = mn;
+  }
+  const float gm = kh::wave_max(m);
+  s = s == 0.0f ? 0.0f : s * kh::exp2_hw((m - gm) * kh::kLog2e);
+  const float inv = 1.0f / kh::wave_sum(s);
+  for (int64_t c = lane; c < cols; c += kh::kWave) yr[c] = kh::exp2_hw((xr[c] - gm) * kh::kLog2e) * inv;
+}
+
 // Which register paths a symbol compiles in: the kernel's register
 // allocation is that of its widest path, so the narrow symbol stays lean
 // (more rows in flight per CU).
@@ -337,6 +356,36 @@ __device__ __forceinline__ void softmax_rows(const float *__restrict__ X, float 
 extern "C" __global__ void __launch_bounds__(1024)
 softmax(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
   KH_SOFTMAX_BODY(kNarrow);
+}
+
+// Same arguments and results for rows of 257..512 floats: a wave per row and
+// nothing else, without LDS. The path is `softmax`'s, instruction for
+// instruction, but as one of that symbol's many it took 2-9% longer: 9300x272
+// 6.25 -> 5.80 us, 40000x272 16.9 -> 15.8, 16384x300 9.0 -> 8.6, 16384x512 13.2 ->
+// 12.8; at 700 and 1024 columns it is 1% slower (40000x1024 53.6 -> 54.3), which is
+// where the line lies.
+extern "C" __global__ void __launch_bounds__(256)
+softmax_wave(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
+  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();
+  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, y_base, y_off, y_s0, gw, nb);
+  const float *__restrict__ X = KH_PTR(x);
+  float *__restrict__ Y = KH_PTR(y);
+  const int bd = (int)kh::threads_x_of(gw);
+  const int64_t rows = x_n0, cols = x_n1, step = (int64_t)(bd / kh::kWave) * nb;
+  if (bd % kh::kWave != 0) {
+    for (int64_t r = (int64_t)blockIdx.x * bd + threadIdx.x; r < rows; r += (int64_t)bd * nb)
+      softmax_row_serial(X + r * x_s0, Y + r * y_s0, cols);
+    return;
+  }
+  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  for (int64_t r = (int64_t)blockIdx.x * (bd / kh::kWave) + wave; r < rows; r += step) {
+    if (cols <= 256)
+      softmax_row_regs<1>(X + r * x_s0, Y + r * y_s0, (int)cols, lane);
+    else if (cols <= 512)
+      softmax_row_regs<2>(X + r * x_s0, Y + r * y_s0, (int)cols, lane);
+    else
+      softmax_row_wave(X + r * x_s0, Y + r * y_s0, cols, lane);
+  }
 }
 
 // Same arguments and results for rows of 1025..4096 floats (the launcher picks

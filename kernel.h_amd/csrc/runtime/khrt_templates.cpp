@@ -417,6 +417,7 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   const char *narrow = softmax ? "softmax" : "layernorm", *wide = softmax ? "softmax_wide" : "layernorm_wide",
              *block = softmax ? "softmax_block" : "layernorm_block";
   if (cols <= KH_ROW16_COLS) return {narrow, 256, 16};
+  if (softmax && cols <= 512) return {"softmax_wave", 256, 4};
   if (cols <= 1024) return {narrow, 256, 4};
   if (cols <= 2048) return {wide, 256, 4};
   if (cols > KH_ROW_BLOCK_MAX) return {block, 1024, 1};

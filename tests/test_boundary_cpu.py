@@ -287,7 +287,7 @@ def test_launcher_geometry(name, shape, grid, block):
 
 @pytest.mark.parametrize("name", ["softmax", "layernorm"])
 @pytest.mark.parametrize("rows,cols,suffix,grid,threads", [
-    (5, 256, "", 1, 256), (5, 1024, "", 2, 256), (5, 1025, "_wide", 2, 256), (5, 2048, "_wide", 2, 256),
+    (5, 256, "", 1, 256), (5, 513, "", 2, 256), (5, 1024, "", 2, 256), (5, 1025, "_wide", 2, 256), (5, 2048, "_wide", 2, 256),
     (5, 2049, "_wide", 5, 192), (5, 4096, "_wide", 5, 256),
     # 4, 8 and 16 float4 per thread, at most 768 threads; up to a CU for every row 8 to 1024.
     (5, 4097, "", 5, 320), (5, 12288, "", 5, 768), (5, 12289, "", 5, 448), (5, 24576, "", 5, 768),
@@ -299,6 +299,16 @@ def test_row_plan(name, rows, cols, suffix, grid, threads):
     shape = f"rows={rows},cols={cols}"
     assert kh.launch_symbol(name, shape) == name + suffix
     assert kh.geometry(name, shape) == ((grid, 1, 1), (threads, 1, 1))
+
+
+@pytest.mark.parametrize("shape,symbol,grid", [
+    ("softmax rows=5,cols=257", "softmax_wave", 2), ("softmax rows=40000,cols=512", "softmax_wave", 10000),
+    ("layernorm rows=5,cols=257", "layernorm", 2),
+])
+def test_row_plan_of_one_template(shape, symbol, grid):
+    name, shape = shape.split(" ")
+    assert kh.launch_symbol(name, shape) == symbol
+    assert kh.geometry(name, shape) == ((grid, 1, 1), (256, 1, 1))
 
 
 @pytest.mark.parametrize("name,shape,symbol", [

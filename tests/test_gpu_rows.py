@@ -72,7 +72,7 @@ def test_softmax_reference_geometry(dev):
     assert np.max(np.abs(down(dy, rows * cols).reshape(rows, cols) - O.ref_softmax(x, rows, cols))) <= 1e-4
 
 
-@pytest.mark.parametrize("symbol", ["softmax", "softmax_wide", "layernorm", "layernorm_wide"])
+@pytest.mark.parametrize("symbol", ["softmax", "softmax_wave", "softmax_wide", "layernorm", "layernorm_wide"])
 @pytest.mark.parametrize("cols", [64, 256, 512, 1000, 1024, 2048, 4096, 5000])
 def test_every_row_symbol_at_every_width(dev, symbol, cols):
     # Each symbol of a template computes the same result at every width (the
@@ -233,9 +233,11 @@ def test_softmax_extreme_rows(dev, cols):
     assert np.nanmax(np.abs(got - ref)) <= 1e-6
 
 
-@pytest.mark.parametrize("cols", [40, 100, 250])
-def test_softmax_extreme_rows_partial_wave_blocks(dev, cols):
-    # The same rows in blocks that are not whole waves, a thread per row.
+@pytest.mark.parametrize("symbol,block", [("softmax", 40), ("softmax_wave", 40), ("softmax_wave", 128)])
+@pytest.mark.parametrize("cols", [40, 100, 250, 700])
+def test_softmax_extreme_rows_raw_launches(dev, symbol, block, cols):
+    # The same rows in blocks that are not whole waves, a thread per row, and in
+    # the wave symbol at widths the launcher does not give it.
     low = np.finfo(np.float32).min
     x = O.normal(7 * cols, 0xE28, 0.0, 1.0).reshape(7, cols)
     x[0], x[1], x[2], x[3, : cols // 2], x[4, 0], x[5, : cols // 2] = low, 3e38, -np.inf, low, np.inf, -np.inf
@@ -244,14 +246,15 @@ def test_softmax_extreme_rows_partial_wave_blocks(dev, cols):
         ref = e / e.sum(axis=1, keepdims=True)
     dx, dy = up(x.ravel()), empty(7 * cols)
     args = kh.LaunchArgs().add_memref(dx, [7, cols]).add_memref(dy, [7, cols])
-    say(f"softmax extreme rows, cols={cols}, block={cols}")
-    kh.launch_raw(kh.template_function("softmax"), (7, 1, 1), (cols, 1, 1), args)
+    f = kh.GpuModule(kh.code_object("softmax")).get_function(symbol)
+    say(f"{symbol} extreme rows, cols={cols}, block={block}")
+    kh.launch_raw(f, (3, 1, 1), (block, 1, 1), args)
     got = down(dy, 7 * cols).reshape(7, cols)
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.nanmax(np.abs(got - ref)) <= 1e-6
 
 
-@pytest.mark.parametrize("symbol", ["softmax", "softmax_wide", "softmax_block"])
+@pytest.mark.parametrize("symbol", ["softmax", "softmax_wave", "softmax_wide", "softmax_block"])
 @pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
 @pytest.mark.parametrize("block", [64, 256])
 def test_softmax_padded_rows_any_symbol(dev, symbol, cols, block):
