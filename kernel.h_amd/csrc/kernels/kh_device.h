@@ -194,9 +194,18 @@ __device__ __forceinline__ float4 buf_load4(__amdgpu_buffer_rsrc_t r, uint32_t o
   const u32x4_t u = __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0);
   return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
 }
+__device__ __forceinline__ void buf_store4(__amdgpu_buffer_rsrc_t r, uint32_t off, float4 f) {
+  const u32x4_t u = {__float_as_uint(f.x), __float_as_uint(f.y), __float_as_uint(f.z), __float_as_uint(f.w)};
+  __builtin_amdgcn_raw_buffer_store_b128(u, r, off, 0, 0);
+}
 __device__ __forceinline__ void buf_store1(__amdgpu_buffer_rsrc_t r, uint32_t off, float f) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(f), r, off, 0, 0);
 }
+// Whether rows `stride` floats apart from p on start or end inside cache lines.
+__device__ __forceinline__ bool shares_lines(const float *p, int64_t stride) {
+  return (((uint32_t)reinterpret_cast<uintptr_t>(p) & 127) | ((uint32_t)stride & 31)) != 0;
+}
+
 // An offset outside every span_rsrc: loads read 0, stores are dropped.
 constexpr uint32_t kOutside = 0x80000000u;
 

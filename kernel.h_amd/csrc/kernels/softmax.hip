@@ -96,7 +96,14 @@ __device__ __forceinline__ float4 scale4(float4 v, float f) {
 // the one float4 that straddles cols goes out as dwords. Against a wave per
 // row (a wave of 1 KiB of lanes for a 256-byte row): 32768x64 9.1 -> 5.0 us;
 // at 256 columns (32768 rows, 12.5 us, 5.4 TB/s) the two are level.
-template <int V>
+//
+// A row's 256-byte pieces are whole cache lines only where its start and stride
+// are. Where they are not, each store leaves parts of lines that the next one
+// completes, so from three pieces a row on those go through the cache (PARTS);
+// streamed past it they cost the memory system twice: 16384x200 7.3 -> 6.8 us,
+// 300000x200 91 -> 86, 300000x255 147 -> 121 (whole lines through it cost 2-5%,
+// 300000x160 64 -> 67, and rows of two pieces 4%, 300000x100 43.6 -> 45.2).
+template <int V, bool PARTS = false>
 __device__ __forceinline__ void softmax_rows16(const float *__restrict__ X, float *__restrict__ Y, int64_t r0,
                                                int64_t rows, int cols, int64_t xs, int64_t ys, int lane) {
   const int nr = rows - r0 < 4 ? (int)(rows - r0) : 4;
@@ -121,7 +128,10 @@ __device__ __forceinline__ void softmax_rows16(const float *__restrict__ X, floa
     const int col = col0 + 64 * j;
     const uint32_t off = yo + (uint32_t)col * 4u;
     v[j] = scale4(v[j], inv);
-    kh::buf_store4_nt(ry, col + 3 < cols ? off : kh::kOutside, v[j]);
+    if constexpr (PARTS)
+      kh::buf_store4(ry, col + 3 < cols ? off : kh::kOutside, v[j]);
+    else
+      kh::buf_store4_nt(ry, col + 3 < cols ? off : kh::kOutside, v[j]);
     if ((cols & 3) != 0 && cols / 64 == j) {  // uniform: the float4s that hold the rows' last columns
       const bool last = col < cols && col + 3 >= cols;
       kh::buf_store1(ry, last ? off : kh::kOutside, v[j].x);
@@ -304,11 +314,14 @@ __device__ __forceinline__ void softmax_rows(const float *__restrict__ X, float 
   const int64_t w0 = (int64_t)blockIdx.x * waves_per_block + wave;
   const int c = (int)(cols <= KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
   if (S == kNarrow && c <= KH_ROW16_COLS && xs >= cols && ys >= cols && (xs | ys) < (1 << 26)) {
+    const bool parts = rows > KH_ROW16_CACHED_ROWS && kh::shares_lines(Y, ys);
     for (int64_t r = 4 * w0; r < rows; r += 4 * nwaves) {
       if (c <= 64)
         softmax_rows16<1>(X, Y, r, rows, c, xs, ys, lane);
       else if (c <= 128)
         softmax_rows16<2>(X, Y, r, rows, c, xs, ys, lane);
+      else if (parts)
+        softmax_rows16<4, true>(X, Y, r, rows, c, xs, ys, lane);
       else
         softmax_rows16<4>(X, Y, r, rows, c, xs, ys, lane);
     }

@@ -303,6 +303,9 @@ def test_row_plan(name, rows, cols, suffix, grid, threads):
 
 @pytest.mark.parametrize("shape,symbol,grid", [
     ("softmax rows=5,cols=257", "softmax_wave", 2), ("softmax rows=40000,cols=512", "softmax_wave", 10000),
+    ("softmax rows=16385,cols=200", "softmax_wave", 4097), ("softmax rows=16384,cols=200", "softmax", 1024),
+    ("softmax rows=16385,cols=224", "softmax", 1025), ("softmax rows=16385,cols=180", "softmax", 1025),
+    ("softmax rows=16385,cols=256", "softmax", 1025),
     ("layernorm rows=5,cols=257", "layernorm", 2),
 ])
 def test_row_plan_of_one_template(shape, symbol, grid):

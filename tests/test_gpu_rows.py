@@ -338,3 +338,26 @@ def test_row_is_read_whole_before_it_is_written(dev, template, cols):
         dg, db = up(g), up(b)
         kh.layernorm(buf.ptr, dg, db, buf.ptr + 4 * shift, 1, cols)
     assert np.array_equal(down(buf, shift + cols)[shift:], ref.ravel())
+
+
+@pytest.mark.parametrize("template", ["softmax", "layernorm"])
+@pytest.mark.parametrize("rows,cols", [(203, 132), (203, 160), (17000, 196), (17000, 255), (9300, 224), (4097, 252)])
+@pytest.mark.parametrize("odd", [0, 1, 8])
+def test_rows_that_share_cache_lines(dev, template, rows, cols, odd):
+    # Outputs whose rows' starts and ends are parts of cache lines, and whole
+    # ones, from starts of several alignments, with guards on both sides.
+    guard = 64
+    x = O.normal(rows * cols, 0x5AC + cols, 0.0, 4.0)
+    g, b = O.uniform(cols, 0x1A7F, 0.5, 1.5), O.uniform(cols, 0x1A80, -0.1, 0.1)
+    dx, dy = up(x), empty(guard + rows * cols + guard, -7.0)
+    say(f"{template} rows={rows} cols={cols} y {odd} floats past a line")
+    if template == "softmax":
+        kh.softmax(dx, dy.ptr + 4 * odd, rows, cols)
+        ref = O.ref_softmax(x, rows, cols)
+    else:
+        dg, db = up(g), up(b)
+        kh.layernorm(dx, dg, db, dy.ptr + 4 * odd, rows, cols)
+        ref = O.ref_layernorm(x, g, b, rows, cols)
+    out = down(dy, guard + rows * cols + guard)
+    assert np.all(out[:odd] == -7.0) and np.all(out[odd + rows * cols:] == -7.0)
+    assert np.max(np.abs(out[odd:odd + rows * cols].reshape(rows, cols) - ref)) <= 1e-5
