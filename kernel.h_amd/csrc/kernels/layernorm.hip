@@ -11,7 +11,8 @@
 // its width:
 //
 //   cols <= 256            16 lanes, four rows per wavefront (rows16)
-//   cols <= 2048           one wavefront (rows_regs; the wide symbol past 1024)
+//   cols <= 2048           one wavefront (rows_regs; layernorm_wave from 65 to 256
+//                          with few rows, the wide symbol past 1024)
 //   cols <= 65536          one workgroup (row_block)
 //   beyond                 one workgroup, three sweeps (row_stream)
 //
@@ -315,6 +316,23 @@ __device__ __forceinline__ void layernorm_row_serial(const float *__restrict__ x
   for (int64_t c = 0; c < cols; ++c) yr[c] = fmaf((xr[c] - mean) * inv, G[c], B[c]);
 }
 
+// Any width in one wavefront, for launches of layernorm_wave past what its
+// registers hold: three sweeps, a float per lane at a time.
+__device__ __forceinline__ void layernorm_row_wave(const float *__restrict__ xr, const float *__restrict__ G,
+                                                   const float *__restrict__ B, float *__restrict__ yr, int64_t cols,
+                                                   int lane) {
+  float s = 0.0f;
+  for (int64_t c = lane; c < cols; c += kh::kWave) s += xr[c];
+  const float mean = kh::wave_sum(s) / (float)cols;
+  float q = 0.0f;
+  for (int64_t c = lane; c < cols; c += kh::kWave) {
+    const float d = xr[c] - mean;
+    q += d * d;
+  }
+  const float inv = __builtin_amdgcn_rsqf(kh::wave_sum(q) / (float)cols + kEps);
+  for (int64_t c = lane; c < cols; c += kh::kWave) yr[c] = fmaf((xr[c] - mean) * inv, G[c], B[c]);
+}
+
 // Which register paths a symbol compiles in: the kernel's register
 // allocation is that of its widest path. Gs and Bs hold kStageCols floats
 // each in the narrow symbol and are unused (null) in the others.
@@ -387,6 +405,34 @@ layernorm(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1
   __shared__ __attribute__((aligned(16))) float Gs[kStageCols];
   __shared__ __attribute__((aligned(16))) float Bs[kStageCols];
   KH_LAYERNORM_BODY(kNarrow, Gs, Bs);
+}
+
+// Same arguments and results for rows of 65..256 floats in launches of few rows
+// (KH_LAYERNORM_WAVE_ROWS): a wave per row and nothing else. One more choice in
+// the reference symbol cost its other rows 0.1 us.
+extern "C" __global__ void __launch_bounds__(256)
+layernorm_wave(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
+               KH_MEMREF2(float, y)) {
+  __shared__ __attribute__((aligned(16))) float Gs[4 * kh::kWave];
+  __shared__ __attribute__((aligned(16))) float Bs[4 * kh::kWave];
+  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();
+  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, gamma_base, gamma_off, beta_base, beta_off, y_base, y_off, y_s0,
+                gw, nb);
+  const float *__restrict__ X = KH_PTR(x), *__restrict__ G = KH_PTR(gamma), *__restrict__ B = KH_PTR(beta);
+  float *__restrict__ Y = KH_PTR(y);
+  const int bd = (int)kh::threads_x_of(gw);
+  const int64_t rows = x_n0, cols = x_n1;
+  if (bd % kh::kWave != 0) {
+    for (int64_t r = (int64_t)blockIdx.x * bd + threadIdx.x; r < rows; r += (int64_t)bd * nb)
+      layernorm_row_serial(X + r * x_s0, G, B, Y + r * y_s0, cols);
+    return;
+  }
+  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int64_t r0 = (int64_t)blockIdx.x * (bd / kh::kWave) + wave, rstep = (int64_t)(bd / kh::kWave) * nb;
+  if (cols <= 4 * kh::kWave)
+    layernorm_rows_regs<1, true>(X, G, B, Y, rows, (int)cols, x_s0, y_s0, r0, rstep, bd, lane, Gs, Bs);
+  else
+    for (int64_t r = r0; r < rows; r += rstep) layernorm_row_wave(X + r * x_s0, G, B, Y + r * y_s0, cols, lane);
 }
 
 // Same arguments and results for rows of 1025..4096 floats (the launcher

@@ -9,8 +9,8 @@
 // traffic per element. What holds a row depends on its width:
 //
 //   cols <= 256            16 lanes, four rows per wavefront (rows16)
-//   cols <= 2048           one wavefront (row_regs; softmax_wave up to 512, the
-//                          wide symbol past 1024)
+//   cols <= 2048           one wavefront (row_regs; softmax_wave up to 512 and,
+//                          with few rows, from 65; the wide symbol past 1024)
 //   cols <= 65536          one workgroup (row_block)
 //   beyond                 one workgroup in two sweeps (row_stream)
 //
@@ -371,8 +371,9 @@ softmax(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
   KH_SOFTMAX_BODY(kNarrow);
 }
 
-// Same arguments and results for rows of 257..512 floats: a wave per row and
-// nothing else, without LDS. The path is `softmax`'s, instruction for
+// Same arguments and results for rows of 257..512 floats, and for narrower ones
+// where row_plan says (khrt_templates.cpp): a wave per row and nothing else,
+// without LDS. The path is `softmax`'s, instruction for
 // instruction, but as one of that symbol's many it took 2-9% longer: 9300x272
 // 6.25 -> 5.80 us, 40000x272 16.9 -> 15.8, 16384x300 9.0 -> 8.6, 16384x512 13.2 ->
 // 12.8; at 700 and 1024 columns it is 1% slower (40000x1024 53.6 -> 54.3), which is

@@ -416,13 +416,22 @@ struct RowPlan {
 RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   const char *narrow = softmax ? "softmax" : "layernorm", *wide = softmax ? "softmax_wide" : "layernorm_wide",
              *block = softmax ? "softmax_block" : "layernorm_block";
+  // Too few rows for four to a wave.
+  const bool few = rows <= (softmax ? KH_SOFTMAX_WAVE_ROWS(cols) : KH_LAYERNORM_WAVE_ROWS(cols));
   // Many rows of 193..255 floats whose ends share cache lines: a wave's four rows
   // leave more parts of lines than it pays in one (softmax 40000x200 14.6 us,
   // 14.1 through the cache, 13.3 in a wave each; 300000x252 118, 107, 99; with
   // 16384 rows and fewer 2-7% the other way).
-  if (softmax && cols > 192 && cols < KH_ROW16_COLS && cols % 32 != 0 && rows > 16384) return {"softmax_wave", 256, 4};
-  if (cols <= KH_ROW16_COLS) return {narrow, 256, 16};
+  const bool many_parts = softmax && cols > 192 && cols % 32 != 0 && rows > 16384;
+  if (cols <= KH_ROW16_COLS && !few && !many_parts) {
+    // Between two and three workgroups of 16 rows per CU the last ones leave CUs
+    // idle for longer than half as large ones do (layernorm 8500x256 5.2 vs 4.6 us,
+    // 9300x224 5.5 vs 4.7, 12000x256 5.9 vs 5.5; past three within 4% either way).
+    if (!softmax && cols > 128 && rows > 2 * 16 * KH_GEMM_CUS && rows < 3 * 16 * KH_GEMM_CUS) return {narrow, 128, 8};
+    return {narrow, 256, 16};
+  }
   if (softmax && cols <= 512) return {"softmax_wave", 256, 4};
+  if (cols <= KH_ROW16_COLS) return {"layernorm_wave", 256, 4};
   if (cols <= 1024) return {narrow, 256, 4};
   if (cols <= 2048) return {wide, 256, 4};
   if (cols > KH_ROW_BLOCK_MAX) return {block, 1024, 1};

@@ -72,7 +72,8 @@ def test_softmax_reference_geometry(dev):
     assert np.max(np.abs(down(dy, rows * cols).reshape(rows, cols) - O.ref_softmax(x, rows, cols))) <= 1e-4
 
 
-@pytest.mark.parametrize("symbol", ["softmax", "softmax_wave", "softmax_wide", "layernorm", "layernorm_wide"])
+@pytest.mark.parametrize("symbol", ["softmax", "softmax_wave", "softmax_wide", "layernorm", "layernorm_wave",
+                                    "layernorm_wide"])
 @pytest.mark.parametrize("cols", [64, 256, 512, 1000, 1024, 2048, 4096, 5000])
 def test_every_row_symbol_at_every_width(dev, symbol, cols):
     # Each symbol of a template computes the same result at every width (the
@@ -298,7 +299,7 @@ def test_layernorm_path_edges(dev, cols):
     assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-5
 
 
-@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wide", "layernorm_block"])
+@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wave", "layernorm_wide", "layernorm_block"])
 @pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
 @pytest.mark.parametrize("block", [64, 256])
 def test_layernorm_padded_rows_any_symbol(dev, symbol, cols, block):
