@@ -15,11 +15,12 @@
 // few to fill the chip four at a time, and a row in 16 lanes takes its two or
 // four loads and their share of the reductions one after another. Four rows to a
 // wave against one: softmax 1000x100 2.72 vs 2.62 us, 1000x252 3.0 vs 2.7, 2500x252
-// 3.3 vs 3.2, 4096x252 3.6 vs 3.6, 4096x160 3.2 vs 3.4; layernorm 1000x100 2.9 vs 2.7,
-// 2500x100 level, 4096x200 3.8 vs 3.4, 8192x200 4.7 vs 4.1, 8500x200 5.0 vs 5.1 (a round
-// of the chip is 8192 waves). Rows of one float4 per lane (up to 64) are level.
+// 3.3 vs 3.2, 4096x252 3.6 vs 3.6, 4096x160 3.2 vs 3.4; layernorm 1000x100 2.94 vs 2.72,
+// 2500x100 level, 6144x200 4.32 vs 3.76, 6144x160 3.78 vs 3.64. Between there and 8192
+// rows it depends on the width (6500x252 4.61 vs 4.08, 8192x160 3.90 vs 4.00, 8192x224
+// 4.16 vs 4.27). Rows of one float4 per lane (up to 64) are level.
 #define KH_SOFTMAX_WAVE_ROWS(cols) ((cols) <= 64 ? 0 : (cols) <= 128 ? 1024 : 2048)
-#define KH_LAYERNORM_WAVE_ROWS(cols) ((cols) <= 64 ? 0 : (cols) <= 128 ? 1024 : 8192)
+#define KH_LAYERNORM_WAVE_ROWS(cols) ((cols) <= 64 ? 0 : (cols) <= 128 ? 1024 : 6144)
 // Launches of more rows than this send stores of parts of cache lines through
 // the cache (softmax.hip); with fewer there is nothing to merge them with in
 // time (softmax 4096x240 3.35 us streamed, 3.7 cached; 9300x240 5.3 and 5.0).

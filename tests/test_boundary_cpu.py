@@ -287,7 +287,7 @@ def test_launcher_geometry(name, shape, grid, block):
 
 @pytest.mark.parametrize("name", ["softmax", "layernorm"])
 @pytest.mark.parametrize("rows,cols,suffix,grid,threads", [
-    (5, 64, "", 1, 256), (12288, 256, "", 768, 256), (1025, 65, "", 65, 256), (5, 513, "", 2, 256), (5, 1024, "", 2, 256), (5, 1025, "_wide", 2, 256), (5, 2048, "_wide", 2, 256),
+    (5, 64, "", 1, 256), (6145, 256, "", 385, 256), (1025, 65, "", 65, 256), (5, 513, "", 2, 256), (5, 1024, "", 2, 256), (5, 1025, "_wide", 2, 256), (5, 2048, "_wide", 2, 256),
     (5, 2049, "_wide", 5, 192), (5, 4096, "_wide", 5, 256),
     # 4, 8 and 16 float4 per thread, at most 768 threads; up to a CU for every row 8 to 1024.
     (5, 4097, "", 5, 320), (5, 12288, "", 5, 768), (5, 12289, "", 5, 448), (5, 24576, "", 5, 768),
@@ -310,7 +310,7 @@ def test_row_plan(name, rows, cols, suffix, grid, threads):
     ("softmax rows=1024,cols=65", "softmax_wave", 256), ("softmax rows=1025,cols=128", "softmax", 65),
     ("softmax rows=2048,cols=129", "softmax_wave", 512), ("softmax rows=2049,cols=256", "softmax", 129),
     ("layernorm rows=1024,cols=65", "layernorm_wave", 256), ("layernorm rows=1025,cols=128", "layernorm", 65),
-    ("layernorm rows=8192,cols=129", "layernorm_wave", 2048),
+    ("layernorm rows=6144,cols=129", "layernorm_wave", 1536), ("layernorm rows=6145,cols=256", "layernorm", 385),
     ("layernorm rows=5,cols=257", "layernorm", 2),
 ])
 def test_row_plan_of_one_template(shape, symbol, grid):
@@ -320,7 +320,7 @@ def test_row_plan_of_one_template(shape, symbol, grid):
 
 
 @pytest.mark.parametrize("rows,cols,grid,threads", [
-    (8193, 129, 1025, 128), (12287, 256, 1536, 128), (12288, 256, 768, 256),
+    (8192, 129, 512, 256), (8193, 129, 1025, 128), (12287, 256, 1536, 128), (12288, 256, 768, 256),
     (8193, 128, 513, 256),
 ])
 def test_layernorm_plan_between_rounds(rows, cols, grid, threads):
