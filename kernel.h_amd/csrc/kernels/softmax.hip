@@ -413,7 +413,8 @@ softmax_wide(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
 }
 
 // Same arguments and results; one workgroup per row with 16 float4 per
-// thread, for rows past what the reference symbol's eight hold.
+// thread, for rows past what the reference symbol's eight hold, and of a single
+// wave for 2049..4096 floats where row_plan says.
 extern "C" __global__ void __launch_bounds__(1024)
 softmax_block(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
   KH_SOFTMAX_BODY(kBlock);

@@ -435,6 +435,15 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   if (cols <= 1024) return {narrow, 256, 4};
   if (cols <= 2048) return {wide, 256, 4};
   if (cols > KH_ROW_BLOCK_MAX) return {block, 1024, 1};
+  // softmax of 2049..4096 floats in up to ten rows per CU, once there is enough to
+  // move: a wave per row (16 float4 per lane) holds the chip's rows all at once
+  // and crosses no barriers; in workgroups of 192 or 256 threads their bursts of
+  // loads meet. Workgroup against wave: 1700x2560 8.0 vs 7.1 us, 2048x3328 11.4 vs
+  // 9.2, 2048x4096 13.4 vs 11.3, 2560x2304 10.4 vs 9.2, and the other way 1100x2052
+  // 5.3 vs 5.9, 1500x2560 6.4 vs 6.7, 1200x2816 6.0 vs 6.1, 3000x4096 18.2 vs 18.7,
+  // 8192x2560 28.5 vs 30.5.
+  if (softmax && cols <= 4096 && rows <= 10 * KH_GEMM_CUS && (rows * cols >= 15 << 18 || 2 * rows >= 13 * KH_GEMM_CUS))
+    return {block, 64, 1};
   // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
   // per thread: the fewest that need at most 768 threads, so that a CU's 2048
   // hold two workgroups and one's loads fill the other's reductions and

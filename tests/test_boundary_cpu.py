@@ -319,6 +319,19 @@ def test_row_plan_of_one_template(shape, symbol, grid):
     assert kh.geometry(name, shape) == ((grid, 1, 1), (256, 1, 1))
 
 
+@pytest.mark.parametrize("rows,cols,symbol,grid,threads", [
+    (1664, 2049, "softmax_block", 1664, 64), (1663, 2049, "softmax_wide", 1663, 192),
+    (960, 4096, "softmax_block", 960, 64), (959, 4096, "softmax_wide", 959, 256),
+    (2560, 4096, "softmax_block", 2560, 64), (2561, 4096, "softmax_wide", 2561, 256),
+    (2560, 2048, "softmax_wide", 640, 256), (2560, 4097, "softmax", 2560, 320),
+])
+def test_softmax_wave_of_sixteen_float4(rows, cols, symbol, grid, threads):
+    # 2049..4096 columns in up to ten rows per CU: a wave each once there are enough floats, or rows.
+    shape = f"rows={rows},cols={cols}"
+    assert kh.launch_symbol("softmax", shape) == symbol
+    assert kh.geometry("softmax", shape) == ((grid, 1, 1), (threads, 1, 1))
+
+
 @pytest.mark.parametrize("rows,cols,grid,threads", [
     (8192, 129, 512, 256), (8193, 129, 1025, 128), (12287, 256, 1536, 128), (12288, 256, 768, 256),
     (8193, 128, 513, 256),

@@ -216,6 +216,22 @@ def test_softmax_path_edges(dev, cols):
     assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-6 * np.max(ref)
 
 
+@pytest.mark.parametrize("rows,cols", [(1664, 2049), (1000, 4095), (2560, 2051), (970, 4096), (257, 24577), (300, 32001)])
+def test_softmax_path_of_many_rows(dev, rows, cols):
+    # Launches whose symbol depends on the number of rows too: odd addresses, a
+    # guard, and the tolerance as above.
+    guard = 64
+    x = O.normal(rows * cols, 0x50F8 + cols, 0.0, 4.0)
+    ref = O.ref_softmax(x, rows, cols)
+    dx, dy = up(np.concatenate([np.full(1, np.nan, np.float32), x])), empty(rows * cols + guard, -7.0)
+    say(f"softmax rows={rows} cols={cols}")
+    assert kh.launch_symbol("softmax", f"rows={rows},cols={cols}") == "softmax_block"
+    kh.softmax(dx.ptr + 4, dy, rows, cols)
+    out = down(dy, rows * cols + guard)
+    assert np.all(out[rows * cols:] == -7.0)
+    assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-6 * np.max(ref)
+
+
 @pytest.mark.parametrize("cols", [40, 200, 300, 700, 1500, 3001, 5000, 20001, 40001, 70001])
 def test_softmax_extreme_rows(dev, cols):
     # Rows of the type's lowest value, of one large value, half masked with
