@@ -12,7 +12,9 @@
 //
 //   cols <= 256            16 lanes, four rows per wavefront (rows16)
 //   cols <= 2048           one wavefront (rows_regs; layernorm_wave from 65 to 256
-//                          with few rows, the wide symbol past 1024)
+//                          with few rows, the wide symbol past 1024), and many
+//                          rows of 2689..4095 that share cache lines
+//                          (layernorm_wide_parts)
 //   cols <= 65536          one workgroup (row_block)
 //   beyond                 one workgroup, three sweeps (row_stream)
 //
@@ -407,32 +409,57 @@ layernorm(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1
   KH_LAYERNORM_BODY(kNarrow, Gs, Bs);
 }
 
+namespace {
+
+// Rows of up to 4 V floats per lane in a wave each, and nothing else.
+template <int V, bool STAGED>
+__device__ __forceinline__ void layernorm_waves(const float *__restrict__ X, const float *__restrict__ G,
+                                                const float *__restrict__ B, float *__restrict__ Y, int64_t rows,
+                                                int64_t cols, int64_t xs, int64_t ys, int bd, int64_t nb, float *Gs,
+                                                float *Bs) {
+  if (bd % kh::kWave != 0) {
+    for (int64_t r = (int64_t)blockIdx.x * bd + threadIdx.x; r < rows; r += bd * nb)
+      layernorm_row_serial(X + r * xs, G, B, Y + r * ys, cols);
+    return;
+  }
+  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  const int64_t r0 = (int64_t)blockIdx.x * (bd / kh::kWave) + wave, rstep = (bd / kh::kWave) * nb;
+  if (cols <= 4 * V * kh::kWave)
+    layernorm_rows_regs<V, STAGED>(X, G, B, Y, rows, (int)cols, xs, ys, r0, rstep, bd, lane, Gs, Bs);
+  else
+    for (int64_t r = r0; r < rows; r += rstep) layernorm_row_wave(X + r * xs, G, B, Y + r * ys, cols, lane);
+}
+
+}  // namespace
+
+#define KH_LAYERNORM_WAVES(V, STAGED, GS, BS)                                                                  \
+  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();                                         \
+  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, gamma_base, gamma_off, beta_base, beta_off, y_base, y_off,    \
+                y_s0, gw, nb);                                                                                 \
+  layernorm_waves<V, STAGED>(KH_PTR(x), KH_PTR(gamma), KH_PTR(beta), KH_PTR(y), x_n0, x_n1, x_s0, y_s0,        \
+                             (int)kh::threads_x_of(gw), nb, GS, BS)
+
 // Same arguments and results for rows of 65..256 floats in launches of few rows
-// (KH_LAYERNORM_WAVE_ROWS): a wave per row and nothing else. One more choice in
-// the reference symbol cost its other rows 0.1 us.
+// (KH_LAYERNORM_WAVE_ROWS): a wave per row. One more choice in the reference
+// symbol cost its other rows 0.1 us.
 extern "C" __global__ void __launch_bounds__(256)
 layernorm_wave(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
                KH_MEMREF2(float, y)) {
   __shared__ __attribute__((aligned(16))) float Gs[4 * kh::kWave];
   __shared__ __attribute__((aligned(16))) float Bs[4 * kh::kWave];
-  const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();
-  KH_ARGS_READY(x_base, x_off, x_n0, x_n1, x_s0, gamma_base, gamma_off, beta_base, beta_off, y_base, y_off, y_s0,
-                gw, nb);
-  const float *__restrict__ X = KH_PTR(x), *__restrict__ G = KH_PTR(gamma), *__restrict__ B = KH_PTR(beta);
-  float *__restrict__ Y = KH_PTR(y);
-  const int bd = (int)kh::threads_x_of(gw);
-  const int64_t rows = x_n0, cols = x_n1;
-  if (bd % kh::kWave != 0) {
-    for (int64_t r = (int64_t)blockIdx.x * bd + threadIdx.x; r < rows; r += (int64_t)bd * nb)
-      layernorm_row_serial(X + r * x_s0, G, B, Y + r * y_s0, cols);
-    return;
-  }
-  const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
-  const int64_t r0 = (int64_t)blockIdx.x * (bd / kh::kWave) + wave, rstep = (int64_t)(bd / kh::kWave) * nb;
-  if (cols <= 4 * kh::kWave)
-    layernorm_rows_regs<1, true>(X, G, B, Y, rows, (int)cols, x_s0, y_s0, r0, rstep, bd, lane, Gs, Bs);
-  else
-    for (int64_t r = r0; r < rows; r += rstep) layernorm_row_wave(X + r * x_s0, G, B, Y + r * y_s0, cols, lane);
+  KH_LAYERNORM_WAVES(1, true, Gs, Bs);
+}
+
+// Same arguments and results for many rows of 2689..4095 floats that share cache
+// lines (row_plan, khrt_templates.cpp): a wave per row, held to two on a SIMD by
+// the registers it is given. Bound by memory, and here the fewer rows a CU has in
+// flight the better: 40000x3000 177 us in workgroups at eight rows a CU
+// (layernorm_wide), 168 at five, 191 in waves at twenty, 163 in waves at eight.
+// At 40000x3072, whole lines, the same four take 161, 158, 179 and 160.
+extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+layernorm_wide_parts(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
+                     KH_MEMREF2(float, y)) {
+  KH_LAYERNORM_WAVES(16, false, nullptr, nullptr);
 }
 
 // Same arguments and results for rows of 1025..4096 floats (the launcher

@@ -312,11 +312,18 @@ def test_row_plan(name, rows, cols, suffix, grid, threads):
     ("layernorm rows=1024,cols=65", "layernorm_wave", 256), ("layernorm rows=1025,cols=128", "layernorm", 65),
     ("layernorm rows=6144,cols=129", "layernorm_wave", 1536), ("layernorm rows=6145,cols=256", "layernorm", 385),
     ("layernorm rows=5,cols=257", "layernorm", 2),
+    # Many wide rows that share cache lines.
+    ("layernorm rows=12289,cols=2689", "layernorm_wide_parts", 3073), ("layernorm rows=40000,cols=4095", "layernorm_wide_parts", 10000),
 ])
 def test_row_plan_of_one_template(shape, symbol, grid):
     name, shape = shape.split(" ")
     assert kh.launch_symbol(name, shape) == symbol
     assert kh.geometry(name, shape) == ((grid, 1, 1), (256, 1, 1))
+
+
+@pytest.mark.parametrize("rows,cols", [(12288, 2689), (12289, 2687), (12289, 2720), (40000, 4096)])
+def test_layernorm_wide_parts_lines(rows, cols):
+    assert kh.launch_symbol("layernorm", f"rows={rows},cols={cols}") == "layernorm_wide"
 
 
 @pytest.mark.parametrize("rows,cols,symbol,grid,threads", [

@@ -73,7 +73,7 @@ def test_softmax_reference_geometry(dev):
 
 
 @pytest.mark.parametrize("symbol", ["softmax", "softmax_wave", "softmax_wide", "layernorm", "layernorm_wave",
-                                    "layernorm_wide"])
+                                    "layernorm_wide", "layernorm_wide_parts"])
 @pytest.mark.parametrize("cols", [64, 256, 512, 1000, 1024, 2048, 4096, 5000])
 def test_every_row_symbol_at_every_width(dev, symbol, cols):
     # Each symbol of a template computes the same result at every width (the
@@ -315,7 +315,47 @@ def test_layernorm_path_edges(dev, cols):
     assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-5
 
 
-@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wave", "layernorm_wide", "layernorm_block"])
+@pytest.mark.parametrize("rows,cols,symbol", [(12289, 2689, "layernorm_wide_parts"), (12290, 4095, "layernorm_wide_parts"),
+                                              (300, 24579, "layernorm_block"), (8200, 131, "layernorm"),
+                                              (6001, 254, "layernorm_wave")])
+def test_layernorm_path_of_many_rows(dev, rows, cols, symbol):
+    # Launches whose symbol depends on the number of rows too: every operand at an
+    # odd address, a guard, and the tolerance as above.
+    guard = 64
+    x = O.normal(rows * cols, 0x1A81 + cols, 3.0, 4.0)
+    g, b = O.uniform(cols, 0x1A7F, 0.5, 1.5), O.uniform(cols, 0x1A80, -0.1, 0.1)
+    ref = O.ref_layernorm(x, g, b, rows, cols)
+    nan = np.full(1, np.nan, np.float32)
+    dx, dg, db = (up(np.concatenate([nan, t, nan])) for t in (x, g, b))
+    dy = empty(rows * cols + guard, -7.0)
+    say(f"layernorm rows={rows} cols={cols}")
+    assert kh.launch_symbol("layernorm", f"rows={rows},cols={cols}") == symbol
+    kh.layernorm(dx.ptr + 4, dg.ptr + 4, db.ptr + 4, dy, rows, cols)
+    out = down(dy, rows * cols + guard)
+    assert np.all(out[rows * cols:] == -7.0)
+    assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-5
+
+
+@pytest.mark.parametrize("cols", [40, 100, 200, 300, 700, 1500, 3001, 5000, 20001, 40001, 70001])
+def test_layernorm_infinities_and_nan(dev, cols):
+    # A row with an infinity or NaN has no finite mean: all NaN, as in 64 bits,
+    # and the rows beside it (four to a wave, one or a workgroup) are untouched.
+    rows = 9
+    x = O.normal(rows * cols, 0x1A82, 3.0, 4.0).reshape(rows, cols)
+    x[1, 0], x[3, cols - 1], x[4, cols // 2], x[6, 5:9] = np.inf, np.nan, -np.inf, [np.inf, -np.inf, np.inf, np.nan]
+    g, b = O.uniform(cols, 0x1A7F, 0.5, 1.5), O.uniform(cols, 0x1A80, -0.1, 0.1)
+    dx, dg, db, dy = up(x.ravel()), up(g), up(b), empty(rows * cols)
+    say(f"layernorm infinities and NaN, cols={cols}")
+    kh.layernorm(dx, dg, db, dy, rows, cols)
+    got = down(dy, rows * cols).reshape(rows, cols)
+    bad = [1, 3, 4, 6]
+    ok = [r for r in range(rows) if r not in bad]
+    assert np.all(np.isnan(got[bad]))
+    assert np.max(np.abs(got[ok] - O.ref_layernorm(x[ok].ravel(), g, b, len(ok), cols))) <= 1e-5
+
+
+@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wave", "layernorm_wide", "layernorm_wide_parts",
+                                    "layernorm_block"])
 @pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
 @pytest.mark.parametrize("block", [64, 256])
 def test_layernorm_padded_rows_any_symbol(dev, symbol, cols, block):
