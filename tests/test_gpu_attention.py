@@ -278,3 +278,35 @@ def test_attention_split_refuses(dev, symbol, bad):
     kh.launch_raw(f, (2, h, b), (256, 1, 1), args)
     out = down(bufs[3], n + guard)
     assert np.all(np.isnan(out[:n])) and np.all(out[n:] == 1.0)
+
+
+@pytest.mark.parametrize("symbol,rows", [("attention", 128), ("attention_split", 32), ("attention_split16", 16)])
+@pytest.mark.parametrize("s", [1, 100, 300])
+def test_attention_infinities_and_nan(dev, symbol, rows, s):
+    """Infinities and NaN among valid keys reach the outputs that 64 bits say
+    they reach and no other, and nothing past O is written. A slice each: none;
+    one V element NaN; one infinite; one K element NaN; one -inf (a key of
+    weight 0 for queries on its one side, NaN for the others); one query row
+    NaN, and one infinite. The tolerance of finite elements is that of
+    test_attention_split_launches."""
+    b, h, guard = 2, 3, 256
+    n, t = b * h * s * D, s - 1 - s // 3
+    Q, K, V = (O.normal(n, 61 + i, 0.0, 1.0).reshape(b * h, s, D) for i in range(3))
+    V[1, t, 5], V[2, t, 63], K[3, t, 17], K[4, t, 0], Q[5, t, 9], Q[5, 0, 1] = (np.nan, np.inf, np.nan, -np.inf, np.nan,
+                                                                              np.inf)
+    dq, dk, dv, do = up(Q.ravel()), up(K.ravel()), up(V.ravel()), empty(n + guard, -7.0)
+    args = kh.LaunchArgs()
+    for x in (dq, dk, dv, do):
+        args.add_memref(x, [b, h, s, D])
+    f = kh.GpuModule(kh.code_object("attention")).get_function(symbol)
+    say(f"{symbol} infinities and NaN s={s}")
+    kh.kernel_launch(f, ((s + rows - 1) // rows, h, b), (256, 1, 1), args)
+    out = down(do, n + guard)
+    assert np.all(out[n:] == -7.0)
+    got = out[:n].reshape(-1, D)
+    bh, qi = _rows(b, h, s, None, 0)
+    ref = O.ref_attention_rows(Q.ravel(), K.ravel(), V.ravel(), s, D, bh, qi)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and not np.any(np.isneginf(got))
+    fin = np.isfinite(ref)
+    assert np.max(np.abs(got[fin] - ref[fin])) <= 1e-5
