@@ -135,7 +135,7 @@ gemm_mid(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(floa
 
 // Same arguments and results with 64x64 tiles on eight waves (4 x 2, each
 // 16x32 as 1x2 blocks of v_mfma_f32_16x16x4f32), 32-deep slabs through
-// `gemm`'s persistent direct-to-LDS ring; 49.5 KB of LDS and 86 VGPRs, so
+// `gemm`'s persistent direct-to-LDS ring; 49.5 KB of LDS and 83 VGPRs, so
 // two workgroups per CU. Kernel trace, interleaved launches, same bits,
 // against the 64x64 tiles it replaced (four waves, register-staged
 // slabs; and `gemm_small_pf2` where that was the launcher's choice):

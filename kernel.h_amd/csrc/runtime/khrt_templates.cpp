@@ -444,21 +444,22 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   // 8192x2560 28.5 vs 30.5.
   if (softmax && cols <= 4096 && rows <= 10 * KH_GEMM_CUS && (rows * cols >= 15 << 18 || 2 * rows >= 13 * KH_GEMM_CUS))
     return {block, 64, 1};
-  // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
-  // per thread: the fewest that need at most 768 threads, so that a CU's 2048
-  // hold two workgroups and one's loads fill the other's reductions and
-  // stores. Rotated launches, softmax / layernorm: 300x13000 9.5 / 10.5 us at
-  // 832 threads, 7.0 / 7.6 at 448; 1024x16000 26.7 / 28.5 at 1024, 23.6 / 25.6
-  // at 512; 512x32001 27.7 / 28.7 at 1024, 24.7 / 25.7 at 512. At 768 and
-  // below the two splits are within 4% (2000x10000, 4000x12000). With a CU for
-  // every row there is no second workgroup, and 16 float4 gain nothing over 8
-  // (256x32001: 14.2 us at 1024 threads, 14.4 at 512).
   // layernorm of many rows that share cache lines keeps fewer of them in flight
   // (layernorm_wide_parts): 40000x2800 157.6 vs 150.4 us, 40000x3000 177.9 vs 163.1,
   // 40000x3676 209 vs 194, 16384x3792 87.9 vs 84.0; 8192x3000 37.0 vs 37.1, 12300x2564
   // 46.3 vs 47.2, and rows of whole lines 16384x3072 67.8 vs 68.5.
   if (!softmax && cols > 2688 && cols <= 4096 && cols % 32 != 0 && rows > 48 * KH_GEMM_CUS)
     return {"layernorm_wide_parts", 256, 4};
+  // A workgroup per row, as few whole waves as hold it at 4, 8 or 16 float4
+  // per thread: the fewest that need at most 768 threads. At 4 and 8 (at most 64
+  // registers) a CU then holds two workgroups or more, and one's loads fill the
+  // other's reductions and stores; at 16 (96 and 94 registers, 20 waves on a CU)
+  // two up to 640 threads, 40960 columns. Rotated launches, softmax / layernorm:
+  // 300x13000 9.5 / 10.5 us at 832 threads, 7.0 / 7.6 at 448; 1024x16000 26.7 / 28.5
+  // at 1024, 23.6 / 25.6 at 512; 512x32001 27.7 / 28.7 at 1024, 24.7 / 25.7 at 512. At
+  // 768 and below the two splits are within 4% (2000x10000, 4000x12000). With a CU
+  // for every row there is no second workgroup, and 16 float4 gain nothing over 8
+  // (256x32001: 14.2 us at 1024 threads, 14.4 at 512).
   auto threads = [&](int v) { return static_cast<unsigned>(64 * ceil_div(ceil_div(cols, 4), 64 * v)); };
   if (cols <= 4096) return {wide, threads(4), 1};
   if (threads(4) <= 768) return {narrow, threads(4), 1};

@@ -535,9 +535,9 @@ def _direct(name: str):
     """A second prototype of a template's entry point that takes its device
     pointers as integers: ctypes converts an int, or a handle through its
     `_as_parameter_`, and refuses anything else (a c_void_p would take bytes
-    and host arrays). With the launcher's kept functions this took vecadd of
-    4099 elements from 4.49 to 4.03 us a call, nearly all of it now in the HIP
-    runtime (ctypes alone 0.3 us; _ptr on every argument was another 0.3).
+    and host arrays). Against _ptr on every argument a call takes 0.24 us less
+    (vecadd of 4099 elements 3.10 against 3.34 us in one process, turn about;
+    the prototype alone 3.04); the rest is the entry point and the HIP runtime.
     What is refused here (None for an optional buffer, other integer types) goes
     through _ptr."""
     fn = lib[name]
