@@ -233,8 +233,8 @@ KHRT_API int khrt_template_geometry(const char *name, const char *shape, khrt_di
  * the template name itself or a variant in the same code object with the
  * same arguments and results (gemm_small, gemm_wide, gemm_ksplit*,
  * softmax_wave, softmax_wide, softmax_block, layernorm_wave, layernorm_wide,
- * layernorm_wide_parts, layernorm_block, attention_split, attention_split16). Writes a NUL-terminated name of at most cap
- * bytes. No reference counterpart: the reference compiles one symbol per
+ * layernorm_wide_many, layernorm_wide_parts, layernorm_block, attention_split,
+ * attention_split16). Writes a NUL-terminated name of at most cap bytes. No reference counterpart: the reference compiles one symbol per
  * template and shape (emitter.cpp:733-736); callers that report resources
  * for a launch (kernelh compile --resources) need the symbol it runs. */
 KHRT_API int khrt_template_launch_symbol(const char *name, const char *shape, char *out, size_t cap);

@@ -12,7 +12,7 @@
 //
 //   cols <= 256            16 lanes, four rows per wavefront (rows16)
 //   cols <= 2048           one wavefront (rows_regs; layernorm_wave from 65 to 256
-//                          with few rows, the wide symbol past 1024), and many
+//                          with few rows, the wide symbols past 1024), and many
 //                          rows of 2689..4095 that share cache lines
 //                          (layernorm_wide_parts)
 //   cols <= 65536          one workgroup (row_block)
@@ -147,8 +147,9 @@ __device__ __forceinline__ void layernorm_rows16(const float *__restrict__ X, co
 // more float4 per lane, the loads go out in two halves, the second once the
 // first has landed (kh::kFirstBurst). Without STAGED, gamma and beta are read
 // the same way; with it, from LDS (a lane past cols reads a staged slot it
-// does not use: every path that stages has 4 V float4 <= kStageCols).
-template <int V, bool STAGED>
+// does not use: every path that stages has 4 V float4 <= kStageCols). With AHEAD
+// they are read beside the row instead of after its reductions.
+template <int V, bool STAGED, bool AHEAD = false>
 __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X, const float *__restrict__ G,
                                                     const float *__restrict__ B, float *__restrict__ Y,
                                                     int64_t rows, int cols, int64_t xs, int64_t ys,
@@ -180,9 +181,17 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
     stage_affine(G, B, cols, bd, Gs, Bs);
   }
   const __amdgpu_buffer_rsrc_t rg = kh::span_rsrc(G, row_bytes), rb = kh::span_rsrc(B, row_bytes);
+  float4 ga[AHEAD ? V : 1], ba[AHEAD ? V : 1];
   for (int64_t r = r0; r < rows; r += rstep) {
     const __amdgpu_buffer_rsrc_t ry = kh::span_rsrc(Y + r * ys, row_bytes);
     if (!STAGED || r != r0) load_row(r, std::false_type{});
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        ga[j] = kh::buf_load4(rg, (uint32_t)(lane + j * kh::kWave) * 16u);
+        ba[j] = kh::buf_load4(rb, (uint32_t)(lane + j * kh::kWave) * 16u);
+      }
+    }
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < V; ++j) s += sum4(v[j]);
@@ -202,6 +211,9 @@ __device__ __forceinline__ void layernorm_rows_regs(const float *__restrict__ X,
       if constexpr (STAGED) {
         g = *reinterpret_cast<const float4 *>(Gs + c);
         b = *reinterpret_cast<const float4 *>(Bs + c);
+      } else if constexpr (AHEAD) {
+        g = ga[j];
+        b = ba[j];
       } else {
         g = kh::buf_load4(rg, 4u * c);
         b = kh::buf_load4(rb, 4u * c);
@@ -338,7 +350,7 @@ __device__ __forceinline__ void layernorm_row_wave(const float *__restrict__ xr,
 // Which register paths a symbol compiles in: the kernel's register
 // allocation is that of its widest path. Gs and Bs hold kStageCols floats
 // each in the narrow symbol and are unused (null) in the others.
-enum Symbol { kNarrow, kWide, kBlock };
+enum Symbol { kNarrow, kWide, kMany, kBlock };
 
 template <Symbol S>
 __device__ __forceinline__ void layernorm_all(const float *__restrict__ X, const float *__restrict__ G,
@@ -371,8 +383,8 @@ __device__ __forceinline__ void layernorm_all(const float *__restrict__ X, const
     layernorm_rows_regs<2, true>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, Gs, Bs);
   } else if (S == kNarrow && c <= 1024) {
     layernorm_rows_regs<4, true>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, Gs, Bs);
-  } else if (S == kWide && c <= 2048) {
-    layernorm_rows_regs<8, false>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, nullptr, nullptr);
+  } else if ((S == kWide || S == kMany) && c <= 2048) {
+    layernorm_rows_regs<8, false, S == kWide>(X, G, B, Y, rows, c, xs, ys, r0, rstep, bd, lane, nullptr, nullptr);
   } else {
     for (int64_t r = blockIdx.x; r < rows; r += nb) {
       const float *xr = X + r * xs;
@@ -454,7 +466,7 @@ layernorm_wave(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_ME
 // lines (row_plan, khrt_templates.cpp): a wave per row, held to two on a SIMD by
 // the registers it is given. Bound by memory, and here the fewer rows a CU has in
 // flight the better: 40000x3000 177 us in workgroups at eight rows a CU
-// (layernorm_wide), 168 at five, 191 in waves at twenty, 163 in waves at eight.
+// (layernorm_wide_many), 168 at five, 191 in waves at twenty, 163 in waves at eight.
 // At 40000x3072, whole lines, the same four take 161, 158, 179 and 160.
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 layernorm_wide_parts(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
@@ -462,12 +474,23 @@ layernorm_wide_parts(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma),
   KH_LAYERNORM_WAVES(16, false, nullptr, nullptr);
 }
 
-// Same arguments and results for rows of 1025..4096 floats (the launcher
-// picks it there): a wave per row up to 2048, a workgroup past that. Events
-// around rotated launches, wave against workgroup: 4096x1100 7.4 vs 8.7 us,
-// 4096x2048 10.9 vs 13.0, 1024x2047 4.8 vs 4.6; past 2048 the wave's 16
-// float4 and its share of gamma and beta took 242 registers (16384x4096 91.4
-// vs 88.5).
+// Same arguments and results for rows of 1025..4096 floats (the launcher picks
+// it there, up to 2048 from four rows a CU on): a wave per row up to 2048, a
+// workgroup past that. Events around rotated launches, wave against workgroup:
+// 4096x1100 7.4 vs 8.7 us, 4096x2048 10.9 vs 13.0, 1024x2047 4.8 vs 4.6; past 2048
+// the wave's 16 float4 and its share of gamma and beta took 242 registers
+// (16384x4096 91.4 vs 88.5).
+extern "C" __global__ void __launch_bounds__(256)
+layernorm_wide_many(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
+                    KH_MEMREF2(float, y)) {
+  KH_LAYERNORM_BODY(kMany, nullptr, nullptr);
+}
+
+// The same for rows of 1025..2048 floats in at most four a CU: gamma and beta are
+// under way beside the row. With one wave on a SIMD nothing else covers their
+// latency after the reductions (in the same workgroups 600x1468 4.09 -> 3.88 us,
+// 200x2048 3.91 -> 3.72). It takes 125 registers for 81, so with more rows it loses
+// (1100x1468 5.2 vs 5.9).
 extern "C" __global__ void __launch_bounds__(256)
 layernorm_wide(KH_MEMREF2(const float, x), KH_MEMREF1(const float, gamma), KH_MEMREF1(const float, beta),
                KH_MEMREF2(float, y)) {

@@ -414,7 +414,7 @@ struct RowPlan {
 };
 
 RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
-  const char *narrow = softmax ? "softmax" : "layernorm", *wide = softmax ? "softmax_wide" : "layernorm_wide",
+  const char *narrow = softmax ? "softmax" : "layernorm", *wide = softmax ? "softmax_wide" : "layernorm_wide_many",
              *block = softmax ? "softmax_block" : "layernorm_block";
   // Too few rows for four to a wave.
   const bool few = rows <= (softmax ? KH_SOFTMAX_WAVE_ROWS(cols) : KH_LAYERNORM_WAVE_ROWS(cols));
@@ -433,6 +433,14 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
   if (softmax && cols <= 512) return {"softmax_wave", 256, 4};
   if (cols <= KH_ROW16_COLS) return {"layernorm_wave", 256, 4};
   if (cols <= 1024) return {narrow, 256, 4};
+  // layernorm in at most one wave on a SIMD (layernorm_wide; layernorm_wide_many
+  // otherwise, as from 1100x1468, 5.2 vs 5.9 us, and 1000x2000, 4.8 vs 5.0): four
+  // rows to a workgroup, or one while that gives a CU two at most (200x1468 3.47 vs
+  // 3.30 us, 512x2000 4.00 vs 3.64, 512x1100 3.61 vs 3.67, 800x1468 4.08 vs 4.30).
+  if (!softmax && cols <= 2048 && rows <= 4 * KH_GEMM_CUS && rows * cols <= 7 << 18) {
+    if (rows <= 2 * KH_GEMM_CUS) return {"layernorm_wide", 64, 1};
+    return {"layernorm_wide", 256, 4};
+  }
   if (cols <= 2048) return {wide, 256, 4};
   if (cols > KH_ROW_BLOCK_MAX) return {block, 1024, 1};
   // softmax of 2049..4096 floats in up to ten rows per CU, once there is enough to

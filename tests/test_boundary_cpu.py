@@ -287,7 +287,7 @@ def test_launcher_geometry(name, shape, grid, block):
 
 @pytest.mark.parametrize("name", ["softmax", "layernorm"])
 @pytest.mark.parametrize("rows,cols,suffix,grid,threads", [
-    (5, 64, "", 1, 256), (6145, 256, "", 385, 256), (1025, 65, "", 65, 256), (5, 513, "", 2, 256), (5, 1024, "", 2, 256), (5, 1025, "_wide", 2, 256), (5, 2048, "_wide", 2, 256),
+    (5, 64, "", 1, 256), (6145, 256, "", 385, 256), (1025, 65, "", 65, 256), (5, 513, "", 2, 256), (5, 1024, "", 2, 256), (1025, 1025, "_wide", 257, 256), (1025, 2048, "_wide", 257, 256),
     (5, 2049, "_wide", 5, 192), (5, 4096, "_wide", 5, 256),
     # 4, 8 and 16 float4 per thread, at most 768 threads; up to a CU for every row 8 to 1024.
     (5, 4097, "", 5, 320), (5, 12288, "", 5, 768), (5, 12289, "", 5, 448), (5, 24576, "", 5, 768),
@@ -297,6 +297,7 @@ def test_launcher_geometry(name, shape, grid, block):
 ])
 def test_row_plan(name, rows, cols, suffix, grid, threads):
     shape = f"rows={rows},cols={cols}"
+    suffix = "_wide_many" if name == "layernorm" and suffix == "_wide" else suffix
     assert kh.launch_symbol(name, shape) == name + suffix
     assert kh.geometry(name, shape) == ((grid, 1, 1), (threads, 1, 1))
 
@@ -323,7 +324,19 @@ def test_row_plan_of_one_template(shape, symbol, grid):
 
 @pytest.mark.parametrize("rows,cols", [(12288, 2689), (12289, 2687), (12289, 2720), (40000, 4096)])
 def test_layernorm_wide_parts_lines(rows, cols):
-    assert kh.launch_symbol("layernorm", f"rows={rows},cols={cols}") == "layernorm_wide"
+    assert kh.launch_symbol("layernorm", f"rows={rows},cols={cols}") == "layernorm_wide_many"
+
+
+@pytest.mark.parametrize("rows,cols,symbol,grid,threads", [
+    (1, 1025, "layernorm_wide", 1, 64), (512, 2048, "layernorm_wide", 512, 64),
+    (513, 1025, "layernorm_wide", 129, 256), (1024, 1792, "layernorm_wide", 256, 256),
+    (1024, 1793, "layernorm_wide_many", 256, 256), (1025, 1025, "layernorm_wide_many", 257, 256), (512, 1024, "layernorm", 128, 256),
+    (512, 2049, "layernorm_wide_many", 512, 192),
+])
+def test_layernorm_wide_one_wave_a_simd(rows, cols, symbol, grid, threads):
+    shape = f"rows={rows},cols={cols}"
+    assert kh.launch_symbol("layernorm", shape) == symbol
+    assert kh.geometry("layernorm", shape) == ((grid, 1, 1), (threads, 1, 1))
 
 
 @pytest.mark.parametrize("rows,cols,symbol,grid,threads", [

@@ -73,7 +73,7 @@ def test_softmax_reference_geometry(dev):
 
 
 @pytest.mark.parametrize("symbol", ["softmax", "softmax_wave", "softmax_wide", "layernorm", "layernorm_wave",
-                                    "layernorm_wide", "layernorm_wide_parts"])
+                                    "layernorm_wide", "layernorm_wide_many", "layernorm_wide_parts"])
 @pytest.mark.parametrize("cols", [64, 256, 512, 1000, 1024, 2048, 4096, 5000])
 def test_every_row_symbol_at_every_width(dev, symbol, cols):
     # Each symbol of a template computes the same result at every width (the
@@ -317,7 +317,8 @@ def test_layernorm_path_edges(dev, cols):
 
 @pytest.mark.parametrize("rows,cols,symbol", [(12289, 2689, "layernorm_wide_parts"), (12290, 4095, "layernorm_wide_parts"),
                                               (300, 24579, "layernorm_block"), (8200, 131, "layernorm"),
-                                              (6001, 254, "layernorm_wave")])
+                                              (6001, 254, "layernorm_wave"), (511, 1026, "layernorm_wide"),
+                                              (895, 2047, "layernorm_wide"), (1025, 1027, "layernorm_wide_many")])
 def test_layernorm_path_of_many_rows(dev, rows, cols, symbol):
     # Launches whose symbol depends on the number of rows too: every operand at an
     # odd address, a guard, and the tolerance as above.
@@ -354,8 +355,8 @@ def test_layernorm_infinities_and_nan(dev, cols):
     assert np.max(np.abs(got[ok] - O.ref_layernorm(x[ok].ravel(), g, b, len(ok), cols))) <= 1e-5
 
 
-@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wave", "layernorm_wide", "layernorm_wide_parts",
-                                    "layernorm_block"])
+@pytest.mark.parametrize("symbol", ["layernorm", "layernorm_wave", "layernorm_wide", "layernorm_wide_many",
+                                    "layernorm_wide_parts", "layernorm_block"])
 @pytest.mark.parametrize("cols", [30, 250, 1500, 4096, 9000])
 @pytest.mark.parametrize("block", [64, 256])
 def test_layernorm_padded_rows_any_symbol(dev, symbol, cols, block):
