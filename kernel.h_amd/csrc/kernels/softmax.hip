@@ -371,13 +371,13 @@ softmax(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
   KH_SOFTMAX_BODY(kNarrow);
 }
 
-// Same arguments and results for rows of 257..512 floats, and for narrower ones
-// where row_plan says (khrt_templates.cpp): a wave per row and nothing else,
+// Same arguments and results for rows of 257..512 floats, and for others up to
+// 1023 where row_plan says (khrt_templates.cpp): a wave per row and nothing else,
 // without LDS. The path is `softmax`'s, instruction for
 // instruction, but as one of that symbol's many it took 2-9% longer: 9300x272
 // 6.25 -> 5.80 us, 40000x272 16.9 -> 15.8, 16384x300 9.0 -> 8.6, 16384x512 13.2 ->
-// 12.8; at 700 and 1024 columns it is 1% slower (40000x1024 53.6 -> 54.3), which is
-// where the line lies.
+// 12.8; at 700 and 1024 columns it is 1% slower (40000x1024 53.6 -> 54.3) but where
+// a launch just about fills the chip once (8192x640 10.0 -> 8.9).
 extern "C" __global__ void __launch_bounds__(256)
 softmax_wave(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
   const uint32_t gw = kh::group_size_word(), nb = kh::grid_blocks_x();
@@ -392,13 +392,18 @@ softmax_wave(KH_MEMREF2(const float, x), KH_MEMREF2(float, y)) {
     return;
   }
   const int lane = kh::lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kh::kWave);
+  bool split = kh::split_first_burst((int64_t)bd * nb);  // each wave's first row only
   for (int64_t r = (int64_t)blockIdx.x * (bd / kh::kWave) + wave; r < rows; r += step) {
     if (cols <= 256)
       softmax_row_regs<1>(X + r * x_s0, Y + r * y_s0, (int)cols, lane);
     else if (cols <= 512)
       softmax_row_regs<2>(X + r * x_s0, Y + r * y_s0, (int)cols, lane);
+    else if (cols <= 1024)
+      split ? softmax_row_regs<4, true>(X + r * x_s0, Y + r * y_s0, (int)cols, lane)
+            : softmax_row_regs<4>(X + r * x_s0, Y + r * y_s0, (int)cols, lane);
     else
       softmax_row_wave(X + r * x_s0, Y + r * y_s0, cols, lane);
+    split = false;
   }
 }
 

@@ -431,6 +431,11 @@ RowPlan row_plan(bool softmax, int64_t rows, int64_t cols) {
     return {narrow, 256, 16};
   }
   if (softmax && cols <= 512) return {"softmax_wave", 256, 4};
+  // Launches that just about fill the chip once, 28 to 34 rows a CU: `softmax` took
+  // 7200x640 8.9 us, 8.2 in softmax_wave, 8192x640 10.0 and 8.9, 8192x768 10.9 and 10.0,
+  // 8400x900 12.8 and 12.6, 8192x1024 13.4 and 13.4; with fewer rows the two are
+  // level (7000x576 7.05 and 7.28), with more `softmax` is 1% faster.
+  if (softmax && cols < 1024 && rows > 28 * KH_GEMM_CUS && rows <= 34 * KH_GEMM_CUS) return {"softmax_wave", 256, 4};
   if (cols <= KH_ROW16_COLS) return {"layernorm_wave", 256, 4};
   if (cols <= 1024) return {narrow, 256, 4};
   // layernorm in at most one wave on a SIMD (layernorm_wide; layernorm_wide_many

@@ -307,6 +307,10 @@ def test_row_plan(name, rows, cols, suffix, grid, threads):
     ("softmax rows=16385,cols=200", "softmax_wave", 4097), ("softmax rows=16384,cols=200", "softmax", 1024),
     ("softmax rows=16385,cols=224", "softmax", 1025), ("softmax rows=16385,cols=180", "softmax", 1025),
     ("softmax rows=16385,cols=256", "softmax", 1025),
+    # Launches that just about fill the chip once.
+    ("softmax rows=7169,cols=513", "softmax_wave", 1793), ("softmax rows=8192,cols=1023", "softmax_wave", 2048),
+    ("softmax rows=7168,cols=513", "softmax", 1792), ("softmax rows=8705,cols=513", "softmax", 2177), ("softmax rows=8704,cols=900", "softmax_wave", 2176),
+    ("softmax rows=8192,cols=1024", "softmax", 2048), ("layernorm rows=8192,cols=640", "layernorm", 2048),
     # Few rows: a wave each.
     ("softmax rows=1024,cols=65", "softmax_wave", 256), ("softmax rows=1025,cols=128", "softmax", 65),
     ("softmax rows=2048,cols=129", "softmax_wave", 512), ("softmax rows=2049,cols=256", "softmax", 129),

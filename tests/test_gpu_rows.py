@@ -216,8 +216,11 @@ def test_softmax_path_edges(dev, cols):
     assert np.max(np.abs(out[:rows * cols].reshape(rows, cols) - ref)) <= 1e-6 * np.max(ref)
 
 
-@pytest.mark.parametrize("rows,cols", [(1664, 2049), (1000, 4095), (2560, 2051), (970, 4096), (257, 24577), (300, 32001)])
-def test_softmax_path_of_many_rows(dev, rows, cols):
+@pytest.mark.parametrize("rows,cols,symbol", [
+    (1664, 2049, "softmax_block"), (1000, 4095, "softmax_block"), (2560, 2051, "softmax_block"), (970, 4096, "softmax_block"),
+    (257, 24577, "softmax_block"), (300, 32001, "softmax_block"), (7170, 514, "softmax_wave"), (8191, 1023, "softmax_wave"),
+])
+def test_softmax_path_of_many_rows(dev, rows, cols, symbol):
     # Launches whose symbol depends on the number of rows too: odd addresses, a
     # guard, and the tolerance as above.
     guard = 64
@@ -225,7 +228,7 @@ def test_softmax_path_of_many_rows(dev, rows, cols):
     ref = O.ref_softmax(x, rows, cols)
     dx, dy = up(np.concatenate([np.full(1, np.nan, np.float32), x])), empty(rows * cols + guard, -7.0)
     say(f"softmax rows={rows} cols={cols}")
-    assert kh.launch_symbol("softmax", f"rows={rows},cols={cols}") == "softmax_block"
+    assert kh.launch_symbol("softmax", f"rows={rows},cols={cols}") == symbol
     kh.softmax(dx.ptr + 4, dy, rows, cols)
     out = down(dy, rows * cols + guard)
     assert np.all(out[rows * cols:] == -7.0)
