@@ -450,8 +450,10 @@ __device__ __forceinline__ void ks_any(const float *__restrict__ A, const float 
 
 // The same with 64-bit addresses, at any strides and spans: launches ks_any_ok
 // turns down (K from 2^23, a wave's share of B past 2^31 bytes, rows that
-// overlap). Its callers take tiles one block wide, whose addresses fit beside
-// the registers of the other forms (two blocks and more took 140-210). Rows past
+// overlap), in `gemm_ksplit_16x16` alone, where the launcher sends such products.
+// In the other symbols it costs their general form 4-6% (32x64 at 1271x218x3364 34.5
+// -> 36.4 us, `gemm_ksplit_deep` at 2000x128x8190 49.3 -> 51.2, 32x16 at 200x400x5000
+// 24.5 -> 25.5, its scalars spilling), there nothing (16x4096x4096 17.2). Rows past
 // M and columns past N load the last one's, which is in range, and are not
 // stored; k past the wave's range only occur in its last partial batch, where
 // the loads are clamped and both operands zeroed. So the loop has no conditional
@@ -549,8 +551,8 @@ __device__ __forceinline__ void ks_wide(const float *__restrict__ A, const float
   }
 }
 
-// Blocks without a whole wave: an element per thread. Summed in runs of 1024
-// k, so that a long K costs no precision.
+// What is left, blocks of less than a wave among it: an element per thread.
+// Summed in runs of 1024 k, so that a long K costs no precision.
 __device__ __forceinline__ void ks_plain(const float *__restrict__ A, const float *__restrict__ B,
                                          float *__restrict__ C, int64_t M, int64_t N, int64_t K, int64_t lda,
                                          int64_t ldb, int64_t ldc, int64_t threads, int64_t nblocks) {
@@ -575,13 +577,13 @@ __device__ __forceinline__ void ks_plain(const float *__restrict__ A, const floa
   const uint32_t gw = kh::group_size_word(), gz = kh::group_size_z_word(), nb = kh::grid_blocks_x();          \
   KH_ARGS_READY(A_base, A_off, A_n0, A_n1, A_s0, B_base, B_off, B_n1, B_s0, C_base, C_off, C_s0, gw, gz, nb)
 
-#define KH_KSPLIT_ANY(TM, TN, NB)                                                                              \
+#define KH_KSPLIT_ANY(TM, TN, NB, WIDE)                                                                        \
   const int nw = (int)kh::threads_x_of(gw) / kh::kWave; /* a partial last wave takes no k and no output */    \
   if (ks_any_ok(nw, A_n0, B_n1, A_n1, A_s0, B_s0, C_s0))                                                      \
     ks_any<TM, TN, NB>(KH_PTR(A), KH_PTR(B), KH_PTR(C), (int)A_n0, (int)B_n1, (int)A_n1, A_s0, B_s0, C_s0,    \
                        nw, (int)nb, red);                                                                     \
-  else if (nw > 0)                                                                                            \
-    ks_wide<TM, 1>(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, nw, nb, red);         \
+  else if (WIDE && nw > 0)                                                                                    \
+    ks_wide<TM, TN>(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, nw, nb, red);        \
   else                                                                                                        \
     ks_plain(KH_PTR(A), KH_PTR(B), KH_PTR(C), A_n0, B_n1, A_n1, A_s0, B_s0, C_s0, kh::threads_x_of(gw), nb)
 
@@ -595,7 +597,7 @@ __device__ __forceinline__ void ks_plain(const float *__restrict__ A, const floa
                 (int)C_s0, (int)nb, red);                                                                    \
     return;                                                                                                   \
   }                                                                                                           \
-  KH_KSPLIT_ANY(2, 2, NB)
+  KH_KSPLIT_ANY(2, 2, NB, false)
 
 extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
@@ -615,19 +617,19 @@ extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit_16x16(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
   __shared__ float red[kKsMaxWaves * 4 * 64];
   KH_KSPLIT_ARGS();
-  KH_KSPLIT_ANY(1, 1, 2);
+  KH_KSPLIT_ANY(1, 1, 2, true);
 }
 
 extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit_32x16(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
   __shared__ float red[kKsMaxWaves * 8 * 64];
   KH_KSPLIT_ARGS();
-  KH_KSPLIT_ANY(2, 1, 2);
+  KH_KSPLIT_ANY(2, 1, 2, false);
 }
 
 extern "C" __global__ void __launch_bounds__(KH_GEMM_KSPLIT_THREADS)
 gemm_ksplit_32x64(KH_MEMREF2(const float, A), KH_MEMREF2(const float, B), KH_MEMREF2(float, C)) {
   __shared__ float red[kKsMaxWaves * 32 * 64];
   KH_KSPLIT_ARGS();
-  KH_KSPLIT_ANY(2, 4, 1);
+  KH_KSPLIT_ANY(2, 4, 1, false);
 }

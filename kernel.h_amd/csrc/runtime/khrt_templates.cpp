@@ -355,7 +355,11 @@ const char *heuristic_gemm_symbol(int64_t m, int64_t n, int64_t k) {
   const bool whole = m % KH_GEMM_KSPLIT_BM == 0 && n % KH_GEMM_KSPLIT_BN == 0 && k % KH_GEMM_KSPLIT_INTERIOR_K == 0;
   const bool deep = k >= KH_GEMM_KSPLIT_DEEP_K &&
                     (whole || static_cast<double>(m + n) * static_cast<double>(k) >= KH_GEMM_KSPLIT_DEEP_FLOATS);
-  const char *ks32 = deep ? "gemm_ksplit_deep" : "gemm_ksplit";
+  // Past the K splits' 32-bit offsets (gemm.hip, ks_any_ok at 8 waves) only the 16x16
+  // tiles have a form with 64-bit ones.
+  const int64_t span = int64_t(1) << 29;  // floats
+  const bool far = k >= span / 64 || (k / 8 + 64) * n >= span;
+  const char *ks32 = far ? "gemm_ksplit_16x16" : deep ? "gemm_ksplit_deep" : "gemm_ksplit";
   const int64_t tiles64 = ks_tiles(KH_GEMM_SMALL_BM, KH_GEMM_SMALL_BN);
   // Whole 32x32 tiles move 16 k a batch and wave, the smaller tiles 32, so that
   // an odd multiple of 128 leaves each of their waves half a batch of padding.
@@ -365,13 +369,13 @@ const char *heuristic_gemm_symbol(int64_t m, int64_t n, int64_t k) {
   // 23.8). A 16x16 tile wins but at K = 128: 3.3-3.5 vs 2.9-3.2 us (256 3.4 vs 3.9).
   const bool half = whole && k % (2 * KH_GEMM_KSPLIT_INTERIOR_K) != 0;
   if (ks_tiles(16, 16) <= KH_GEMM_CUS) return half && k == KH_GEMM_KSPLIT_INTERIOR_K ? ks32 : "gemm_ksplit_16x16";
-  if (ks_tiles(32, 16) <= KH_GEMM_CUS) return half && k < KH_GEMM_KSPLIT_DEEP_K ? ks32 : "gemm_ksplit_32x16";
+  if (ks_tiles(32, 16) <= KH_GEMM_CUS) return far || (half && k < KH_GEMM_KSPLIT_DEEP_K) ? ks32 : "gemm_ksplit_32x16";
   if (ks_tiles(KH_GEMM_KSPLIT_BM, KH_GEMM_KSPLIT_BN) <= KH_GEMM_CUS) return ks32;
   if (tiles64 < KH_GEMM_CUS && whole && k >= KH_GEMM_KSPLIT_MIN_K) return ks32;
   // Past a slab of the 64x64 tiles only: their merge of eight waves' partial
   // tiles costs more than a single slab's products (448x640, K of 1 to 32: 4.5 us
   // against 4.0 in `gemm_small`; K = 33: 4.6 against 4.9).
-  if (k > KH_GEMM_SMALL_BK && ks_tiles(32, 64) <= KH_GEMM_CUS) return "gemm_ksplit_32x64";
+  if (k > KH_GEMM_SMALL_BK && ks_tiles(32, 64) <= KH_GEMM_CUS) return far ? ks32 : "gemm_ksplit_32x64";
   const double big = gemm_score(ceil_div(m, KH_GEMM_BM) * ceil_div(n, KH_GEMM_BN), KH_GEMM_ROUND_BIG,
                                 KH_GEMM_RATE_BIG);
   const double mid = gemm_score(ceil_div(m, KH_GEMM_MID_BM) * ceil_div(n, KH_GEMM_MID_BN), KH_GEMM_ROUND_MID,

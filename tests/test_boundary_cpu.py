@@ -326,6 +326,16 @@ def test_row_plan_of_one_template(shape, symbol, grid):
     assert kh.geometry(name, shape) == ((grid, 1, 1), (256, 1, 1))
 
 
+@pytest.mark.parametrize("shape,symbol", [
+    ("m=500,n=500,k=8388607", "gemm_ksplit_deep"), ("m=500,n=500,k=8388608", "gemm_ksplit_16x16"),
+    ("m=40,n=1000,k=8388608", "gemm_ksplit_16x16"), ("m=33,n=5000,k=858487", "gemm_ksplit_32x64"),
+    ("m=33,n=5000,k=858488", "gemm_ksplit_16x16"),
+])
+def test_gemm_past_32_bit_offsets(shape, symbol):
+    # The K-split symbol with 64-bit addresses takes what the others would do an element at a time.
+    assert kh.launch_symbol("gemm", shape) == symbol
+
+
 @pytest.mark.parametrize("rows,cols", [(12288, 2689), (12289, 2687), (12289, 2720), (40000, 4096)])
 def test_layernorm_wide_parts_lines(rows, cols):
     assert kh.launch_symbol("layernorm", f"rows={rows},cols={cols}") == "layernorm_wide_many"
