@@ -314,17 +314,19 @@ __device__ __forceinline__ void softmax_rows(const float *__restrict__ X, float 
   const int64_t w0 = (int64_t)blockIdx.x * waves_per_block + wave;
   const int c = (int)(cols <= KH_ROW_BLOCK_MAX ? cols : KH_ROW_BLOCK_MAX + 1);
   if (S == kNarrow && c <= KH_ROW16_COLS && xs >= cols && ys >= cols && (xs | ys) < (1 << 26)) {
-    const bool parts = rows > KH_ROW16_CACHED_ROWS && kh::shares_lines(Y, ys);
-    for (int64_t r = 4 * w0; r < rows; r += 4 * nwaves) {
-      if (c <= 64)
-        softmax_rows16<1>(X, Y, r, rows, c, xs, ys, lane);
-      else if (c <= 128)
-        softmax_rows16<2>(X, Y, r, rows, c, xs, ys, lane);
-      else if (parts)
-        softmax_rows16<4, true>(X, Y, r, rows, c, xs, ys, lane);
-      else
-        softmax_rows16<4>(X, Y, r, rows, c, xs, ys, lane);
-    }
+    // One loop per width: with the choice inside one loop a group of rows of up to
+    // 64 floats, over in a microsecond, took 4-6% longer (185147x9 15.6 vs 14.2 us).
+    const auto each = [&](auto go) __attribute__((always_inline)) {
+      for (int64_t r = 4 * w0; r < rows; r += 4 * nwaves) go(r);
+    };
+    if (c <= 64)
+      each([&](int64_t r) __attribute__((always_inline)) { softmax_rows16<1>(X, Y, r, rows, c, xs, ys, lane); });
+    else if (c <= 128)
+      each([&](int64_t r) __attribute__((always_inline)) { softmax_rows16<2>(X, Y, r, rows, c, xs, ys, lane); });
+    else if (rows > KH_ROW16_CACHED_ROWS && kh::shares_lines(Y, ys))
+      each([&](int64_t r) __attribute__((always_inline)) { softmax_rows16<4, true>(X, Y, r, rows, c, xs, ys, lane); });
+    else
+      each([&](int64_t r) __attribute__((always_inline)) { softmax_rows16<4>(X, Y, r, rows, c, xs, ys, lane); });
     return;
   }
   if (S != kBlock && c <= (S == kWide ? 2048 : 1024)) {
